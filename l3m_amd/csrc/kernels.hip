@@ -3248,6 +3248,7 @@ __global__ void __launch_bounds__(NTE) k_pf_gemm(l3m_dmat W, const uint8_t *act,
     }
 }
 
+// The form for the other head dims (k_pf_attn takes multiples of 16 up to 128).
 // Attention of token t, head h over positions 0..t (ops.c:42-73): one wavefront per (t, h), positions in
 // chunks of 64 (a lane per position) with a running maximum and sum; then each lane sums its output
 // dims over the chunk's weights. q from qkv (after RoPE), K and V from the cache as bf16.
@@ -3354,6 +3355,182 @@ __global__ void __launch_bounds__(64) k_pf_attend(const float *qkv, int P, int n
     for (int i = 0; i < 4; i++) {
         const int d = lane + 64 * i;
         if (d < hd) att[(size_t)t * n_heads * hd + h * hd + d] = o[i] / l;
+    }
+}
+
+// Causal attention of the prompt on the matrix cores (ops.c:42-73), for head dims that are multiples of 16
+// up to 128: a workgroup takes 16 consecutive tokens of one head, its PFA_W wavefronts every PFA_W-th chunk
+// of 32 positions, each with a running maximum, and their results meet in LDS at the end.
+//  - Scores transposed: A = the chunk's K rows as they lie in the cache (lane l: row l % 16, 8 dims at
+//    8 (l / 16) of each 32), B = the tokens' q as three bf16 parts (split3: every product exact in f32). A
+//    lane then holds one token's (l % 16) scores of positions 4 (l / 16) + i of both 16-position tiles, so
+//    the softmax is per lane: the maximum meets the token's other three lanes in two permlane swaps.
+//  - Those 8 positions are also the lane's share of the contraction of P.V (the order within a product is
+//    free, V's operand takes the same): p, as three bf16 parts, goes from the softmax to B in registers.
+//    A = V^T, dims by positions: the wavefront transposes the chunk's V rows (4 positions x 8 dims a lane)
+//    into its own LDS span, rows of 40 elements, the lane's 8 positions contiguous.
+// No barrier before the end. Bound by the chunk's chain (loads, two products, expf, LDS round trip), not by
+// bytes or products: 9 heads of 64, 479 tokens: 11.1 us a layer, against 55.7 for k_pf_attend (one wavefront
+// per token and head, a lane per position: every token reads every K and V row again); 63 tokens: 5.0 (7.0).
+constexpr int PFA_W = 4, PFA_T = 16, PFA_C = 32, PFA_VROW = 40;
+template <int HD>
+__global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qkv, int P, int n_heads, int n_kv, int ctx, int layer, float scale,
+                                                        const uint16_t *kc, const uint16_t *vc, float *att, uint8_t *act, int astride) {
+    constexpr int KS = (HD + 31) / 32, NT16 = HD / 16, D8 = HD / 8, UNITS = (HD + 63) / 64, OROW = HD + 4;
+    constexpr size_t VT = (size_t)HD * PFA_VROW * 2;                     // one wavefront's V^T chunk; its merge span is no larger
+    static_assert((size_t)PFA_T * OROW * 4 <= VT, "the merge spans fit the V^T spans");
+    __shared__ __align__(16) uint8_t lds[PFA_W * VT];
+    __shared__ float ml[2][PFA_W][PFA_T];
+    const int lane = tidx() & 63, wave = wave_id(), c16 = lane & 15, quarter = lane >> 4;
+    // the tiles with the most positions first
+    const int t0 = PFA_T * ((int)gridDim.x - 1 - (int)blockIdx.x), h = blockIdx.y, kv = h / (n_heads / n_kv);
+    const int width = (n_heads + 2 * n_kv) * HD, tmax = (t0 + PFA_T < P ? t0 + PFA_T : P) - 1, tok = min(t0 + c16, tmax);
+    const uint16_t *K = kc + ((size_t)layer * n_kv + kv) * ctx * HD, *V = vc + ((size_t)layer * n_kv + kv) * ctx * HD;
+    uint16_t *vt = (uint16_t *)(lds + wave * VT);
+    bf16x8 q[3][KS];
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+        const int d = 32 * s + 8 * quarter;
+        const float *src = qkv + (size_t)tok * width + h * HD + (d < HD ? d : 0);
+        const float4 a = ldg16f(src, 0), b = ldg16f(src, 1);
+        const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            __bf16 p0, p1, p2;
+            split3(d < HD ? x[j] : 0.f, p0, p1, p2);
+            q[0][s][j] = p0; q[1][s][j] = p1; q[2][s][j] = p2;
+        }
+    }
+    f32x4 o[NT16];
+#pragma unroll
+    for (int n = 0; n < NT16; n++) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    for (int p0 = PFA_C * wave; p0 <= tmax; p0 += PFA_C * PFA_W) {
+        bf16x8 kk[2][KS];
+        u32x4 vv[UNITS][4];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const uint16_t *row = K + (size_t)min(p0 + 16 * u + c16, tmax) * HD;   // positions past the last: its row, masked below
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                const int d = 32 * s + 8 * quarter;
+                kk[u][s] = __builtin_bit_cast(bf16x8, *gp<u32x4>(row + (d < HD ? d : 0)));   // past HD: times zeros of q
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < UNITS; u++) {
+            const int id = lane + 64 * u, dg = id % D8, pq = id / D8 < 8 ? id / D8 : 7;
+#pragma unroll
+            for (int e = 0; e < 4; e++) vv[u][e] = *gp<u32x4>(V + (size_t)min(p0 + 4 * pq + e, tmax) * HD + 8 * dg);
+        }
+        f32x4 sc[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            sc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int part = 2; part >= 0; part--)
+#pragma unroll
+                for (int s = 0; s < KS; s++) sc[u] = mfma_bf16(kk[u][s], q[part][s], sc[u]);
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                sc[u][i] = p0 + 16 * u + 4 * quarter + i <= tok ? sc[u][i] * scale : -INFINITY;
+                mx = fmaxf(mx, sc[u][i]);
+            }
+        float lo, hi;
+        swap16(mx, lo, hi); mx = fmaxf(lo, hi);
+        swap32(mx, lo, hi); mx = fmaxf(lo, hi);
+        const float nm = fmaxf(m, mx), base = nm == -INFINITY ? 0.f : nm;   // no position yet: every p is 0
+        const float r = expf(m - base);
+        l *= r;
+        bf16x8 p[3];
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float e = expf(sc[u][i] - base);
+                __bf16 x0, x1, x2;
+                l += e;
+                split3(e, x0, x1, x2);
+                p[0][4 * u + i] = x0; p[1][4 * u + i] = x1; p[2][4 * u + i] = x2;
+            }
+        m = nm;
+        // V^T: position quad pq (positions 4 pq ..) at element 4 ((pq % 4) * 2 + pq / 4), so that a lane's 8
+        // positions (4 quarter + i, 16 + 4 quarter + i) are 16 contiguous bytes
+#pragma unroll
+        for (int u = 0; u < UNITS; u++) {
+            const int id = lane + 64 * u, dg = id % D8, pq = id / D8;
+            if (pq < 8) {
+                uint16_t *dst = vt + (size_t)8 * dg * PFA_VROW + 4 * ((pq & 3) * 2 + (pq >> 2));
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    *(u32x2 *)(dst + (2 * j) * PFA_VROW) = u32x2{__builtin_amdgcn_perm(vv[u][1][j], vv[u][0][j], 0x05040100u),
+                                                                __builtin_amdgcn_perm(vv[u][3][j], vv[u][2][j], 0x05040100u)};
+                    *(u32x2 *)(dst + (2 * j + 1) * PFA_VROW) = u32x2{__builtin_amdgcn_perm(vv[u][1][j], vv[u][0][j], 0x07060302u),
+                                                                    __builtin_amdgcn_perm(vv[u][3][j], vv[u][2][j], 0x07060302u)};
+                }
+            }
+        }
+        // the span is the wavefront's own and its LDS accesses complete in order: only the compiler has to
+        // keep them so
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int n = 0; n < NT16; n++) {
+            const bf16x8 a = *(const bf16x8 *)(vt + (size_t)(16 * n + c16) * PFA_VROW + 8 * quarter);
+            o[n][0] *= r; o[n][1] *= r; o[n][2] *= r; o[n][3] *= r;
+#pragma unroll
+            for (int part = 2; part >= 0; part--) o[n] = mfma_bf16(a, p[part], o[n]);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+    }
+    float lo, hi;
+    swap16(l, lo, hi); l = lo + hi;
+    swap32(l, lo, hi); l = lo + hi;
+    float *om = (float *)vt + c16 * OROW;
+#pragma unroll
+    for (int n = 0; n < NT16; n++) *(float4 *)(om + 16 * n + 4 * quarter) = make_float4(o[n][0], o[n][1], o[n][2], o[n][3]);
+    if (quarter == 0) { ml[0][wave][c16] = m; ml[1][wave][c16] = l; }
+    __syncthreads();
+    // each thread 4 dims of a token: the wavefronts' parts in order, scaled to the common maximum (wavefront 0
+    // always has position 0)
+    for (int u = tidx(); u < PFA_T * HD / 4; u += 64 * PFA_W) {
+        const int tt = u / (HD / 4), d4 = u % (HD / 4), t = t0 + tt;
+        float mm = ml[0][0][tt];
+#pragma unroll
+        for (int w = 1; w < PFA_W; w++) mm = fmaxf(mm, ml[0][w][tt]);
+        float den = 0.f;
+        float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < PFA_W; w++) {
+            const float f = expf(ml[0][w][tt] - mm);
+            const float4 x = *(const float4 *)((const float *)(lds + w * VT) + tt * OROW + 4 * d4);
+            den += ml[1][w][tt] * f;
+            y.x += x.x * f; y.y += x.y * f; y.z += x.z * f; y.w += x.w * f;
+        }
+        y = make_float4(y.x / den, y.y / den, y.z / den, y.w / den);
+        if constexpr (HD % 32 == 0) {
+            // the head's 32-blocks prepared here (8 lanes a block, prep_body's formulas)
+            const float am = lanes_max<8>(fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w))));
+            const float inv = am > 0.f ? 127.0f / am : 0.f;
+            const int q0 = (int)rintf(y.x * inv), q1 = (int)rintf(y.y * inv), q2 = (int)rintf(y.z * inv), q3 = (int)rintf(y.w * inv);
+            const int sum = lanes_sumi<8>(q0 + q1 + q2 + q3);
+            if (t < P) {
+                uint8_t *row = act + (size_t)t * astride;
+                const int nb = (n_heads * HD) >> 5, e = h * HD + 4 * d4;
+                *(uint32_t *)(row + e) = (uint32_t)(q0 & 255) | (uint32_t)(q1 & 255) << 8 | (uint32_t)(q2 & 255) << 16 | (uint32_t)(q3 & 255) << 24;
+                if ((d4 & 7) == 0) {
+                    ((float *)(row + 32 * nb))[e >> 5] = am / 127.0f;
+                    ((int *)(row + 36 * nb))[e >> 5] = sum;
+                }
+            }
+        } else if (t < P) {
+            *(float4 *)(att + (size_t)t * n_heads * HD + h * HD + 4 * d4) = y;
+        }
     }
 }
 
@@ -3661,6 +3838,19 @@ template <int DT, int HDT, bool G2> int decode_fits(int hd, int grid, unsigned l
         if (hd == 48) return decode_fits_hd<DT, HDT, G2, 48>(grid, lds);
     }
     return decode_fits_hd<DT, HDT, G2, 0>(grid, lds);
+}
+
+// The prompt's attention in layer l: on the matrix cores for head dims of 16, 32, ... 128 (k_pf_attn), else
+// k_pf_attend.
+void pf_attention(const l3m_dmodel *M, const l3m_pfbuf *B, int P, int l, bool fuse, hipStream_t st) {
+#define PF_ATTN(HD) \
+    case HD: hipLaunchKernelGGL(k_pf_attn<HD>, dim3((P + PFA_T - 1) / PFA_T, M->n_heads), dim3(64 * PFA_W), 0, st, (const float *)B->qkv, P, \
+                                M->n_heads, M->n_kv, M->ctx, l, M->att_scale, (const uint16_t *)M->kc, (const uint16_t *)M->vc, B->att, \
+                                B->act, B->astride); return;
+    switch (M->hd) { PF_ATTN(16) PF_ATTN(32) PF_ATTN(48) PF_ATTN(64) PF_ATTN(80) PF_ATTN(96) PF_ATTN(112) PF_ATTN(128) }
+#undef PF_ATTN
+    hipLaunchKernelGGL(k_pf_attend, dim3(P, M->n_heads), dim3(64), 0, st, (const float *)B->qkv, P, M->n_heads, M->n_kv, M->hd, M->ctx, l,
+                       M->att_scale, (const uint16_t *)M->kc, (const uint16_t *)M->vc, B->att, fuse ? B->act : nullptr, B->astride);
 }
 
 template <int DT> int launch_step_mv(int form, const l3m_dmat &m, const float *x, int k, float *y, int tpw, hipStream_t st) {
@@ -4059,8 +4249,7 @@ int l3m_prefill(const l3m_dmodel *M, const l3m_pflayer *L, const l3m_pfbuf *B, i
         gemm(W.qkv, B->qkv, width, 0, &E);
         if (l == M->n_layers - 1) break;              // the last layer's K/V rows are all its prompt positions leave
         const bool fuse = hd % 32 == 0;               // whole blocks per head: the attention prepares its output
-        hipLaunchKernelGGL(k_pf_attend, dim3(P, M->n_heads), dim3(64), 0, st, (const float *)B->qkv, P, M->n_heads, M->n_kv, hd, M->ctx, l,
-                           M->att_scale, (const uint16_t *)M->kc, (const uint16_t *)M->vc, B->att, fuse ? B->act : nullptr, B->astride);
+        pf_attention(M, B, P, l, fuse, st);
         if (!fuse) hipLaunchKernelGGL(k_pf_prep, dim3(P), dim3(NTE), 0, st, (const float *)B->att, nq, nq, B->act, B->astride);
         gemm(W.wo, B->x, dim, 1, nullptr);
         hipLaunchKernelGGL(k_pf_norm_prep, dim3(P), dim3(NTE), 0, st, (const float *)B->x, W.ffn_norm, dim, M->eps, B->act, B->astride);

@@ -183,3 +183,26 @@ def test_prefill_graph_cache_replaces_the_oldest(models, monkeypatch):
         assert got == want, (i, n_prompt)
         assert np.array_equal(graph.logits, loose.logits), (i, n_prompt)
     graph.close(); loose.close()
+
+
+@pytest.mark.parametrize("n_prompt", [8, 17, 34, 130])
+@pytest.mark.parametrize("hd", [16, 24, 80, 96, 112, 128])
+def test_prefill_attention_head_dims(models, oracle, hd, n_prompt):
+    """The prompt's attention at head dims off the other tests': multiples of 16 up to 128 on the matrix cores
+    (16-token tiles, 32-position chunks dealt to four wavefronts: 7, 16, 33 and 129 positions), 24 in the form
+    with a wavefront per token and head; grouped KV heads. Logits and the second layer's K/V rows (which the
+    first layer's attention enters) meet the bars of test_prefill_logits against the oracle."""
+    heads = 4
+    cfg = A.Config(f"pf_attn{hd}", dim=heads * hd, n_layers=2, n_heads=heads, n_kv_heads=2, ffn_dim=256, vocab=512, ctx=160, dtype="q8_0")
+    path = models.get(cfg, cfg.dtype, seed=11, std=0.05, norm_jitter=0.1)
+    ids = A.prompt(12, cfg.vocab, n_prompt)
+    om = oracle.load(path, ctx=160)
+    om.generate(ids, 0)
+    with A.Model(path, ctx=160) as m:
+        m.generate(ids, 0)
+        assert m.prefilled == n_prompt - 1
+        assert close(m.logits, om.logits())
+        for kvh in range(2):
+            for got, want in zip(m.kv_rows(1, kvh, 0, n_prompt - 1), om.kv_rows(1, kvh, 0, n_prompt - 1, hd)):
+                g, w = bf16(got), bf16(want)
+                assert np.abs(g - w).max() <= 0.02 * np.abs(w).max(), kvh
