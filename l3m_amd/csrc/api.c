@@ -549,16 +549,16 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
     d->po = dalloc(m, (size_t)d->n_groups * d->dim * 4);
     d->pd = dalloc(m, (size_t)d->n_chunks * d->dim * 4);
     if (m->pf) {
-        int mk = d->dim > d->n_heads * d->hd ? d->dim : d->n_heads * d->hd;
-        if (d->ffn > mk) mk = d->ffn;
-        const size_t kp = (size_t)(mk + 31) / 32 * 32, ctx = (size_t)d->ctx;
-        m->pfb.astride = (int)((kp + 8 * (kp / 32) + 15) / 16 * 16);   // int8 values, f32 scales, i32 sums
+        // activations of whole 64-token groups (a GEMM's workgroup reads up to 64 tokens)
+        const size_t nqd = (size_t)d->n_heads * d->hd, mk = (size_t)d->dim > nqd ? (size_t)d->dim : nqd, ctx = (size_t)d->ctx, c64 = (ctx + 63) / 64 * 64;
         m->pfb.x = dalloc(m, ctx * d->dim * 4);
-        m->pfb.act = dalloc(m, ctx * m->pfb.astride);
-        m->pfb.qkv = dalloc(m, ctx * (size_t)(d->n_heads + 2 * d->n_kv) * d->hd * 4);
-        m->pfb.att = dalloc(m, ctx * (size_t)d->n_heads * d->hd * 4);
-        m->pfb.gu = dalloc(m, ctx * 2 * (size_t)d->ffn * 4);
-        if (!m->pfb.x || !m->pfb.act || !m->pfb.qkv || !m->pfb.att || !m->pfb.gu) return fail(m, "out of device memory");
+        m->pfb.act.q = dalloc(m, c64 * mk);
+        m->pfb.act.s = dalloc(m, c64 * mk / 32 * 4);
+        m->pfb.hact.q = dalloc(m, c64 * d->ffn);
+        m->pfb.hact.s = dalloc(m, c64 * d->ffn / 32 * 4);
+        m->pfb.q = dalloc(m, ctx * nqd * 4);
+        m->pfb.att = dalloc(m, ctx * nqd * 4);
+        if (!m->pfb.x || !m->pfb.act.q || !m->pfb.act.s || !m->pfb.hact.q || !m->pfb.hact.s || !m->pfb.q || !m->pfb.att) return fail(m, "out of device memory");
         const char *pg = getenv("L3M_PREFILL_GRAPH");  // 0: loose launches (for comparison)
         if ((!pg || strcmp(pg, "0")) && !(m->pfg = l3m_pfgraphs_new())) return fail(m, "out of host memory");
     }

@@ -154,13 +154,18 @@ typedef struct {
     l3m_dmat     down;           // dim x ffn
     const float *attn_norm, *ffn_norm;
 } l3m_pflayer;
+// A prepared activation of the prompt's tokens, in blocks of 16 tokens x 32 inputs (kernels.hip, pf_slot): values
+// [ceil64(ctx) / 16][k / 32][16][32] and block scales [ceil64(ctx) / 16][k / 32][16].
 typedef struct {
-    float   *x;                  // [ctx][dim] residual stream
-    uint8_t *act;                // [ctx][astride] int8 prep of each token's matrix input
-    float   *qkv;                // [ctx][(n_heads + 2 n_kv) hd]
-    float   *att;                // [ctx][n_heads hd]
-    float   *gu;                 // [ctx][2 ffn]
-    int      astride;
+    uint8_t *q;
+    float   *s;
+} l3m_pfact;
+typedef struct {
+    float    *x;                 // [ctx][dim] residual stream
+    l3m_pfact act;               // the input of the q/k/v, Wo and gate/up matrices
+    l3m_pfact hact;              // the input of Wdown (the gate/up kernel writes it while it reads act)
+    float    *q;                 // [ctx][n_heads hd], after RoPE
+    float    *att;               // [ctx][n_heads hd], for head dims that are not whole 32-blocks
 } l3m_pfbuf;
 // K/V rows of positions 0..P-1 of every layer from the token ids on the device (m->tokens); the last
 // layer's FFN is skipped (nothing reads it). -1 on a launch error.

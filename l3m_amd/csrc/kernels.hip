@@ -3113,156 +3113,275 @@ __global__ void __launch_bounds__(NTE) k_pf_embed(l3m_dmat embed, const int32_t 
     if (4 * f < dim) ((float4 *)(x + (size_t)t * dim))[f] = lt_elem4(embed, tokens[t], 4 * f);
 }
 
-// act[t] = the int8 prep of RMSNorm(x[t]) * w (engine.c:241, 261); one workgroup per token.
-__global__ void __launch_bounds__(NTE) k_pf_norm_prep(const float *x, const float *w, int dim, float eps, uint8_t *act, int astride) {
-    __shared__ float scr[32];
-    const int t = blockIdx.x, f = tidx(), own = 4 * f < dim ? f : 0;
-    const float4 xv = 4 * f < dim ? ((const float4 *)(x + (size_t)t * dim))[own] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 nw = ((const float4 *)w)[own];
-    Red red{scr, 0};
-    norm_prep<L3M_Q8_0>(xv, nw, dim, kpad(dim), eps, act + (size_t)t * astride, red);
+// A prefill activation: per 16 tokens and 32-input block the tokens' blocks, [token / 16][block][16][32] int8
+// with its scale beside it in [token / 16][block][16] (the prep of pack.c:101-123; the block sums are not
+// needed), so that a product's operand is one contiguous run, as a weight tile's is. Rows of tokens past the
+// prompt's end hold whatever was there: a product's column depends on its own token alone, and theirs are not
+// stored.
+__device__ __forceinline__ size_t pf_slot(int t, int b, int nb) { return ((size_t)(t >> 4) * nb + b) * 16 + (t & 15); }
+
+// Values e .. e + 3 (e a multiple of 4) of token t's activation, 8 consecutive lanes a block: prep_body's
+// formulas. All lanes of a block take part; store: whether they write.
+__device__ __forceinline__ void pf_put4(const l3m_pfact &a, int t, int nb, int e, float4 y, bool store) {
+    const float am = lanes_max<8>(fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w))));
+    const float inv = am > 0.f ? 127.0f / am : 0.f;
+    const int q0 = (int)rintf(y.x * inv), q1 = (int)rintf(y.y * inv), q2 = (int)rintf(y.z * inv), q3 = (int)rintf(y.w * inv);
+    if (!store) return;
+    const size_t slot = pf_slot(t, e >> 5, nb);
+    *(uint32_t *)(a.q + slot * 32 + (e & 31)) = (uint32_t)(q0 & 255) | (uint32_t)(q1 & 255) << 8 | (uint32_t)(q2 & 255) << 16 | (uint32_t)(q3 & 255) << 24;
+    if ((e & 31) == 0) a.s[slot] = am / 127.0f;
 }
 
-// act[t] = the int8 prep of y[t][0..k) (the attention output before Wo); one workgroup per token.
-__global__ void __launch_bounds__(NTE) k_pf_prep(const float *y, int ystride, int k, uint8_t *act, int astride) {
-    const int t = blockIdx.x, f = tidx();
-    const float4 v = 4 * f < k ? ((const float4 *)(y + (size_t)t * ystride))[f] : make_float4(0.f, 0.f, 0.f, 0.f);
-    prep_owned<L3M_Q8_0>(v, act + (size_t)t * astride, kpad(k));
-}
-
-// act[t] = the int8 prep of up * silu(gate) (ops.c:49-51) from gu[t] = [gate 0..ffn) | up 0..ffn)].
-__global__ void __launch_bounds__(NTE) k_pf_silu_prep(const float *gu, int ffn, uint8_t *act, int astride) {
-    const int t = blockIdx.x, f = tidx();
-    float4 h = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (4 * f < ffn) {
-        const float4 g = ((const float4 *)(gu + (size_t)t * 2 * ffn))[f], u = ((const float4 *)(gu + (size_t)t * 2 * ffn + ffn))[f];
-        h = make_float4(silu_mul(u.x, g.x), silu_mul(u.y, g.y), silu_mul(u.z, g.z), silu_mul(u.w, g.w));
+// act[t] = the prep of y[t][0..k), or (NORM) of RMSNorm(y[t]) * w (engine.c:241, 261): a wavefront per token, 4
+// values a lane for every 256, the sum of squares added as norm_prep adds it (per 256, then the 16 slots'
+// tree). One wavefront per token instead of a 1024-thread workgroup, no LDS or barrier: 479 tokens of 576
+// values 4.7 us, as before (4.8): what is left is one kernel's fixed cost, loads and launch.
+template <bool NORM, int C>                          // C: 256-value pieces of a row
+__global__ void __launch_bounds__(256) k_pf_rows(const float *y, int k, const float *w, float eps, l3m_pfact act, int P) {
+    const int t = 4 * blockIdx.x + wave_id(), lane = tidx() & 63, nb = k >> 5;
+    if (t >= P) return;
+    const float *row = y + (size_t)t * k;
+    // every load first (past k: buffer loads past the range, no branch and no access), the weights' among them
+    float4 v[C], nw[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) v[c] = ld16f_if<false>(row, 64 * c + lane, 256 * c + 4 * lane < k);
+    if constexpr (NORM) {
+#pragma unroll
+        for (int c = 0; c < C; c++) nw[c] = ld16f_if<false>(w, 64 * c + lane, 256 * c + 4 * lane < k);
     }
-    prep_owned<L3M_Q8_0>(h, act + (size_t)t * astride, kpad(ffn));
+    float s = 1.f;
+    if constexpr (NORM) {
+        float part[16], q[4];
+#pragma unroll
+        for (int c = 0; c < 16; c++) part[c] = 0.f;
+#pragma unroll
+        for (int c = 0; c < C; c++) part[c] = lanes_sum<64>(v[c].x * v[c].x + v[c].y * v[c].y + v[c].z * v[c].z + v[c].w * v[c].w);
+#pragma unroll
+        for (int i = 0; i < 4; i++) q[i] = (part[4 * i] + part[4 * i + 1]) + (part[4 * i + 2] + part[4 * i + 3]);
+        s = 1.0f / sqrtf(((q[0] + q[1]) + (q[2] + q[3])) / (float)k + eps);
+    }
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int e = 256 * c + 4 * lane;
+        float4 x = v[c];
+        if constexpr (NORM) x = make_float4(x.x * s * nw[c].x, x.y * s * nw[c].y, x.z * s * nw[c].z, x.w * s * nw[c].w);
+        pf_put4(act, t, nb, e, x, e < k);
+    }
 }
 
-// y[t][r] = sum over blocks b of d_w[r][b] * s_t[b] * (the int8 dot of row r and token t over block b):
-// the q8_0 gemv of every token at once (kernels_scalar.c:30-45), with the integer dots on
-// v_mfma_i32_16x16x32_i8 (one 32-input block per product). A workgroup takes one 16-row tile and 16
-// tokens; its S = blockDim / 64 wavefronts (pf_split) split the blocks into S contiguous ranges of at most
-// PF_BATCH blocks each (more only past 16 * PF_BATCH blocks), each range's loads issued before its
-// products. The kernel is short: its time goes to instruction issue, so a wavefront gets few blocks. Lane
-// l holds weights of row l % 16 and activations of token l % 16, 8 bytes each at byte 8 (l / 16) of the
-// block, and gets rows 4 (l / 16) + i of that token; the S ranges' sums are added in range order through
-// LDS. add: y += the result (the residual adds, engine.c:259, 275), else y = it.
+// The matrices of a prompt (the q8_0 gemv of every token at once, kernels_scalar.c:30-45): per 16 rows x 16
+// tokens and 32-input block one v_mfma_i32_16x16x32_i8, its i32 result scaled by the row's and the token's
+// block scales into the f32 sum, blocks in order. Lane l holds row (token) l % 16, 8 bytes at byte 8 (l / 16) of
+// the block, and gets rows 4 (l / 16) + i of token l % 16.
+//
+// A row's blocks fall into ranges of PF_RANGE blocks or so (pf_ranges), each summed by itself, then added in
+// order. A wavefront takes RT x TT tiles over its share of the ranges: KS = blockDim / (64 WR) wavefronts split
+// them, and their sums are added in order through LDS; WR wavefronts of each share lie side by side. Operands come straight from L2 in the layouts they lie in (512 contiguous bytes a tile and
+// block), PB blocks ahead; nothing is staged. Per product a lane spends 12 VALU instructions on the scales
+// (48 clocks of its SIMD against 8 for the product), which bounds the largest shapes; RT = TT = 2 loads each
+// operand once for two products. The others are bound by latency, a chain of loads over few wavefronts: they
+// split the blocks (pf_gemm's rule). 479 tokens, 30 layers of dim 576 and ffn 1536 (kernel trace), against one
+// 16 x 16 tile a workgroup with each token's input in a row of its own: q/k/v 14.8 -> 7.7 us, Wo 10.8 -> 7.2,
+// gate/up 36.7 -> 12.0 with the SiLU and prep kernel (4.9) gone into it, Wdown 24.4 -> 9.3.
+//
+// EPI 0: y += the product (the residual adds, engine.c:259, 275).
+// EPI 1: the q/k/v rows: RoPE on q and k (pairs (2i, 2i + 1) of each head rotated by angle i of position t from
+//        the host table, ops.c:29-40), q into y, the k and v rows rounded to bf16 into the cache
+//        (engine.c:247-248). A lane's four rows are two whole pairs.
+// EPI 2: gate and up rows (RT = 2: the same rows' gate tile and up tile), up * silu(gate) (ops.c:49-51) and its
+//        int8 prep into out: the workgroup's 2 x 16 rows are one 32-block of the next matrix's input.
 typedef int v4i32 __attribute__((ext_vector_type(4)));
-constexpr int PF_BATCH = 4;
-__host__ __device__ inline int pf_split(int nb) {
-    const int s = (nb + PF_BATCH - 1) / PF_BATCH;
-    return s < 1 ? 1 : s > NWE ? NWE : s;
-}
-// The qkv matrix's epilogue (PfQkv): RoPE on the q and k rows (pairs (2i, 2i+1) of each head rotated by
-// the angle i of position t from the host table, ops.c:29-40), q into y, the k and v rows rounded to bf16
-// into the cache (engine.c:247-248). A lane's four rows are two whole pairs.
-struct PfQkv {
-    const float *rope;
+constexpr int PF_RANGE = 4;
+__host__ __device__ inline int pf_ranges(int nb) { return min(max((nb + PF_RANGE - 1) / PF_RANGE, 1), 16); }
+struct PfGemm {
+    l3m_dmat W;
+    l3m_pfact x, out;
+    int P, ystride;
+    float *y;
+    const float *rope;                                // EPI 1
     uint16_t *kc, *vc;
     int layer, ctx, nq, nk, hd, n_kv;
 };
-template <bool QKV>
-__global__ void __launch_bounds__(NTE) k_pf_gemm(l3m_dmat W, const uint8_t *act, int astride, int P, float *y, int ystride, int add,
-                                                 PfQkv E) {
-    __shared__ f32x4 part[NWE][64];
-    const int lane = tidx() & 63, wave = wave_id(), S = blockDim.x >> 6, tile = blockIdx.x, tg = blockIdx.y;
-    const int nb = W.nb, kp = 32 * nb, quarter = lane >> 4, col = lane & 15;
-    const int per = (nb + S - 1) / S, r0 = wave * per, r1 = r0 + per < nb ? r0 + per : nb;   // this wavefront's blocks
-    const int tok = tg * 16 + col < P ? tg * 16 + col : P - 1;
-    const uint8_t *wq = (const uint8_t *)W.q + (size_t)tile * nb * 512 + col * 32 + quarter * 8;
-    const uint16_t *ws = (const uint16_t *)W.s + (size_t)tile * nb * 16 + quarter * 4;
-    const uint8_t *aq = act + (size_t)tok * astride + quarter * 8;
-    const float *as = (const float *)(act + (size_t)tok * astride + kp);
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int b0 = r0; b0 < r1; b0 += PF_BATCH) {
-        long a8[PF_BATCH], x8[PF_BATCH];
-        u32x2 sw[PF_BATCH];
-        float sa[PF_BATCH];
+template <int RT_, int TT_> struct PfFrag {
+    long a[RT_], x[TT_];
+    u32x2 sw[RT_];
+    float sx[TT_];
+};
+template <int EPI, int RT_, int TT_, int WR, int KMAX>
+__global__ void __launch_bounds__(64 * WR * KMAX) k_pf_gemm(PfGemm G) {
+    constexpr int PB = 4;
+    __shared__ f32x4 part[KMAX > 1 ? (KMAX - 1) * WR * RT_ * TT_ : 1][64];
+    __shared__ float amx[EPI == 2 ? WR * TT_ : 1][16];
+    const int lane = tidx() & 63, wave = wave_id(), c16 = lane & 15, quarter = lane >> 4;
+    const int kw = wave / WR, wr = wave % WR, nb = G.W.nb;
+    const int KS = KMAX > 1 ? (int)blockDim.x / (64 * WR) : 1, R = pf_ranges(nb), per = (nb + R - 1) / R;
+    const int k0 = min(kw * R / KS * per, nb), k1 = min((kw + 1) * R / KS * per, nb);
+    int rt[RT_], tt[TT_];                             // 16-row tiles, 16-token tiles
 #pragma unroll
-        for (int i = 0; i < PF_BATCH; i++) {
-            const int b = b0 + i < r1 ? b0 + i : r1 - 1;
-            a8[i] = *gp<long>(wq + (size_t)b * 512);
-            x8[i] = *gp<long>(aq + (size_t)b * 32);
-            sw[i] = *gp<u32x2>(ws + (size_t)b * 16);
-            sa[i] = *gp<float>(as + b);
-        }
-        // every load of the batch is issued before the first product: the loads cannot sink below the
-        // memory clobber, and the products read their operands through the moves after it
-        asm volatile("" ::: "memory");
+    for (int r = 0; r < RT_; r++)
+        rt[r] = EPI == 2 ? (int)blockIdx.x * WR + wr + r * (G.W.tiles >> 1) : ((int)blockIdx.x * WR + wr) * RT_ + r;
 #pragma unroll
-        for (int i = 0; i < PF_BATCH; i++) asm volatile("" : "+v"(a8[i]), "+v"(x8[i]), "+v"(sw[i]), "+v"(sa[i]));
+    for (int t = 0; t < TT_; t++) tt[t] = (int)blockIdx.y * TT_ + t;
+    const uint8_t *wq[RT_], *xq[TT_];
+    const uint16_t *ws[RT_];
+    const float *xs[TT_];
 #pragma unroll
-        for (int i = 0; i < PF_BATCH; i++) {
-            const v4i32 c = __builtin_amdgcn_mfma_i32_16x16x32_i8(a8[i], x8[i], v4i32{0, 0, 0, 0}, 0, 0, 0);
-            const float m = b0 + i < r1 ? sa[i] : 0.f;
-            acc[0] += (float)c[0] * (f16_f32(sw[i].x & 0xFFFF) * m);
-            acc[1] += (float)c[1] * (f16_f32(sw[i].x >> 16) * m);
-            acc[2] += (float)c[2] * (f16_f32(sw[i].y & 0xFFFF) * m);
-            acc[3] += (float)c[3] * (f16_f32(sw[i].y >> 16) * m);
-        }
+    for (int r = 0; r < RT_; r++) {
+        const size_t at = (size_t)min(rt[r], G.W.tiles - 1) * nb * 16;   // tiles past the last: it again, not stored
+        wq[r] = G.W.q + (at + c16) * 32 + quarter * 8;
+        ws[r] = (const uint16_t *)G.W.s + at + quarter * 4;
     }
-    if (wave) part[wave][lane] = acc;
-    __syncthreads();
-    const int t = tg * 16 + col;
-    if (wave == 0 && t < P) {
-        for (int w = 1; w < S; w++) {
-            const f32x4 p = part[w][lane];
-            acc[0] += p[0]; acc[1] += p[1]; acc[2] += p[2]; acc[3] += p[3];
-        }
-        if constexpr (QKV) {
-            const int r0 = tile * 16 + 4 * quarter;   // even: rows r0 .. r0 + 3 are pairs (r0, r0 + 1), (r0 + 2, r0 + 3)
-            const float2 *cs = (const float2 *)(E.rope + (size_t)t * E.hd);
 #pragma unroll
-            for (int i = 0; i < 4; i += 2) {
-                const int e = r0 + i;
-                if (e < E.nq + E.nk) {
-                    const int j = (e < E.nq ? e : e - E.nq) % E.hd;
-                    const float2 c = cs[j >> 1];
-                    const float a = acc[i], b = acc[i + 1];
-                    acc[i] = a * c.x - b * c.y;
-                    acc[i + 1] = a * c.y + b * c.x;
+    for (int t = 0; t < TT_; t++) {
+        const size_t at = (size_t)tt[t] * nb * 16 + c16;
+        xq[t] = G.x.q + at * 32 + quarter * 8;
+        xs[t] = G.x.s + at;
+    }
+    PfFrag<RT_, TT_> f[PB];
+    auto load = [&](PfFrag<RT_, TT_> &g, int b) {
+        b = min(b, nb - 1);                           // past the range: a block in bounds, not used
+#pragma unroll
+        for (int r = 0; r < RT_; r++) {
+            g.a[r] = *gp<long>(wq[r] + (size_t)b * 512);
+            g.sw[r] = *gp<u32x2>(ws[r] + (size_t)b * 16);
+        }
+#pragma unroll
+        for (int t = 0; t < TT_; t++) {
+            g.x[t] = *gp<long>(xq[t] + (size_t)b * 512);
+            g.sx[t] = *gp<float>(xs[t] + (size_t)b * 16);
+        }
+    };
+    f32x4 acc[RT_][TT_], cur[RT_][TT_];               // the sum of the ranges done, the current range's
+#pragma unroll
+    for (int r = 0; r < RT_; r++)
+#pragma unroll
+        for (int t = 0; t < TT_; t++) acc[r][t] = cur[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int next = k0 + per;
+#pragma unroll
+    for (int i = 0; i < PB; i++) load(f[i], k0 + i);
+    for (int b0 = k0; b0 < k1; b0 += PB) {
+#pragma unroll
+        for (int i = 0; i < PB; i++) {
+            if (b0 + i < k1) {                        // uniform
+#pragma unroll
+                for (int r = 0; r < RT_; r++) {
+                    const float d[4] = {f16_f32(f[i].sw[r].x & 0xFFFF), f16_f32(f[i].sw[r].x >> 16), f16_f32(f[i].sw[r].y & 0xFFFF),
+                                        f16_f32(f[i].sw[r].y >> 16)};
+#pragma unroll
+                    for (int t = 0; t < TT_; t++) {
+                        const v4i32 c = __builtin_amdgcn_mfma_i32_16x16x32_i8(f[i].a[r], f[i].x[t], v4i32{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                        for (int j = 0; j < 4; j++) cur[r][t][j] += (float)c[j] * (d[j] * f[i].sx[t]);
+                    }
+                }
+                if (b0 + i + 1 == next || b0 + i + 1 == k1) {   // uniform: the range is done
+                    next += per;
+#pragma unroll
+                    for (int r = 0; r < RT_; r++)
+#pragma unroll
+                        for (int t = 0; t < TT_; t++) { acc[r][t] += cur[r][t]; cur[r][t] = f32x4{0.f, 0.f, 0.f, 0.f}; }
                 }
             }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int r = r0 + i;
-                if (r < E.nq) y[(size_t)t * ystride + r] = acc[i];
-                else if (r < W.rows) {
-                    const int kv = r < E.nq + E.nk ? 0 : 1, rr = r - E.nq - kv * E.nk, h = rr / E.hd, j = rr - h * E.hd;
-                    (kv ? E.vc : E.kc)[(((size_t)E.layer * E.n_kv + h) * E.ctx + t) * E.hd + j] = f32_bf16(acc[i]);
-                }
-            }
-            return;
+            load(f[i], b0 + PB + i);
         }
+    }
+    if constexpr (KMAX > 1) {
+        if (kw) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int r = tile * 16 + 4 * quarter + i;
-            if (r < W.rows) {
-                float *o = y + (size_t)t * ystride + r;
-                *o = add ? *o + acc[i] : acc[i];
+            for (int r = 0; r < RT_; r++)
+#pragma unroll
+                for (int t = 0; t < TT_; t++) part[((kw - 1) * WR + wr) * RT_ * TT_ + r * TT_ + t][lane] = acc[r][t];
+        }
+        __syncthreads();
+        if (kw == 0) {
+#pragma unroll
+            for (int k = 1; k < KMAX; k++) {
+                if (k >= KS) break;
+#pragma unroll
+                for (int r = 0; r < RT_; r++)
+#pragma unroll
+                    for (int t = 0; t < TT_; t++) {
+                        const f32x4 p = part[((k - 1) * WR + wr) * RT_ * TT_ + r * TT_ + t][lane];
+                        acc[r][t][0] += p[0]; acc[r][t][1] += p[1]; acc[r][t][2] += p[2]; acc[r][t][3] += p[3];
+                    }
             }
         }
     }
+    if constexpr (EPI == 2) {
+        float4 h[TT_];
+        float am[TT_];
+        if (kw == 0) {
+#pragma unroll
+            for (int t = 0; t < TT_; t++) {
+                const f32x4 g = acc[0][t], u = acc[RT_ - 1][t];
+                h[t] = make_float4(silu_mul(u[0], g[0]), silu_mul(u[1], g[1]), silu_mul(u[2], g[2]), silu_mul(u[3], g[3]));
+                float m = fmaxf(fmaxf(fabsf(h[t].x), fabsf(h[t].y)), fmaxf(fabsf(h[t].z), fabsf(h[t].w))), lo, hi;
+                swap16(m, lo, hi); m = fmaxf(lo, hi);
+                swap32(m, lo, hi); am[t] = fmaxf(lo, hi);
+                if (quarter == 0) amx[wr * TT_ + t][c16] = am[t];
+            }
+        }
+        __syncthreads();
+        if (kw == 0) {
+#pragma unroll
+            for (int t = 0; t < TT_; t++) {
+                const int tok = 16 * tt[t] + c16;
+                const float m = fmaxf(am[t], amx[(wr ^ 1) * TT_ + t][c16]);   // WR = 2: the block's other 16 rows
+                const float inv = m > 0.f ? 127.0f / m : 0.f;
+                const int q0 = (int)rintf(h[t].x * inv), q1 = (int)rintf(h[t].y * inv), q2 = (int)rintf(h[t].z * inv), q3 = (int)rintf(h[t].w * inv);
+                if (tok < G.P) {
+                    const size_t slot = pf_slot(tok, blockIdx.x, G.W.tiles >> 2);
+                    *(uint32_t *)(G.out.q + slot * 32 + 16 * wr + 4 * quarter) =
+                        (uint32_t)(q0 & 255) | (uint32_t)(q1 & 255) << 8 | (uint32_t)(q2 & 255) << 16 | (uint32_t)(q3 & 255) << 24;
+                    if (wr == 0 && quarter == 0) G.out.s[slot] = m / 127.0f;
+                }
+            }
+        }
+        return;
+    }
+    if (kw) return;
+#pragma unroll
+    for (int r = 0; r < RT_; r++)
+#pragma unroll
+        for (int t = 0; t < TT_; t++) {
+            const int tok = 16 * tt[t] + c16, r0 = 16 * rt[r] + 4 * quarter;
+            if (tok >= G.P || r0 >= G.W.rows) continue;
+            f32x4 v = acc[r][t];
+            if constexpr (EPI == 0) {                 // rows: whole 32-blocks
+                float4 *o = (float4 *)(G.y + (size_t)tok * G.ystride + r0);
+                const float4 x = *o;
+                *o = make_float4(x.x + v[0], x.y + v[1], x.z + v[2], x.w + v[3]);
+            } else {
+                // q, k and v rows each begin at a multiple of 8: the four rows lie in one of them
+                const bool isq = r0 < G.nq, isv = r0 >= G.nq + G.nk;
+                const int e = isq ? r0 : isv ? r0 - G.nq - G.nk : r0 - G.nq, hh = e / G.hd, j = e - hh * G.hd;
+                if (!isv) {
+                    const float4 cs = *(const float4 *)(G.rope + (size_t)tok * G.hd + j);   // the two pairs' (cos, sin)
+                    const float a = v[0], b = v[1], c = v[2], d = v[3];
+                    v[0] = a * cs.x - b * cs.y; v[1] = a * cs.y + b * cs.x;
+                    v[2] = c * cs.z - d * cs.w; v[3] = c * cs.w + d * cs.z;
+                }
+                if (isq) *(float4 *)(G.y + (size_t)tok * G.ystride + r0) = make_float4(v[0], v[1], v[2], v[3]);
+                else *(uint2 *)((isv ? G.vc : G.kc) + (((size_t)G.layer * G.n_kv + hh) * G.ctx + tok) * G.hd + j) =
+                    make_uint2((uint32_t)f32_bf16(v[0]) | (uint32_t)f32_bf16(v[1]) << 16, (uint32_t)f32_bf16(v[2]) | (uint32_t)f32_bf16(v[3]) << 16);
+            }
+        }
 }
 
 // The form for the other head dims (k_pf_attn takes multiples of 16 up to 128).
 // Attention of token t, head h over positions 0..t (ops.c:42-73): one wavefront per (t, h), positions in
 // chunks of 64 (a lane per position) with a running maximum and sum; then each lane sums its output
-// dims over the chunk's weights. q from qkv (after RoPE), K and V from the cache as bf16.
-__global__ void __launch_bounds__(64) k_pf_attend(const float *qkv, int P, int n_heads, int n_kv, int hd, int ctx, int layer,
-                                                  float scale, const uint16_t *kc, const uint16_t *vc, float *att, uint8_t *act,
-                                                  int astride) {
+// dims over the chunk's weights. q from qb (after RoPE), K and V from the cache as bf16.
+__global__ void __launch_bounds__(64) k_pf_attend(const float *qb, int P, int n_heads, int n_kv, int hd, int ctx, int layer,
+                                                  float scale, const uint16_t *kc, const uint16_t *vc, float *att) {
     constexpr int VMAX = 32;                          // V rows a lane loads per 64-position chunk (h8 <= 32)
     __shared__ float qs[256], ps[64], part[64 * 8];
     const int t = blockIdx.x, h = blockIdx.y, lane = tidx(), hpk = n_heads / n_kv, kv = h / hpk;
-    const int width = n_heads * hd + 2 * n_kv * hd, h8 = hd >> 3;
+    const int width = n_heads * hd, h8 = hd >> 3;
     // P.V: lane = jg * h8 + dg takes dims [8 dg, 8 dg + 8) at positions jg, jg + JG, ... of a chunk
     const int JG = 64 / h8, jg = lane / h8, dg = lane - jg * h8;
     const bool vlane = jg < JG;
-    for (int d = lane; d < hd; d += 64) qs[d] = qkv[(size_t)t * width + h * hd + d];
+    for (int d = lane; d < hd; d += 64) qs[d] = qb[(size_t)t * width + h * hd + d];
     __syncthreads();
     const uint16_t *K = kc + ((size_t)layer * n_kv + kv) * ctx * hd, *V = vc + ((size_t)layer * n_kv + kv) * ctx * hd;
     float m = -INFINITY, l = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};   // output dims lane, lane + 64, ... (hd <= 256)
@@ -3326,31 +3445,6 @@ __global__ void __launch_bounds__(64) k_pf_attend(const float *qkv, int P, int n
         m = nm;
         __syncthreads();
     }
-    if (act) {
-        // hd a multiple of 32: the head's 32-blocks of the output prepared here, as k_pf_prep would (per block
-        // amax, inv = 127 / amax, q = rint(x * inv), the scale amax / 127 and the sum of q), into act[t]
-        uint8_t *row = act + (size_t)t * astride;
-        const int nb = (n_heads * hd) >> 5;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            if (64 * i >= hd) break;                  // uniform; a group of 32 lanes is a whole block or past hd
-            const int d = lane + 64 * i;
-            const float x = d < hd ? o[i] / l : 0.f;
-            const float am = lanes_max<32>(fabsf(x));
-            const float inv = am > 0.f ? 127.0f / am : 0.f;
-            const int q = (int)rintf(x * inv);
-            const float qs32 = lanes_sum<32>((float)q);   // |sum| <= 32 * 127: exact in float
-            if (d < hd) {
-                const int blk = (h * hd + d) >> 5;
-                row[h * hd + d] = (uint8_t)(q & 255);
-                if ((lane & 31) == 0) {
-                    ((float *)(row + 32 * nb))[blk] = am / 127.0f;
-                    ((int *)(row + 36 * nb))[blk] = (int)qs32;
-                }
-            }
-        }
-        return;
-    }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int d = lane + 64 * i;
@@ -3374,8 +3468,8 @@ __global__ void __launch_bounds__(64) k_pf_attend(const float *qkv, int P, int n
 // per token and head, a lane per position: every token reads every K and V row again); 63 tokens: 5.0 (7.0).
 constexpr int PFA_W = 4, PFA_T = 16, PFA_C = 32, PFA_VROW = 40;
 template <int HD>
-__global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qkv, int P, int n_heads, int n_kv, int ctx, int layer, float scale,
-                                                        const uint16_t *kc, const uint16_t *vc, float *att, uint8_t *act, int astride) {
+__global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qb, int P, int n_heads, int n_kv, int ctx, int layer, float scale,
+                                                        const uint16_t *kc, const uint16_t *vc, float *att, l3m_pfact act) {
     constexpr int KS = (HD + 31) / 32, NT16 = HD / 16, D8 = HD / 8, UNITS = (HD + 63) / 64, OROW = HD + 4;
     constexpr size_t VT = (size_t)HD * PFA_VROW * 2;                     // one wavefront's V^T chunk; its merge span is no larger
     static_assert((size_t)PFA_T * OROW * 4 <= VT, "the merge spans fit the V^T spans");
@@ -3384,14 +3478,14 @@ __global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qkv, int P,
     const int lane = tidx() & 63, wave = wave_id(), c16 = lane & 15, quarter = lane >> 4;
     // the tiles with the most positions first
     const int t0 = PFA_T * ((int)gridDim.x - 1 - (int)blockIdx.x), h = blockIdx.y, kv = h / (n_heads / n_kv);
-    const int width = (n_heads + 2 * n_kv) * HD, tmax = (t0 + PFA_T < P ? t0 + PFA_T : P) - 1, tok = min(t0 + c16, tmax);
+    const int width = n_heads * HD, tmax = (t0 + PFA_T < P ? t0 + PFA_T : P) - 1, tok = min(t0 + c16, tmax);
     const uint16_t *K = kc + ((size_t)layer * n_kv + kv) * ctx * HD, *V = vc + ((size_t)layer * n_kv + kv) * ctx * HD;
     uint16_t *vt = (uint16_t *)(lds + wave * VT);
     bf16x8 q[3][KS];
 #pragma unroll
     for (int s = 0; s < KS; s++) {
         const int d = 32 * s + 8 * quarter;
-        const float *src = qkv + (size_t)tok * width + h * HD + (d < HD ? d : 0);
+        const float *src = qb + (size_t)tok * width + h * HD + (d < HD ? d : 0);
         const float4 a = ldg16f(src, 0), b = ldg16f(src, 1);
         const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
@@ -3513,21 +3607,8 @@ __global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qkv, int P,
             y.x += x.x * f; y.y += x.y * f; y.z += x.z * f; y.w += x.w * f;
         }
         y = make_float4(y.x / den, y.y / den, y.z / den, y.w / den);
-        if constexpr (HD % 32 == 0) {
-            // the head's 32-blocks prepared here (8 lanes a block, prep_body's formulas)
-            const float am = lanes_max<8>(fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w))));
-            const float inv = am > 0.f ? 127.0f / am : 0.f;
-            const int q0 = (int)rintf(y.x * inv), q1 = (int)rintf(y.y * inv), q2 = (int)rintf(y.z * inv), q3 = (int)rintf(y.w * inv);
-            const int sum = lanes_sumi<8>(q0 + q1 + q2 + q3);
-            if (t < P) {
-                uint8_t *row = act + (size_t)t * astride;
-                const int nb = (n_heads * HD) >> 5, e = h * HD + 4 * d4;
-                *(uint32_t *)(row + e) = (uint32_t)(q0 & 255) | (uint32_t)(q1 & 255) << 8 | (uint32_t)(q2 & 255) << 16 | (uint32_t)(q3 & 255) << 24;
-                if ((d4 & 7) == 0) {
-                    ((float *)(row + 32 * nb))[e >> 5] = am / 127.0f;
-                    ((int *)(row + 36 * nb))[e >> 5] = sum;
-                }
-            }
+        if constexpr (HD % 32 == 0) {                 // whole blocks of the head: prepared here, 8 lanes a block
+            pf_put4(act, t, (n_heads * HD) >> 5, h * HD + 4 * d4, y, t < P);
         } else if (t < P) {
             *(float4 *)(att + (size_t)t * n_heads * HD + h * HD + 4 * d4) = y;
         }
@@ -3840,17 +3921,46 @@ template <int DT, int HDT, bool G2> int decode_fits(int hd, int grid, unsigned l
     return decode_fits_hd<DT, HDT, G2, 0>(grid, lds);
 }
 
+// k_pf_rows for rows of k <= 4096 values.
+template <bool NORM> void pf_rows(const float *y, int k, const float *w, float eps, const l3m_pfact &act, int P, hipStream_t st) {
+    const dim3 grid((P + 3) / 4), block(256);
+    if (k <= 512) hipLaunchKernelGGL((k_pf_rows<NORM, 2>), grid, block, 0, st, y, k, w, eps, act, P);
+    else if (k <= 1024) hipLaunchKernelGGL((k_pf_rows<NORM, 4>), grid, block, 0, st, y, k, w, eps, act, P);
+    else hipLaunchKernelGGL((k_pf_rows<NORM, 16>), grid, block, 0, st, y, k, w, eps, act, P);
+}
+
 // The prompt's attention in layer l: on the matrix cores for head dims of 16, 32, ... 128 (k_pf_attn), else
-// k_pf_attend.
-void pf_attention(const l3m_dmodel *M, const l3m_pfbuf *B, int P, int l, bool fuse, hipStream_t st) {
+// k_pf_attend; its output prepared into B->act.
+void pf_attention(const l3m_dmodel *M, const l3m_pfbuf *B, int P, int l, hipStream_t st) {
+    const float *q = B->q;
+    const uint16_t *kc = M->kc, *vc = M->vc;
+    const int hd = M->hd, nq = M->n_heads * hd;
+    const dim3 grid((P + PFA_T - 1) / PFA_T, M->n_heads), block(64 * PFA_W);
 #define PF_ATTN(HD) \
-    case HD: hipLaunchKernelGGL(k_pf_attn<HD>, dim3((P + PFA_T - 1) / PFA_T, M->n_heads), dim3(64 * PFA_W), 0, st, (const float *)B->qkv, P, \
-                                M->n_heads, M->n_kv, M->ctx, l, M->att_scale, (const uint16_t *)M->kc, (const uint16_t *)M->vc, B->att, \
-                                B->act, B->astride); return;
-    switch (M->hd) { PF_ATTN(16) PF_ATTN(32) PF_ATTN(48) PF_ATTN(64) PF_ATTN(80) PF_ATTN(96) PF_ATTN(112) PF_ATTN(128) }
+    case HD: hipLaunchKernelGGL(k_pf_attn<HD>, grid, block, 0, st, q, P, M->n_heads, M->n_kv, M->ctx, l, M->att_scale, kc, vc, B->att, B->act); break;
+    switch (hd) {
+        PF_ATTN(16) PF_ATTN(32) PF_ATTN(48) PF_ATTN(64) PF_ATTN(80) PF_ATTN(96) PF_ATTN(112) PF_ATTN(128)
+    default:
+        hipLaunchKernelGGL(k_pf_attend, dim3(P, M->n_heads), dim3(64), 0, st, q, P, M->n_heads, M->n_kv, hd, M->ctx, l, M->att_scale, kc, vc, B->att);
+    }
 #undef PF_ATTN
-    hipLaunchKernelGGL(k_pf_attend, dim3(P, M->n_heads), dim3(64), 0, st, (const float *)B->qkv, P, M->n_heads, M->n_kv, M->hd, M->ctx, l,
-                       M->att_scale, (const uint16_t *)M->kc, (const uint16_t *)M->vc, B->att, fuse ? B->act : nullptr, B->astride);
+    if (hd % 32 || hd > 128)                          // blocks across heads, or the form that prepares nothing
+        pf_rows<false>(B->att, nq, nullptr, 0.f, B->act, P, st);
+}
+
+// One matrix of the prompt. Three splits, by how many 32-row x 32-token tiles there are (for EPI 2 16 gate and 16
+// up rows): many, a wavefront a tile over all blocks, two side by side; fewer, a tile's ranges split over 4
+// wavefronts; fewest, 32 x 16 tiles with the ranges split over up to 8. Measured (30 layers of dim 576, ffn 1536;
+// us to the first logits, each split for every matrix): 64 tokens 2065 / 1685 / 1509, 200 tokens 2282 / 1918 /
+// 1941, 480 tokens 2549 / 2394 / 2846; gate and up alone at 480 tokens 12.0 / 15.1 / 25.9 us, at 64 - / 7.6 / 7.0.
+constexpr int PF_WIDE = 1024;
+template <int EPI> void pf_gemm(const PfGemm &G, hipStream_t st) {
+    constexpr int WR = EPI == 2 ? 2 : 1, MID = EPI == 2 ? 256 : 160;
+    const int rows = EPI == 2 ? G.W.tiles * 8 : G.W.rows;   // EPI 2: the ffn rows
+    const int r32 = (rows + 31) / 32, t32 = (G.P + 31) / 32, R = pf_ranges(G.W.nb), n = WR * r32 * t32;
+    if (n >= PF_WIDE) hipLaunchKernelGGL((k_pf_gemm<EPI, 2, 2, 2, 1>), dim3(EPI == 2 ? r32 : (r32 + 1) / 2, t32), dim3(128), 0, st, G);
+    else if (n >= MID) hipLaunchKernelGGL((k_pf_gemm<EPI, 2, 2, WR, 4>), dim3(r32, t32), dim3(64 * WR * min(R, 4)), 0, st, G);
+    else hipLaunchKernelGGL((k_pf_gemm<EPI, 2, 1, WR, 8>), dim3(r32, (G.P + 15) / 16), dim3(64 * WR * min(R, 8)), 0, st, G);
 }
 
 template <int DT> int launch_step_mv(int form, const l3m_dmat &m, const float *x, int k, float *y, int tpw, hipStream_t st) {
@@ -4223,8 +4333,8 @@ int l3m_step_slots(int dtype, int which) {
     return dtype == L3M_F32 ? nslot_a<L3M_F32>() : dtype == L3M_BF16 ? nslot_a<L3M_BF16>() : dtype == L3M_Q8_0 ? nslot_a<L3M_Q8_0>() : nslot_a<L3M_Q4_0>();
 }
 
-// The shapes the prefill kernels take: one workgroup's 4 values per thread cover dim, ffn and n_heads * hd
-// (the per-token norm and prep), and k_pf_attend's q row and outputs cover hd.
+// The shapes the prefill takes: rows of dim and n_heads * hd values fit k_pf_rows (16 pieces of 256),
+// k_pf_attend's q row and outputs cover hd; longer ffn rows go token by token.
 int l3m_prefill_fits(int dim, int ffn, int nqd, int hd) {
     return dim <= 4 * NTE && ffn <= 4 * NTE && nqd <= 4 * NTE && hd <= 256 && hd % 2 == 0;
 }
@@ -4233,29 +4343,26 @@ int l3m_prefill(const l3m_dmodel *M, const l3m_pflayer *L, const l3m_pfbuf *B, i
     if (P < 1) return 0;
     if (P > M->ctx || !l3m_prefill_fits(M->dim, M->ffn, M->n_heads * M->hd, M->hd)) return fail_msg("prefill: shape out of range");
     hipStream_t st = as_stream(stream);
-    const int dim = M->dim, hd = M->hd, nq = M->n_heads * hd, width = nq + 2 * M->n_kv * hd;
-    const PfQkv none{}, qkv_out{M->rope, M->kc, M->vc, 0, M->ctx, nq, M->n_kv * hd, hd, M->n_kv};
-    auto gemm = [&](const l3m_dmat &W, float *y, int ystride, int add, const PfQkv *E) {
-        const dim3 grid(W.tiles, (P + 15) / 16), block(64 * pf_split(W.nb));
-        if (E) hipLaunchKernelGGL(k_pf_gemm<true>, grid, block, 0, st, W, (const uint8_t *)B->act, B->astride, P, y, ystride, add, *E);
-        else hipLaunchKernelGGL(k_pf_gemm<false>, grid, block, 0, st, W, (const uint8_t *)B->act, B->astride, P, y, ystride, add, none);
-    };
+    const int dim = M->dim, hd = M->hd, nq = M->n_heads * hd;
     hipLaunchKernelGGL(k_pf_embed, dim3(P), dim3(NTE), 0, st, M->embed, (const int32_t *)M->tokens, dim, B->x);
     for (int l = 0; l < M->n_layers; l++) {
         const l3m_pflayer &W = L[l];
-        hipLaunchKernelGGL(k_pf_norm_prep, dim3(P), dim3(NTE), 0, st, (const float *)B->x, W.attn_norm, dim, M->eps, B->act, B->astride);
-        PfQkv E = qkv_out;                            // q (after RoPE) into qkv, k and v into the cache
-        E.layer = l;
-        gemm(W.qkv, B->qkv, width, 0, &E);
+        PfGemm G{};
+        G.P = P;
+        pf_rows<true>(B->x, dim, W.attn_norm, M->eps, B->act, P, st);
+        // q (after RoPE) into B->q, k and v into the cache
+        G.W = W.qkv; G.x = B->act; G.y = B->q; G.ystride = nq;
+        G.rope = M->rope; G.kc = M->kc; G.vc = M->vc; G.layer = l; G.ctx = M->ctx; G.nq = nq; G.nk = M->n_kv * hd; G.hd = hd; G.n_kv = M->n_kv;
+        pf_gemm<1>(G, st);
         if (l == M->n_layers - 1) break;              // the last layer's K/V rows are all its prompt positions leave
-        const bool fuse = hd % 32 == 0;               // whole blocks per head: the attention prepares its output
-        pf_attention(M, B, P, l, fuse, st);
-        if (!fuse) hipLaunchKernelGGL(k_pf_prep, dim3(P), dim3(NTE), 0, st, (const float *)B->att, nq, nq, B->act, B->astride);
-        gemm(W.wo, B->x, dim, 1, nullptr);
-        hipLaunchKernelGGL(k_pf_norm_prep, dim3(P), dim3(NTE), 0, st, (const float *)B->x, W.ffn_norm, dim, M->eps, B->act, B->astride);
-        gemm(W.gu, B->gu, 2 * M->ffn, 0, nullptr);
-        hipLaunchKernelGGL(k_pf_silu_prep, dim3(P), dim3(NTE), 0, st, (const float *)B->gu, M->ffn, B->act, B->astride);
-        gemm(W.down, B->x, dim, 1, nullptr);
+        pf_attention(M, B, P, l, st);
+        G.W = W.wo; G.y = B->x; G.ystride = dim;
+        pf_gemm<0>(G, st);
+        pf_rows<true>(B->x, dim, W.ffn_norm, M->eps, B->act, P, st);
+        G.W = W.gu; G.out = B->hact;
+        pf_gemm<2>(G, st);
+        G.W = W.down; G.x = B->hact;
+        pf_gemm<0>(G, st);
     }
     CKL("prefill");
     return 0;

@@ -206,3 +206,32 @@ def test_prefill_attention_head_dims(models, oracle, hd, n_prompt):
             for got, want in zip(m.kv_rows(1, kvh, 0, n_prompt - 1), om.kv_rows(1, kvh, 0, n_prompt - 1, hd)):
                 g, w = bf16(got), bf16(want)
                 assert np.abs(g - w).max() <= 0.02 * np.abs(w).max(), kvh
+
+
+# 33 tiles of 32 output rows in Wo and Wdown, 99 in q/k/v, 65 blocks of ffn: odd counts at every split of the GEMM
+WIDE = A.Config("pf_wide", dim=1056, n_layers=2, n_heads=11, n_kv_heads=11, ffn_dim=2080, vocab=512, ctx=1024, dtype="q8_0")
+
+
+@pytest.mark.parametrize("n_prompt", [34, 162, 500, 1000])
+def test_prefill_gemm_splits(models, monkeypatch, n_prompt):
+    """The GEMM's three splits: 32 x 16 tiles over up to 8 wavefronts (Wo and Wdown at 33 positions), 32 x 32 tiles
+    over 4 (q/k/v and gate/up at 33, all at 161, Wo and Wdown at 499), a wavefront a tile (q/k/v and gate/up at
+    499, all at 999), with ragged last token tiles. Against the GPU's token-by-token path: the logits' bar of
+    test_prefill_logits, the K/V rows within 2% of the largest, the first layer's (one matrix, before activation
+    rounding can cascade) within 0.5%."""
+    path = models.get(WIDE, "q8_0", seed=13, std=0.03, norm_jitter=0.1)
+    ids = A.prompt(14, WIDE.vocab, n_prompt)
+    out = []
+    for prefill in ("1", "0"):
+        monkeypatch.setenv("L3M_PREFILL", prefill)
+        with A.Model(path, ctx=1024) as m:
+            m.generate(ids, 0)
+            assert m.prefilled == (n_prompt - 1 if prefill == "1" else 0)
+            out.append((m.logits, [[m.kv_rows(layer, kvh, 0, n_prompt - 1) for kvh in (0, 5, 10)] for layer in (0, 1)]))
+    (lf, kf), (ls, ks) = out
+    assert close(lf, ls), (kl(ls, lf), np.abs(lf - ls).max() / np.abs(ls).max())
+    for layer, bar in ((0, 0.005), (1, 0.02)):
+        for got, want in zip(kf[layer], ks[layer]):
+            for g, w in zip(got, want):
+                g, w = bf16(g), bf16(w)
+                assert np.abs(g - w).max() <= bar * np.abs(w).max(), (layer, np.abs(g - w).max() / np.abs(w).max())
