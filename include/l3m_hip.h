@@ -219,7 +219,7 @@ int    l3m_phase_stamps(int mode, int pos, int layer, unsigned long long *out);
 // greedy tokens are checked against the logits they came from).
 int    l3m_logits_at(const l3m_model *m, int pos, float *out);
 // Prompt positions the last generate call ran as one batched prefill (0: token by token). Prompts of at
-// least L3M_PREFILL_MIN (default 8) tokens on q8_0 and q4_0 bodies (and mxfp4 bodies whose blocks widen
+// least L3M_PREFILL_MIN (default 8) tokens on bf16, q8_0 and q4_0 bodies (and mxfp4 bodies whose blocks widen
 // exactly to q8_0) are prefilled unless L3M_PREFILL=0.
 int    l3m_prefill_positions(const l3m_model *m);
 // The attention mode the decode step of m runs at positions inside its K/V window (l3m_attention_mode's

@@ -229,13 +229,13 @@ static const float *vec_or_zero(l3m_model *m, const l3m_mapped *f, int l, const 
     return d;
 }
 
-// A prefill matrix: q8_0 lane tiles (q4_0 widened as the step matrices are; mxfp4 widened exactly).
+// A prefill matrix: bf16 or q8_0 lane tiles (q4_0 widened as the step matrices are; mxfp4 widened exactly).
 static int upload_pf_mat(l3m_model *m, l3m_dmat *out, int src_dtype, int rows, int k, const void *const *src) {
     if (src_dtype == L3M_MXFP4 || src_dtype == L3M_Q4_0) return upload_widened(m, out, src_dtype, rows, k, src);
     return upload_step_mat(m, out, src_dtype, rows, k, src);
 }
 
-// The prefill matrices of layer l: the whole wq|wk|wv, wo, w_gate|w_up and w_down as q8_0 lane tiles. A second copy of the body, not counted in the bytes a decode
+// The prefill matrices of layer l: the whole wq|wk|wv, wo, w_gate|w_up and w_down as lane tiles. A second copy of the body, not counted in the bytes a decode
 // step streams.
 static int upload_prefill(l3m_model *m, const l3m_mapped *f, int l, int dt, const l3m_dlayer *L) {
     const l3m_dmodel *d = &m->dm;
@@ -265,7 +265,7 @@ static int upload_prefill(l3m_model *m, const l3m_mapped *f, int l, int dt, cons
     P->ffn_norm = L->ffn_norm;
     m->weight_bytes = before;
     free(rows);
-    return rc || P->qkv.dtype != L3M_Q8_0 ? -1 : 0;
+    return rc || P->qkv.dtype != (dt == L3M_BF16 ? L3M_BF16 : L3M_Q8_0) ? -1 : 0;
 }
 
 // The file row starting at input column c (whole 32-blocks for quantized rows).
@@ -370,12 +370,12 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
     if (d->n_groups > MAX_PARTS || d->n_chunks > MAX_PARTS) return fail(m, "too many head groups or FFN chunks for the GPU kernels");
     l3m_model_layout(d);
     m->layers = calloc((size_t)d->n_layers, sizeof *m->layers);
-    // batched prefill (q8_0 and q4_0 bodies, and mxfp4 bodies whose blocks widen exactly to q8_0; whole
+    // batched prefill (bf16, q8_0 and q4_0 bodies, and mxfp4 bodies whose blocks widen exactly to q8_0; whole
     // 32-blocks): unless L3M_PREFILL=0
     const char *pe_ = getenv("L3M_PREFILL"), *pm_ = getenv("L3M_PREFILL_MIN");
     const int qb_ = d->dim % 32 == 0 && (d->n_heads * d->hd) % 32 == 0 && d->ffn % 32 == 0;
     if ((!pe_ || strcmp(pe_, "0")) && !m->reference && !gpt2 && qb_ && l3m_prefill_fits(d->dim, d->ffn, d->n_heads * d->hd, d->hd) &&
-        (m->dtype == L3M_Q8_0 || m->dtype == L3M_Q4_0 || m->mx_wide || (m->dtype == L3M_MXFP4 && mxfp4_body_widens(f, d->n_layers))))
+        (m->dtype == L3M_BF16 || m->dtype == L3M_Q8_0 || m->dtype == L3M_Q4_0 || m->mx_wide || (m->dtype == L3M_MXFP4 && mxfp4_body_widens(f, d->n_layers))))
         m->pf = calloc((size_t)d->n_layers, sizeof *m->pf);
     m->prefill_min = pm_ ? atoi(pm_) : 8;
     l3m_dgroup *groups = calloc((size_t)d->n_groups, sizeof *groups);
@@ -552,9 +552,10 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
         // activations of whole 64-token groups (a GEMM's workgroup reads up to 64 tokens)
         const size_t nqd = (size_t)d->n_heads * d->hd, mk = (size_t)d->dim > nqd ? (size_t)d->dim : nqd, ctx = (size_t)d->ctx, c64 = (ctx + 63) / 64 * 64;
         m->pfb.x = dalloc(m, ctx * d->dim * 4);
-        m->pfb.act.q = dalloc(m, c64 * mk);
+        const size_t vb = m->dtype == L3M_BF16 ? 2 : 1;
+        m->pfb.act.q = dalloc(m, c64 * mk * vb);
         m->pfb.act.s = dalloc(m, c64 * mk / 32 * 4);
-        m->pfb.hact.q = dalloc(m, c64 * d->ffn);
+        m->pfb.hact.q = dalloc(m, c64 * d->ffn * vb);
         m->pfb.hact.s = dalloc(m, c64 * d->ffn / 32 * 4);
         m->pfb.q = dalloc(m, ctx * nqd * 4);
         m->pfb.att = dalloc(m, ctx * nqd * 4);

@@ -145,7 +145,7 @@ int      l3m_step_slots(int dtype, int which);   // weight slots per lane (matri
 int      l3m_step_a_dtype(int dtype);            // storage dtype of a step kernel's matrix A for a body of dtype
 int l3m_step_enqueue(const l3m_dmodel *m, const l3m_dlayer *layers, int with_head, void *stream);
 
-// Batched prompt prefill: the full matrices of each layer as q8_0 lane-tile planes (q4_0 widened), and
+// Batched prompt prefill: the full matrices of each layer as q8_0 (q4_0 and mxfp4 widened) or bf16 lane-tile planes, and
 // the activation buffers of up to ctx tokens.
 typedef struct {
     l3m_dmat     qkv;            // (n_heads + 2 n_kv) hd rows (q, then k, then v) x dim
@@ -155,7 +155,7 @@ typedef struct {
     const float *attn_norm, *ffn_norm;
 } l3m_pflayer;
 // A prepared activation of the prompt's tokens, in blocks of 16 tokens x 32 inputs (kernels.hip, pf_slot): values
-// [ceil64(ctx) / 16][k / 32][16][32] and block scales [ceil64(ctx) / 16][k / 32][16].
+// [ceil64(ctx) / 16][k / 32][16][32], int8 or bf16, and int8's block scales [ceil64(ctx) / 16][k / 32][16].
 typedef struct {
     uint8_t *q;
     float   *s;

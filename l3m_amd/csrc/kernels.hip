@@ -3101,11 +3101,10 @@ __global__ void __launch_bounds__(NTE) k_where(int *out) {
 
 // ------------------------------------------------------------------ batched prompt prefill
 // The prompt positions before the last one, all at once: per layer, the same
-// operations as the decode step (engine.c:230-275) on P tokens, with the matrices as int8 GEMMs on the
-// matrix cores. The decode path then runs from the last prompt position on, over the K/V rows these
-// kernels wrote. Weights are q8_0 lane-tile planes of the full matrices (q4_0 widened exactly); the
-// activations of token t are its own int8 prep (act_size bytes at t * astride), as the decode step
-// prepares them.
+// operations as the decode step (engine.c:230-275) on P tokens, with the matrices as GEMMs on the matrix
+// cores. The decode path then runs from the last prompt position on, over the K/V rows these kernels wrote.
+// Weights are lane-tile planes of the full matrices, q8_0 (DT; q4_0 and mxfp4 widened exactly) or bf16; each
+// token's activation is prepared as the decode step prepares it.
 
 // x[t] = the embedding row of tokens[t] (engine.c:236), t < P; one workgroup per token.
 __global__ void __launch_bounds__(NTE) k_pf_embed(l3m_dmat embed, const int32_t *tokens, int dim, float *x) {
@@ -3115,14 +3114,23 @@ __global__ void __launch_bounds__(NTE) k_pf_embed(l3m_dmat embed, const int32_t 
 
 // A prefill activation: per 16 tokens and 32-input block the tokens' blocks, [token / 16][block][16][32] int8
 // with its scale beside it in [token / 16][block][16] (the prep of pack.c:101-123; the block sums are not
-// needed), so that a product's operand is one contiguous run, as a weight tile's is. Rows of tokens past the
+// needed), or [token / 16][block][16][32] bf16, so that a product's operand is one contiguous run, as a weight
+// tile's is. Rows of tokens past the
 // prompt's end hold whatever was there: a product's column depends on its own token alone, and theirs are not
 // stored.
 __device__ __forceinline__ size_t pf_slot(int t, int b, int nb) { return ((size_t)(t >> 4) * nb + b) * 16 + (t & 15); }
 
+__device__ __forceinline__ uint2 pack_bf16(float4 y) {
+    return make_uint2((uint32_t)f32_bf16(y.x) | (uint32_t)f32_bf16(y.y) << 16, (uint32_t)f32_bf16(y.z) | (uint32_t)f32_bf16(y.w) << 16);
+}
 // Values e .. e + 3 (e a multiple of 4) of token t's activation, 8 consecutive lanes a block: prep_body's
 // formulas. All lanes of a block take part; store: whether they write.
+template <int DT>
 __device__ __forceinline__ void pf_put4(const l3m_pfact &a, int t, int nb, int e, float4 y, bool store) {
+    if constexpr (DT == L3M_BF16) {
+        if (store) *(uint2 *)(a.q + pf_slot(t, e >> 5, nb) * 64 + 2 * (e & 31)) = pack_bf16(y);
+        return;
+    }
     const float am = lanes_max<8>(fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w))));
     const float inv = am > 0.f ? 127.0f / am : 0.f;
     const int q0 = (int)rintf(y.x * inv), q1 = (int)rintf(y.y * inv), q2 = (int)rintf(y.z * inv), q3 = (int)rintf(y.w * inv);
@@ -3136,7 +3144,7 @@ __device__ __forceinline__ void pf_put4(const l3m_pfact &a, int t, int nb, int e
 // values a lane for every 256, the sum of squares added as norm_prep adds it (per 256, then the 16 slots'
 // tree). One wavefront per token instead of a 1024-thread workgroup, no LDS or barrier: 479 tokens of 576
 // values 4.7 us, as before (4.8): what is left is one kernel's fixed cost, loads and launch.
-template <bool NORM, int C>                          // C: 256-value pieces of a row
+template <int DT, bool NORM, int C>                  // C: 256-value pieces of a row
 __global__ void __launch_bounds__(256) k_pf_rows(const float *y, int k, const float *w, float eps, l3m_pfact act, int P) {
     const int t = 4 * blockIdx.x + wave_id(), lane = tidx() & 63, nb = k >> 5;
     if (t >= P) return;
@@ -3165,31 +3173,32 @@ __global__ void __launch_bounds__(256) k_pf_rows(const float *y, int k, const fl
         const int e = 256 * c + 4 * lane;
         float4 x = v[c];
         if constexpr (NORM) x = make_float4(x.x * s * nw[c].x, x.y * s * nw[c].y, x.z * s * nw[c].z, x.w * s * nw[c].w);
-        pf_put4(act, t, nb, e, x, e < k);
+        pf_put4<DT>(act, t, nb, e, x, e < k);
     }
 }
 
-// The matrices of a prompt (the q8_0 gemv of every token at once, kernels_scalar.c:30-45): per 16 rows x 16
-// tokens and 32-input block one v_mfma_i32_16x16x32_i8, its i32 result scaled by the row's and the token's
-// block scales into the f32 sum, blocks in order. Lane l holds row (token) l % 16, 8 bytes at byte 8 (l / 16) of
-// the block, and gets rows 4 (l / 16) + i of token l % 16.
+// The matrices of a prompt (the gemv of every token at once, kernels_scalar.c:16-45): per 16 rows x 16 tokens and
+// 32-input block one product. q8_0: v_mfma_i32_16x16x32_i8, its i32 result scaled by the row's and the token's
+// block scales into the f32 sum; bf16: v_mfma_f32_16x16x32_bf16 onto the f32 sum. Blocks in order. Lane l holds
+// row (token) l % 16, the 8 values at 8 (l / 16) of the block, and gets rows 4 (l / 16) + i of token l % 16.
 //
 // A row's blocks fall into ranges of PF_RANGE blocks or so (pf_ranges), each summed by itself, then added in
 // order. A wavefront takes RT x TT tiles over its share of the ranges: KS = blockDim / (64 WR) wavefronts split
-// them, and their sums are added in order through LDS; WR wavefronts of each share lie side by side. Operands come straight from L2 in the layouts they lie in (512 contiguous bytes a tile and
-// block), PB blocks ahead; nothing is staged. Per product a lane spends 12 VALU instructions on the scales
+// them, and their sums are added in order through LDS; WR wavefronts of each share lie side by side. Operands come straight from L2 in the layouts they lie in (a contiguous run a tile and
+// block), PB blocks ahead; nothing is staged. Per q8_0 product a lane spends 12 VALU instructions on the scales
 // (48 clocks of its SIMD against 8 for the product), which bounds the largest shapes; RT = TT = 2 loads each
 // operand once for two products. The others are bound by latency, a chain of loads over few wavefronts: they
 // split the blocks (pf_gemm's rule). 479 tokens, 30 layers of dim 576 and ffn 1536 (kernel trace), against one
 // 16 x 16 tile a workgroup with each token's input in a row of its own: q/k/v 14.8 -> 7.7 us, Wo 10.8 -> 7.2,
-// gate/up 36.7 -> 12.0 with the SiLU and prep kernel (4.9) gone into it, Wdown 24.4 -> 9.3.
+// gate/up 36.7 -> 12.0 with the SiLU and prep kernel (4.9) gone into it, Wdown 24.4 -> 9.3. bf16, 199 tokens, 6
+// layers of dim 288 and ffn 768: 6.2 / 4.8 / 6.1 / 5.8 us, where the prompt had gone token by token.
 //
 // EPI 0: y += the product (the residual adds, engine.c:259, 275).
 // EPI 1: the q/k/v rows: RoPE on q and k (pairs (2i, 2i + 1) of each head rotated by angle i of position t from
 //        the host table, ops.c:29-40), q into y, the k and v rows rounded to bf16 into the cache
 //        (engine.c:247-248). A lane's four rows are two whole pairs.
 // EPI 2: gate and up rows (RT = 2: the same rows' gate tile and up tile), up * silu(gate) (ops.c:49-51) and its
-//        int8 prep into out: the workgroup's 2 x 16 rows are one 32-block of the next matrix's input.
+//        prep into out: the workgroup's 2 x 16 rows are one 32-block of the next matrix's input.
 typedef int v4i32 __attribute__((ext_vector_type(4)));
 constexpr int PF_RANGE = 4;
 __host__ __device__ inline int pf_ranges(int nb) { return min(max((nb + PF_RANGE - 1) / PF_RANGE, 1), 16); }
@@ -3202,14 +3211,15 @@ struct PfGemm {
     uint16_t *kc, *vc;
     int layer, ctx, nq, nk, hd, n_kv;
 };
-template <int RT_, int TT_> struct PfFrag {
-    long a[RT_], x[TT_];
-    u32x2 sw[RT_];
+template <int DT, int RT_, int TT_> struct PfFrag {
+    std::conditional_t<DT == L3M_BF16, bf16x8, long> a[RT_], x[TT_];
+    u32x2 sw[RT_];                                    // q8_0: the scales
     float sx[TT_];
 };
-template <int EPI, int RT_, int TT_, int WR, int KMAX>
+template <int DT, int EPI, int RT_, int TT_, int WR, int KMAX>
 __global__ void __launch_bounds__(64 * WR * KMAX) k_pf_gemm(PfGemm G) {
-    constexpr int PB = 4;
+    constexpr int PB = 4, QB = qbytes(DT);
+    using Frag = PfFrag<DT, RT_, TT_>;
     __shared__ f32x4 part[KMAX > 1 ? (KMAX - 1) * WR * RT_ * TT_ : 1][64];
     __shared__ float amx[EPI == 2 ? WR * TT_ : 1][16];
     const int lane = tidx() & 63, wave = wave_id(), c16 = lane & 15, quarter = lane >> 4;
@@ -3228,27 +3238,33 @@ __global__ void __launch_bounds__(64 * WR * KMAX) k_pf_gemm(PfGemm G) {
 #pragma unroll
     for (int r = 0; r < RT_; r++) {
         const size_t at = (size_t)min(rt[r], G.W.tiles - 1) * nb * 16;   // tiles past the last: it again, not stored
-        wq[r] = G.W.q + (at + c16) * 32 + quarter * 8;
+        wq[r] = G.W.q + (at + c16) * QB + quarter * (QB / 4);
         ws[r] = (const uint16_t *)G.W.s + at + quarter * 4;
     }
 #pragma unroll
     for (int t = 0; t < TT_; t++) {
         const size_t at = (size_t)tt[t] * nb * 16 + c16;
-        xq[t] = G.x.q + at * 32 + quarter * 8;
+        xq[t] = G.x.q + at * QB + quarter * (QB / 4);
         xs[t] = G.x.s + at;
     }
-    PfFrag<RT_, TT_> f[PB];
-    auto load = [&](PfFrag<RT_, TT_> &g, int b) {
+    Frag f[PB];
+    auto load = [&](Frag &g, int b) {
         b = min(b, nb - 1);                           // past the range: a block in bounds, not used
 #pragma unroll
         for (int r = 0; r < RT_; r++) {
-            g.a[r] = *gp<long>(wq[r] + (size_t)b * 512);
-            g.sw[r] = *gp<u32x2>(ws[r] + (size_t)b * 16);
+            if constexpr (DT == L3M_BF16) g.a[r] = __builtin_bit_cast(bf16x8, *gp<u32x4>(wq[r] + (size_t)b * 16 * QB));
+            else {
+                g.a[r] = *gp<long>(wq[r] + (size_t)b * 16 * QB);
+                g.sw[r] = *gp<u32x2>(ws[r] + (size_t)b * 16);
+            }
         }
 #pragma unroll
         for (int t = 0; t < TT_; t++) {
-            g.x[t] = *gp<long>(xq[t] + (size_t)b * 512);
-            g.sx[t] = *gp<float>(xs[t] + (size_t)b * 16);
+            if constexpr (DT == L3M_BF16) g.x[t] = __builtin_bit_cast(bf16x8, *gp<u32x4>(xq[t] + (size_t)b * 16 * QB));
+            else {
+                g.x[t] = *gp<long>(xq[t] + (size_t)b * 16 * QB);
+                g.sx[t] = *gp<float>(xs[t] + (size_t)b * 16);
+            }
         }
     };
     f32x4 acc[RT_][TT_], cur[RT_][TT_];               // the sum of the ranges done, the current range's
@@ -3263,23 +3279,30 @@ __global__ void __launch_bounds__(64 * WR * KMAX) k_pf_gemm(PfGemm G) {
 #pragma unroll
         for (int i = 0; i < PB; i++) {
             if (b0 + i < k1) {                        // uniform
-#pragma unroll
-                for (int r = 0; r < RT_; r++) {
-                    const float d[4] = {f16_f32(f[i].sw[r].x & 0xFFFF), f16_f32(f[i].sw[r].x >> 16), f16_f32(f[i].sw[r].y & 0xFFFF),
-                                        f16_f32(f[i].sw[r].y >> 16)};
-#pragma unroll
-                    for (int t = 0; t < TT_; t++) {
-                        const v4i32 c = __builtin_amdgcn_mfma_i32_16x16x32_i8(f[i].a[r], f[i].x[t], v4i32{0, 0, 0, 0}, 0, 0, 0);
-#pragma unroll
-                        for (int j = 0; j < 4; j++) cur[r][t][j] += (float)c[j] * (d[j] * f[i].sx[t]);
-                    }
-                }
-                if (b0 + i + 1 == next || b0 + i + 1 == k1) {   // uniform: the range is done
-                    next += per;
+                if constexpr (DT == L3M_BF16) {
 #pragma unroll
                     for (int r = 0; r < RT_; r++)
 #pragma unroll
-                        for (int t = 0; t < TT_; t++) { acc[r][t] += cur[r][t]; cur[r][t] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+                        for (int t = 0; t < TT_; t++) acc[r][t] = mfma_bf16(f[i].a[r], f[i].x[t], acc[r][t]);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < RT_; r++) {
+                        const float d[4] = {f16_f32(f[i].sw[r].x & 0xFFFF), f16_f32(f[i].sw[r].x >> 16), f16_f32(f[i].sw[r].y & 0xFFFF),
+                                            f16_f32(f[i].sw[r].y >> 16)};
+#pragma unroll
+                        for (int t = 0; t < TT_; t++) {
+                            const v4i32 c = __builtin_amdgcn_mfma_i32_16x16x32_i8(f[i].a[r], f[i].x[t], v4i32{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                            for (int j = 0; j < 4; j++) cur[r][t][j] += (float)c[j] * (d[j] * f[i].sx[t]);
+                        }
+                    }
+                    if (b0 + i + 1 == next || b0 + i + 1 == k1) {   // uniform: the range is done
+                        next += per;
+#pragma unroll
+                        for (int r = 0; r < RT_; r++)
+#pragma unroll
+                            for (int t = 0; t < TT_; t++) { acc[r][t] += cur[r][t]; cur[r][t] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+                    }
                 }
             }
             load(f[i], b0 + PB + i);
@@ -3315,12 +3338,18 @@ __global__ void __launch_bounds__(64 * WR * KMAX) k_pf_gemm(PfGemm G) {
             for (int t = 0; t < TT_; t++) {
                 const f32x4 g = acc[0][t], u = acc[RT_ - 1][t];
                 h[t] = make_float4(silu_mul(u[0], g[0]), silu_mul(u[1], g[1]), silu_mul(u[2], g[2]), silu_mul(u[3], g[3]));
+                if constexpr (DT == L3M_BF16) {
+                    const int tok = 16 * tt[t] + c16;
+                    if (tok < G.P) *(uint2 *)(G.out.q + pf_slot(tok, blockIdx.x, G.W.tiles >> 2) * 64 + 32 * wr + 8 * quarter) = pack_bf16(h[t]);
+                    continue;
+                }
                 float m = fmaxf(fmaxf(fabsf(h[t].x), fabsf(h[t].y)), fmaxf(fabsf(h[t].z), fabsf(h[t].w))), lo, hi;
                 swap16(m, lo, hi); m = fmaxf(lo, hi);
                 swap32(m, lo, hi); am[t] = fmaxf(lo, hi);
                 if (quarter == 0) amx[wr * TT_ + t][c16] = am[t];
             }
         }
+        if constexpr (DT == L3M_BF16) return;
         __syncthreads();
         if (kw == 0) {
 #pragma unroll
@@ -3363,7 +3392,7 @@ __global__ void __launch_bounds__(64 * WR * KMAX) k_pf_gemm(PfGemm G) {
                 }
                 if (isq) *(float4 *)(G.y + (size_t)tok * G.ystride + r0) = make_float4(v[0], v[1], v[2], v[3]);
                 else *(uint2 *)((isv ? G.vc : G.kc) + (((size_t)G.layer * G.n_kv + hh) * G.ctx + tok) * G.hd + j) =
-                    make_uint2((uint32_t)f32_bf16(v[0]) | (uint32_t)f32_bf16(v[1]) << 16, (uint32_t)f32_bf16(v[2]) | (uint32_t)f32_bf16(v[3]) << 16);
+                    pack_bf16(make_float4(v[0], v[1], v[2], v[3]));
             }
         }
 }
@@ -3467,7 +3496,7 @@ __global__ void __launch_bounds__(64) k_pf_attend(const float *qb, int P, int n_
 // bytes or products: 9 heads of 64, 479 tokens: 11.1 us a layer, against 55.7 for k_pf_attend (one wavefront
 // per token and head, a lane per position: every token reads every K and V row again); 63 tokens: 5.0 (7.0).
 constexpr int PFA_W = 4, PFA_T = 16, PFA_C = 32, PFA_VROW = 40;
-template <int HD>
+template <int DT, int HD>
 __global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qb, int P, int n_heads, int n_kv, int ctx, int layer, float scale,
                                                         const uint16_t *kc, const uint16_t *vc, float *att, l3m_pfact act) {
     constexpr int KS = (HD + 31) / 32, NT16 = HD / 16, D8 = HD / 8, UNITS = (HD + 63) / 64, OROW = HD + 4;
@@ -3607,8 +3636,8 @@ __global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qb, int P, 
             y.x += x.x * f; y.y += x.y * f; y.z += x.z * f; y.w += x.w * f;
         }
         y = make_float4(y.x / den, y.y / den, y.z / den, y.w / den);
-        if constexpr (HD % 32 == 0) {                 // whole blocks of the head: prepared here, 8 lanes a block
-            pf_put4(act, t, (n_heads * HD) >> 5, h * HD + 4 * d4, y, t < P);
+        if constexpr (HD % 32 == 0 || DT == L3M_BF16) {   // whole blocks of the head: prepared here, 8 lanes a block
+            pf_put4<DT>(act, t, (n_heads * HD) >> 5, h * HD + 4 * d4, y, t < P);
         } else if (t < P) {
             *(float4 *)(att + (size_t)t * n_heads * HD + h * HD + 4 * d4) = y;
         }
@@ -3922,30 +3951,31 @@ template <int DT, int HDT, bool G2> int decode_fits(int hd, int grid, unsigned l
 }
 
 // k_pf_rows for rows of k <= 4096 values.
-template <bool NORM> void pf_rows(const float *y, int k, const float *w, float eps, const l3m_pfact &act, int P, hipStream_t st) {
+template <int DT, bool NORM> void pf_rows(const float *y, int k, const float *w, float eps, const l3m_pfact &act, int P, hipStream_t st) {
     const dim3 grid((P + 3) / 4), block(256);
-    if (k <= 512) hipLaunchKernelGGL((k_pf_rows<NORM, 2>), grid, block, 0, st, y, k, w, eps, act, P);
-    else if (k <= 1024) hipLaunchKernelGGL((k_pf_rows<NORM, 4>), grid, block, 0, st, y, k, w, eps, act, P);
-    else hipLaunchKernelGGL((k_pf_rows<NORM, 16>), grid, block, 0, st, y, k, w, eps, act, P);
+    if (k <= 512) hipLaunchKernelGGL((k_pf_rows<DT, NORM, 2>), grid, block, 0, st, y, k, w, eps, act, P);
+    else if (k <= 1024) hipLaunchKernelGGL((k_pf_rows<DT, NORM, 4>), grid, block, 0, st, y, k, w, eps, act, P);
+    else hipLaunchKernelGGL((k_pf_rows<DT, NORM, 16>), grid, block, 0, st, y, k, w, eps, act, P);
 }
 
 // The prompt's attention in layer l: on the matrix cores for head dims of 16, 32, ... 128 (k_pf_attn), else
 // k_pf_attend; its output prepared into B->act.
-void pf_attention(const l3m_dmodel *M, const l3m_pfbuf *B, int P, int l, hipStream_t st) {
+template <int DT> void pf_attention(const l3m_dmodel *M, const l3m_pfbuf *B, int P, int l, hipStream_t st) {
     const float *q = B->q;
     const uint16_t *kc = M->kc, *vc = M->vc;
     const int hd = M->hd, nq = M->n_heads * hd;
     const dim3 grid((P + PFA_T - 1) / PFA_T, M->n_heads), block(64 * PFA_W);
+    bool rows = DT != L3M_BF16 && hd % 32;            // blocks across heads
 #define PF_ATTN(HD) \
-    case HD: hipLaunchKernelGGL(k_pf_attn<HD>, grid, block, 0, st, q, P, M->n_heads, M->n_kv, M->ctx, l, M->att_scale, kc, vc, B->att, B->act); break;
+    case HD: hipLaunchKernelGGL((k_pf_attn<DT, HD>), grid, block, 0, st, q, P, M->n_heads, M->n_kv, M->ctx, l, M->att_scale, kc, vc, B->att, B->act); break;
     switch (hd) {
         PF_ATTN(16) PF_ATTN(32) PF_ATTN(48) PF_ATTN(64) PF_ATTN(80) PF_ATTN(96) PF_ATTN(112) PF_ATTN(128)
     default:
         hipLaunchKernelGGL(k_pf_attend, dim3(P, M->n_heads), dim3(64), 0, st, q, P, M->n_heads, M->n_kv, hd, M->ctx, l, M->att_scale, kc, vc, B->att);
+        rows = true;
     }
 #undef PF_ATTN
-    if (hd % 32 || hd > 128)                          // blocks across heads, or the form that prepares nothing
-        pf_rows<false>(B->att, nq, nullptr, 0.f, B->act, P, st);
+    if (rows) pf_rows<DT, false>(B->att, nq, nullptr, 0.f, B->act, P, st);
 }
 
 // One matrix of the prompt. Three splits, by how many 32-row x 32-token tiles there are (for EPI 2 16 gate and 16
@@ -3954,13 +3984,36 @@ void pf_attention(const l3m_dmodel *M, const l3m_pfbuf *B, int P, int l, hipStre
 // us to the first logits, each split for every matrix): 64 tokens 2065 / 1685 / 1509, 200 tokens 2282 / 1918 /
 // 1941, 480 tokens 2549 / 2394 / 2846; gate and up alone at 480 tokens 12.0 / 15.1 / 25.9 us, at 64 - / 7.6 / 7.0.
 constexpr int PF_WIDE = 1024;
-template <int EPI> void pf_gemm(const PfGemm &G, hipStream_t st) {
+template <int DT, int EPI> void pf_gemm(const PfGemm &G, hipStream_t st) {
     constexpr int WR = EPI == 2 ? 2 : 1, MID = EPI == 2 ? 256 : 160;
     const int rows = EPI == 2 ? G.W.tiles * 8 : G.W.rows;   // EPI 2: the ffn rows
     const int r32 = (rows + 31) / 32, t32 = (G.P + 31) / 32, R = pf_ranges(G.W.nb), n = WR * r32 * t32;
-    if (n >= PF_WIDE) hipLaunchKernelGGL((k_pf_gemm<EPI, 2, 2, 2, 1>), dim3(EPI == 2 ? r32 : (r32 + 1) / 2, t32), dim3(128), 0, st, G);
-    else if (n >= MID) hipLaunchKernelGGL((k_pf_gemm<EPI, 2, 2, WR, 4>), dim3(r32, t32), dim3(64 * WR * min(R, 4)), 0, st, G);
-    else hipLaunchKernelGGL((k_pf_gemm<EPI, 2, 1, WR, 8>), dim3(r32, (G.P + 15) / 16), dim3(64 * WR * min(R, 8)), 0, st, G);
+    if (n >= PF_WIDE) hipLaunchKernelGGL((k_pf_gemm<DT, EPI, 2, 2, 2, 1>), dim3(EPI == 2 ? r32 : (r32 + 1) / 2, t32), dim3(128), 0, st, G);
+    else if (n >= MID) hipLaunchKernelGGL((k_pf_gemm<DT, EPI, 2, 2, WR, 4>), dim3(r32, t32), dim3(64 * WR * min(R, 4)), 0, st, G);
+    else hipLaunchKernelGGL((k_pf_gemm<DT, EPI, 2, 1, WR, 8>), dim3(r32, (G.P + 15) / 16), dim3(64 * WR * min(R, 8)), 0, st, G);
+}
+
+template <int DT> void pf_layers(const l3m_dmodel *M, const l3m_pflayer *L, const l3m_pfbuf *B, int P, hipStream_t st) {
+    const int dim = M->dim, hd = M->hd, nq = M->n_heads * hd;
+    for (int l = 0; l < M->n_layers; l++) {
+        const l3m_pflayer &W = L[l];
+        PfGemm G{};
+        G.P = P;
+        pf_rows<DT, true>(B->x, dim, W.attn_norm, M->eps, B->act, P, st);
+        // q (after RoPE) into B->q, k and v into the cache
+        G.W = W.qkv; G.x = B->act; G.y = B->q; G.ystride = nq;
+        G.rope = M->rope; G.kc = M->kc; G.vc = M->vc; G.layer = l; G.ctx = M->ctx; G.nq = nq; G.nk = M->n_kv * hd; G.hd = hd; G.n_kv = M->n_kv;
+        pf_gemm<DT, 1>(G, st);
+        if (l == M->n_layers - 1) break;              // the last layer's K/V rows are all its prompt positions leave
+        pf_attention<DT>(M, B, P, l, st);
+        G.W = W.wo; G.y = B->x; G.ystride = dim;
+        pf_gemm<DT, 0>(G, st);
+        pf_rows<DT, true>(B->x, dim, W.ffn_norm, M->eps, B->act, P, st);
+        G.W = W.gu; G.out = B->hact;
+        pf_gemm<DT, 2>(G, st);
+        G.W = W.down; G.x = B->hact;
+        pf_gemm<DT, 0>(G, st);
+    }
 }
 
 template <int DT> int launch_step_mv(int form, const l3m_dmat &m, const float *x, int k, float *y, int tpw, hipStream_t st) {
@@ -4343,27 +4396,9 @@ int l3m_prefill(const l3m_dmodel *M, const l3m_pflayer *L, const l3m_pfbuf *B, i
     if (P < 1) return 0;
     if (P > M->ctx || !l3m_prefill_fits(M->dim, M->ffn, M->n_heads * M->hd, M->hd)) return fail_msg("prefill: shape out of range");
     hipStream_t st = as_stream(stream);
-    const int dim = M->dim, hd = M->hd, nq = M->n_heads * hd;
-    hipLaunchKernelGGL(k_pf_embed, dim3(P), dim3(NTE), 0, st, M->embed, (const int32_t *)M->tokens, dim, B->x);
-    for (int l = 0; l < M->n_layers; l++) {
-        const l3m_pflayer &W = L[l];
-        PfGemm G{};
-        G.P = P;
-        pf_rows<true>(B->x, dim, W.attn_norm, M->eps, B->act, P, st);
-        // q (after RoPE) into B->q, k and v into the cache
-        G.W = W.qkv; G.x = B->act; G.y = B->q; G.ystride = nq;
-        G.rope = M->rope; G.kc = M->kc; G.vc = M->vc; G.layer = l; G.ctx = M->ctx; G.nq = nq; G.nk = M->n_kv * hd; G.hd = hd; G.n_kv = M->n_kv;
-        pf_gemm<1>(G, st);
-        if (l == M->n_layers - 1) break;              // the last layer's K/V rows are all its prompt positions leave
-        pf_attention(M, B, P, l, st);
-        G.W = W.wo; G.y = B->x; G.ystride = dim;
-        pf_gemm<0>(G, st);
-        pf_rows<true>(B->x, dim, W.ffn_norm, M->eps, B->act, P, st);
-        G.W = W.gu; G.out = B->hact;
-        pf_gemm<2>(G, st);
-        G.W = W.down; G.x = B->hact;
-        pf_gemm<0>(G, st);
-    }
+    hipLaunchKernelGGL(k_pf_embed, dim3(P), dim3(NTE), 0, st, M->embed, (const int32_t *)M->tokens, M->dim, B->x);
+    if (L->qkv.dtype == L3M_BF16) pf_layers<L3M_BF16>(M, L, B, P, st);
+    else pf_layers<L3M_Q8_0>(M, L, B, P, st);
     CKL("prefill");
     return 0;
 }

@@ -187,14 +187,15 @@ def test_prefill_graph_cache_replaces_the_oldest(models, monkeypatch):
 
 @pytest.mark.parametrize("n_prompt", [8, 17, 34, 130])
 @pytest.mark.parametrize("hd", [16, 24, 80, 96, 112, 128])
-def test_prefill_attention_head_dims(models, oracle, hd, n_prompt):
+@pytest.mark.parametrize("dtype", ["q8_0", "bf16"])
+def test_prefill_attention_head_dims(models, oracle, dtype, hd, n_prompt):
     """The prompt's attention at head dims off the other tests': multiples of 16 up to 128 on the matrix cores
     (16-token tiles, 32-position chunks dealt to four wavefronts: 7, 16, 33 and 129 positions), 24 in the form
     with a wavefront per token and head; grouped KV heads. Logits and the second layer's K/V rows (which the
     first layer's attention enters) meet the bars of test_prefill_logits against the oracle."""
     heads = 4
-    cfg = A.Config(f"pf_attn{hd}", dim=heads * hd, n_layers=2, n_heads=heads, n_kv_heads=2, ffn_dim=256, vocab=512, ctx=160, dtype="q8_0")
-    path = models.get(cfg, cfg.dtype, seed=11, std=0.05, norm_jitter=0.1)
+    cfg = A.Config(f"pf_attn{hd}", dim=heads * hd, n_layers=2, n_heads=heads, n_kv_heads=2, ffn_dim=256, vocab=512, ctx=160, dtype=dtype)
+    path = models.get(cfg, dtype, seed=11, std=0.05, norm_jitter=0.1)
     ids = A.prompt(12, cfg.vocab, n_prompt)
     om = oracle.load(path, ctx=160)
     om.generate(ids, 0)
@@ -213,13 +214,14 @@ WIDE = A.Config("pf_wide", dim=1056, n_layers=2, n_heads=11, n_kv_heads=11, ffn_
 
 
 @pytest.mark.parametrize("n_prompt", [34, 162, 500, 1000])
-def test_prefill_gemm_splits(models, monkeypatch, n_prompt):
+@pytest.mark.parametrize("dtype", ["q8_0", "bf16"])
+def test_prefill_gemm_splits(models, monkeypatch, dtype, n_prompt):
     """The GEMM's three splits: 32 x 16 tiles over up to 8 wavefronts (Wo and Wdown at 33 positions), 32 x 32 tiles
     over 4 (q/k/v and gate/up at 33, all at 161, Wo and Wdown at 499), a wavefront a tile (q/k/v and gate/up at
     499, all at 999), with ragged last token tiles. Against the GPU's token-by-token path: the logits' bar of
     test_prefill_logits, the K/V rows within 2% of the largest, the first layer's (one matrix, before activation
     rounding can cascade) within 0.5%."""
-    path = models.get(WIDE, "q8_0", seed=13, std=0.03, norm_jitter=0.1)
+    path = models.get(WIDE, dtype, seed=13, std=0.03, norm_jitter=0.1)
     ids = A.prompt(14, WIDE.vocab, n_prompt)
     out = []
     for prefill in ("1", "0"):
@@ -235,3 +237,30 @@ def test_prefill_gemm_splits(models, monkeypatch, n_prompt):
             for g, w in zip(got, want):
                 g, w = bf16(g), bf16(w)
                 assert np.abs(g - w).max() <= bar * np.abs(w).max(), (layer, np.abs(g - w).max() / np.abs(w).max())
+
+
+@pytest.mark.parametrize("n_prompt", [8, 9, 17, 65, 100])
+@pytest.mark.parametrize("cfg", [GQA, HD48], ids=["gqa", "hd48"])
+def test_prefill_bf16(models, oracle, monkeypatch, cfg, n_prompt):
+    """A bf16 body's prompt in one batched pass (bf16 products on the matrix cores): the logits' bar of
+    test_prefill_logits against the oracle and the token-by-token path, both layers' K/V rows within 1% of the
+    oracle's largest (an activation rounded to bf16, 2^-9 of its value, the other way after a sum in another
+    order)."""
+    path = models.get(cfg, "bf16", seed=9, std=0.05, norm_jitter=0.1)
+    ids, hd, P = A.prompt(9, cfg.vocab, n_prompt), cfg.dim // cfg.n_heads, n_prompt - 1
+    om = oracle.load(path)
+    om.generate(ids, 0)
+    with A.Model(path) as m:
+        m.generate(ids, 0)
+        assert m.prefilled == P
+        lf, kv = m.logits, [m.kv_rows(layer, kvh, 0, P) for layer in range(cfg.n_layers) for kvh in range(cfg.n_kv_heads)]
+    monkeypatch.setenv("L3M_PREFILL", "0")
+    with A.Model(path) as m:
+        m.generate(ids, 0)
+        assert m.prefilled == 0
+        ls = m.logits
+    assert close(lf, om.logits()) and close(lf, ls)
+    want = [om.kv_rows(layer, kvh, 0, P, hd) for layer in range(cfg.n_layers) for kvh in range(cfg.n_kv_heads)]
+    for g, w in zip(kv, want):
+        for a, b in zip(g, w):
+            assert np.abs(bf16(a) - bf16(b)).max() <= 0.01 * np.abs(bf16(b)).max()
