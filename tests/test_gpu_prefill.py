@@ -242,7 +242,7 @@ def test_prefill_gemm_splits(models, monkeypatch, dtype, n_prompt):
 @pytest.mark.parametrize("n_prompt", [8, 9, 17, 65, 100])
 @pytest.mark.parametrize("cfg", [GQA, HD48], ids=["gqa", "hd48"])
 def test_prefill_bf16(models, oracle, monkeypatch, cfg, n_prompt):
-    """A bf16 body's prompt in one batched pass (bf16 products on the matrix cores): the logits' bar of
+    """A bf16 body's prompt in one batched pass (bf16 products on the matrix cores): the logits' bars of
     test_prefill_logits against the oracle and the token-by-token path, both layers' K/V rows within 1% of the
     oracle's largest (an activation rounded to bf16, 2^-9 of its value, the other way after a sum in another
     order)."""
@@ -259,7 +259,10 @@ def test_prefill_bf16(models, oracle, monkeypatch, cfg, n_prompt):
         m.generate(ids, 0)
         assert m.prefilled == 0
         ls = m.logits
-    assert close(lf, om.logits()) and close(lf, ls)
+    # KL and max-abs bars alone: two logits vectors within d of each other can differ in argmax where the top two
+    # lie within 2 d (65 tokens of the hd 48 model: the token-by-token path and the oracle do)
+    for ref in (om.logits(), ls):
+        assert kl(ref, lf) < 0.01 and np.abs(lf - ref).max() <= 0.02 * np.abs(ref).max()
     want = [om.kv_rows(layer, kvh, 0, P, hd) for layer in range(cfg.n_layers) for kvh in range(cfg.n_kv_heads)]
     for g, w in zip(kv, want):
         for a, b in zip(g, w):
