@@ -189,14 +189,6 @@ __device__ float wg_sum(float v, float *red) {
     __syncthreads();
     return ((red[0] + red[1]) + red[2]) + red[3];
 }
-__device__ float wg_max(float v, float *red) {
-    for (int o = 32; o; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-    const int w = threadIdx.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[w] = v;
-    __syncthreads();
-    return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-}
 // (value, index) maximum; ties and NaN go to the lower index, as the reference's strict '>' scan
 // (engine.c:294, 300).
 __device__ __forceinline__ void better(float &v, int &i, float v2, int i2) {
@@ -582,57 +574,157 @@ __global__ void __launch_bounds__(NT) k_gemv(l3m_dmat m, const uint8_t *__restri
     }
 }
 
-// One workgroup per query head (ops.c:58-73): scores q.K[t] / sqrt(hd) over t = 0..pos, softmax, sum of
-// p[t] V[t]. K, V rows are `stride` elements apart; head h reads kv head h / hpk at k + kvh * kv_stride.
-// dpos, when set, holds pos (device-resident step position).
+// One query head over positions 0..n-1 (ops.c:58-73): scores q.K[t] / sqrt(hd), softmax, sum of p[t] V[t]. K, V
+// rows are `stride` elements apart.
+//
+// Groups of L lanes (the power of two from hd / 8 on) take a row each, 16 bytes a lane, ATT_U rows a batch with
+// every K and V load of the batch issued before the scores, and keep a running maximum, sum and output of their
+// own; nothing crosses a group before the end. The groups meet by shuffles and LDS, and the workgroups' parts (`per` rows each)
+// in ws: the last workgroup to finish (a device-scope count) adds them in order, so the result does not depend on
+// which one that is. One launch, whatever n. Bound by latency: two loads deep, then the hand-over between the
+// workgroups. 4001 rows of 128 (2 MB): 12.9 us in
+// 63 workgroups, 60.9 in one; 229 in one workgroup of a thread per row (dependent 16-byte and 2-byte loads).
+constexpr int ATT_U = 4, ATT_SPLITS = 64, ATT_PART = 256 + 8;   // rows a group loads at once; workgroups; floats of a part
+constexpr size_t ATT_WS = 256 + (size_t)4 * ATT_SPLITS * ATT_PART;   // the count, then the parts [max, sum, .., hd outputs]
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));             // V rows need no alignment beyond an element's
+template <int L>
 __global__ void __launch_bounds__(NT) k_attend(float *__restrict__ out, const float *__restrict__ q, const uint16_t *__restrict__ kc,
-                                               const uint16_t *__restrict__ vc, int pos, const int *dpos, int hd, int stride,
-                                               int hpk, size_t kv_stride) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    if (dpos) pos = *dpos;
-    const int h = blockIdx.x, n = pos + 1, tid = threadIdx.x;
-    float *qs = (float *)smem, *sc = qs + hd, *part = sc + ((n + 3) & ~3), *scr = part + NT;
-    const uint16_t *kh = kc + (size_t)(h / hpk) * kv_stride, *vh = vc + (size_t)(h / hpk) * kv_stride;
-    for (int i = tid; i < hd; i += NT) qs[i] = q[(size_t)h * hd + i];
-    __syncthreads();
+                                               const uint16_t *__restrict__ vc, int n, int hd, int stride, int per, uint8_t *ws) {
+    constexpr int ROWS = NT / L * ATT_U, W = NT / 64;             // rows of a workgroup's batch; wavefronts
+    __shared__ __align__(16) float o_s[W][ATT_PART];              // [8 + d]: a wavefront's outputs; [0], [1]: its maximum and sum
+    __shared__ __align__(16) float sum_s[NT][4];
+    __shared__ float f_s[ATT_SPLITS];
+    __shared__ unsigned last;
+    const int tid = threadIdx.x, grp = tid / L, d8 = tid % L, d0 = 8 * d8 < hd ? 8 * d8 : 0;
+    const bool dl = 8 * d8 < hd;                                  // lanes past the head hold zeros
     const float scale = 1.0f / sqrtf((float)hd);
-    float mx = -INFINITY;
-    for (int t = tid; t < n; t += NT) {
-        const uint4 *kr = (const uint4 *)(kh + (size_t)t * stride);
-        float dot = 0.f;
-        for (int v = 0; v < hd / 8; v++) {
-            const uint4 kk = kr[v];
-            const float *qq = qs + v * 8;
-            dot = fmaf(qq[0], bf16_f32(kk.x & 0xFFFF), dot); dot = fmaf(qq[1], bf16_f32(kk.x >> 16), dot);
-            dot = fmaf(qq[2], bf16_f32(kk.y & 0xFFFF), dot); dot = fmaf(qq[3], bf16_f32(kk.y >> 16), dot);
-            dot = fmaf(qq[4], bf16_f32(kk.z & 0xFFFF), dot); dot = fmaf(qq[5], bf16_f32(kk.z >> 16), dot);
-            dot = fmaf(qq[6], bf16_f32(kk.w & 0xFFFF), dot); dot = fmaf(qq[7], bf16_f32(kk.w >> 16), dot);
+    float qv[8], o[8], m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; j++) { qv[j] = dl ? q[d0 + j] : 0.f; o[j] = 0.f; }
+    const int t0 = blockIdx.x * per, t1 = min(t0 + per, n);
+    for (int tb = t0; tb < t1; tb += ROWS) {
+        uint4 kk[ATT_U];
+        u32x4 vv[ATT_U];
+#pragma unroll
+        for (int u = 0; u < ATT_U; u++) {
+            const size_t row = (size_t)min(tb + u * (NT / L) + grp, n - 1) * stride + d0;   // rows past the end: not used
+            kk[u] = *(const uint4 *)(kc + row);
+            vv[u] = *(const u32x4_a2 *)(vc + row);
         }
-        const float st = dot * scale;
-        sc[t] = st;
-        mx = fmaxf(mx, st);
+        float s[ATT_U], nm = m;
+#pragma unroll
+        for (int u = 0; u < ATT_U; u++) {
+            float dot = 0.f;
+            const uint32_t w[4] = {kk[u].x, kk[u].y, kk[u].z, kk[u].w};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                dot = fmaf(qv[2 * j], dl ? bf16_f32(w[j] & 0xFFFF) : 0.f, dot);
+                dot = fmaf(qv[2 * j + 1], dl ? bf16_f32(w[j] >> 16) : 0.f, dot);
+            }
+            for (int x = 1; x < L; x <<= 1) dot += __shfl_xor(dot, x);
+            s[u] = tb + u * (NT / L) + grp < t1 ? dot * scale : -INFINITY;
+            nm = fmaxf(nm, s[u]);
+        }
+        const float base = nm == -INFINITY ? 0.f : nm, r = expf(m - base);   // no row yet: every p is 0
+        l *= r;
+#pragma unroll
+        for (int j = 0; j < 8; j++) o[j] *= r;
+#pragma unroll
+        for (int u = 0; u < ATT_U; u++) {
+            const float p = expf(s[u] - base);
+            const bool ok = tb + u * (NT / L) + grp < t1;
+            l += p;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t w = ok ? vv[u][j] : 0u;
+                o[2 * j] = fmaf(p, bf16_f32(w & 0xFFFF), o[2 * j]);
+                o[2 * j + 1] = fmaf(p, bf16_f32(w >> 16), o[2 * j + 1]);
+            }
+        }
+        m = nm;
     }
-    mx = wg_max(mx, scr);
-    float sum = 0.f;
-    for (int t = tid; t < n; t += NT) {
-        const float e = expf(sc[t] - mx);
-        sc[t] = e;
-        sum += e;
+    // a part's factor at the common maximum: one without a row (or with no score above -infinity, sum 0) counts nothing
+    auto meet = [](float mw, float mm) { return mw == -INFINITY ? 0.f : expf(mw - mm); };
+    // the wavefront's groups, pairwise
+#pragma unroll
+    for (int x = L; x < 64; x <<= 1) {
+        const float m2 = __shfl_xor(m, x), l2 = __shfl_xor(l, x), nm = fmaxf(m, m2), f = meet(m, nm), f2 = meet(m2, nm);
+        l = l * f + l2 * f2;
+#pragma unroll
+        for (int j = 0; j < 8; j++) o[j] = o[j] * f + __shfl_xor(o[j], x) * f2;
+        m = nm;
     }
-    sum = wg_sum(sum, scr);
-    for (int t = tid; t < n; t += NT) sc[t] = sc[t] / sum;
+    const int w = tid >> 6;
+    if ((tid & 63) == 0) { o_s[w][0] = m; o_s[w][1] = l; }
+    if ((tid & 63) < L && dl)
+#pragma unroll
+        for (int j = 0; j < 8; j++) o_s[w][8 + d0 + j] = o[j];
     __syncthreads();
-    const int groups = NT / hd, i = tid % hd, g = tid / hd;
-    float acc = 0.f;
-    if (g < groups)
-        for (int t = g; t < n; t += groups) acc = fmaf(sc[t], bf16_f32(vh[(size_t)t * stride + i]), acc);
-    part[tid] = acc;
-    __syncthreads();
+    // the wavefronts in order, one thread a dim
+    float mm = o_s[0][0], sum = 0.f, y = 0.f;
+#pragma unroll
+    for (int g = 1; g < W; g++) mm = fmaxf(mm, o_s[g][0]);
     if (tid < hd) {
-        float o = part[tid];
-        for (int gg = 1; gg < groups; gg++) o += part[gg * hd + tid];
-        out[(size_t)h * hd + tid] = o;
+#pragma unroll
+        for (int g = 0; g < W; g++) {
+            const float f = meet(o_s[g][0], mm);
+            sum += o_s[g][1] * f;
+            y += o_s[g][8 + tid] * f;
+        }
     }
+    if (gridDim.x == 1) {
+        if (tid < hd) out[tid] = y / sum;
+        return;
+    }
+    float *parts = (float *)(ws + 256), *part = parts + (size_t)blockIdx.x * ATT_PART;
+    if (tid < hd) part[8 + tid] = y;
+    if (tid == 0) { part[0] = mm; part[1] = sum; }
+    __threadfence();
+    __syncthreads();
+    if (tid == 0) last = __hip_atomic_fetch_add((unsigned *)ws, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    // thread (g, c): dims 4 c .. of parts g, g + ng, ..., the first 8 of them requested before the factors are known
+    const int S = gridDim.x, h4 = hd >> 2, ng = NT / h4, g = tid / h4, c = tid - g * h4;
+    float4 v[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = *(const float4 *)(parts + (size_t)min(g + i * ng, S - 1) * ATT_PART + 8 + 4 * c);
+    if (tid < 64) {                                               // S <= 64: a lane a part
+        const float pm = parts[(size_t)min(tid, S - 1) * ATT_PART], pl = parts[(size_t)min(tid, S - 1) * ATT_PART + 1];
+        float am = pm;
+        for (int x = 32; x; x >>= 1) am = fmaxf(am, __shfl_xor(am, x));
+        const float f = tid < S ? meet(pm, am) : 0.f;
+        float al = tid < S ? pl * f : 0.f;
+        for (int x = 32; x; x >>= 1) al += __shfl_xor(al, x);
+        f_s[tid] = f;
+        if (tid == 0) o_s[0][1] = al;
+    }
+    __syncthreads();
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (g < ng) {
+        for (int p0 = g; p0 < S; p0 += 8 * ng) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                if (p0 + i * ng < S) {
+                    const float f = f_s[p0 + i * ng];
+                    a.x = fmaf(v[i].x, f, a.x); a.y = fmaf(v[i].y, f, a.y); a.z = fmaf(v[i].z, f, a.z); a.w = fmaf(v[i].w, f, a.w);
+                }
+                v[i] = *(const float4 *)(parts + (size_t)min(p0 + (8 + i) * ng, S - 1) * ATT_PART + 8 + 4 * c);
+            }
+        }
+        *(float4 *)sum_s[tid] = a;
+    }
+    __syncthreads();
+    if (tid < h4) {
+        for (int i = 1; i < ng; i++) {
+            const float4 b = *(const float4 *)sum_s[i * h4 + tid];
+            a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+        }
+        const float den = o_s[0][1];
+        out[4 * tid] = a.x / den; out[4 * tid + 1] = a.y / den; out[4 * tid + 2] = a.z / den; out[4 * tid + 3] = a.w / den;
+    }
+    if (tid == 0) *(unsigned *)ws = 0;                            // for the stream's next call
 }
 
 __global__ void __launch_bounds__(NT) k_rmsnorm(float *y, const float *x, const float *w, int n, float eps) {
@@ -3788,6 +3880,10 @@ hipStream_t g_stream;
 // The device address of `scratch` (below) on each device the library set up, from hipGetSymbolAddress: the
 // array's name in host code is a host-side stand-in, not a device address.
 void *g_scratch_dev[16];
+void *g_attend_ws;                   // the same of attend_ws, from the first call that wants one
+hipStream_t g_attend_stream[16];     // the stream of each workspace, under g_attend_lock
+int g_attend_streams;
+pthread_mutex_t g_attend_lock = PTHREAD_MUTEX_INITIALIZER;
 int g_ready = -1;
 char g_name[128];
 unsigned g_lds_max = 65536;
@@ -4036,6 +4132,12 @@ template <int DT> int launch_step_mv(int form, const l3m_dmat &m, const float *x
 // the process ends; every call on a GPU shares it and it keeps the last call's contents.
 constexpr size_t ATTEND_STATIC_BYTES = 4u << 20;
 static __device__ __align__(256) uint8_t scratch[ATTEND_STATIC_BYTES];
+// k_attend's workspaces, one per stream that uses it (calls on one stream follow one another), each stream's from
+// its first call on. A stream past the last one, a stream under capture (its graph may be replayed on another) and
+// the special handles (one name for several streams) have none: their calls take one workgroup.
+constexpr int ATT_STREAMS = 16;
+static __device__ __align__(256) uint8_t attend_ws[ATT_STREAMS][ATT_WS];
+static_assert(ATT_WS % 256 == 0, "every workspace 256-byte aligned");
 
 // =============================================================================================== C ABI
 
@@ -4201,11 +4303,51 @@ int l3m_k_gemv(const l3m_dmat *m, const void *act, int k, float *y, void *stream
     return 0;
 }
 
+// The workspace of a stream, or NULL when it has none. Before l3m_dev_init the library's stream is the null
+// stream: one stream, never captured.
+static uint8_t *attend_workspace(hipStream_t st) {
+    if ((uintptr_t)st == 1 || (uintptr_t)st == 2) return nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (st && (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)) return nullptr;
+    pthread_mutex_lock(&g_attend_lock);
+    if (!g_attend_ws && hipGetSymbolAddress(&g_attend_ws, HIP_SYMBOL(attend_ws)) != hipSuccess) {
+        (void)hipGetLastError();
+        g_attend_ws = nullptr;
+        pthread_mutex_unlock(&g_attend_lock);
+        return nullptr;
+    }
+    int i = 0;
+    while (i < g_attend_streams && g_attend_stream[i] != st) i++;
+    if (i == g_attend_streams && i < ATT_STREAMS) g_attend_stream[g_attend_streams++] = st;
+    pthread_mutex_unlock(&g_attend_lock);
+    return i < ATT_STREAMS ? (uint8_t *)g_attend_ws + (size_t)i * ATT_WS : nullptr;
+}
+
+// k_attend over n rows. Up to ATT_ALONE batches of rows go to one workgroup: a second costs the hand-over (about
+// 3.5 us), a batch about 0.9 us (hd 128, 256 rows: 6.8 us in one; 512 rows: 8.3 us spread, 10.4 in one). More are spread over up to ATT_SPLITS workgroups.
+constexpr int ATT_ALONE = 4;
+static void launch_attend(float *out, const float *q, const uint16_t *k, const uint16_t *v, int n, int hd, int stride, hipStream_t st) {
+    int L = 1;
+    while (8 * L < hd) L *= 2;
+    const int rows = NT / L * ATT_U, batches = (n + rows - 1) / rows;
+    uint8_t *ws = batches > ATT_ALONE ? attend_workspace(st) : nullptr;
+    const int per = rows * (ws ? (batches + ATT_SPLITS - 1) / ATT_SPLITS : batches), grid = (n + per - 1) / per;
+    switch (L) {
+    case 1: hipLaunchKernelGGL(k_attend<1>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws); break;
+    case 2: hipLaunchKernelGGL(k_attend<2>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws); break;
+    case 4: hipLaunchKernelGGL(k_attend<4>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws); break;
+    case 8: hipLaunchKernelGGL(k_attend<8>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws); break;
+    case 16: hipLaunchKernelGGL(k_attend<16>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws); break;
+    default: hipLaunchKernelGGL(k_attend<32>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws);
+    }
+}
+// The most positions a call takes: 4 (hd + ceil4(pos + 1) + NT + 8) bytes within LDS_MAX.
+static bool attend_fits(int pos, int hd) { return 4 * ((size_t)hd + ((pos + 4) & ~3) + NT + 8) <= LDS_MAX; }
+
 int l3m_k_attend(float *out, const float *q, const uint16_t *k, const uint16_t *v, int pos, int hd, int stride, void *stream) {
     if (pos < 0 || hd < 8 || hd % 8 || hd > NT || stride < hd || stride % 8) return fail_msg("attend: bad shape");
-    const size_t sm = 4 * ((size_t)hd + ((pos + 4) & ~3) + NT + 8);
-    if (sm > LDS_MAX) return fail_msg("attend: pos too large");
-    hipLaunchKernelGGL(k_attend, dim3(1), dim3(NT), sm, as_stream(stream), out, q, k, v, pos, (const int *)nullptr, hd, stride, 1, (size_t)0);
+    if (!attend_fits(pos, hd)) return fail_msg("attend: pos too large");
+    launch_attend(out, q, k, v, pos + 1, hd, stride, as_stream(stream));
     CKL("k_attend");
     return 0;
 }
@@ -4257,8 +4399,7 @@ int l3m_hip_attend_noalloc(float *out, const float *q, const uint16_t *k, const 
                  kv, (ATTEND_STATIC_BYTES - 2 * vec) / 2);
         return fail_msg(msg);
     }
-    const size_t sm = 4 * ((size_t)head_dim + ((pos + 4) & ~3) + NT + 8);
-    if (sm > LDS_MAX) return fail_msg("attend_noalloc: pos too large for the kernel's LDS");
+    if (!attend_fits(pos, head_dim)) return fail_msg("attend_noalloc: pos too large");
     uint8_t *base = (uint8_t *)g_scratch_dev[0];
     float *dq = (float *)base, *dout = (float *)(base + vec);
     uint16_t *dk = (uint16_t *)(base + 2 * vec), *dv = (uint16_t *)(base + 2 * vec + up256(kv));
@@ -4267,7 +4408,7 @@ int l3m_hip_attend_noalloc(float *out, const float *q, const uint16_t *k, const 
     if (e == hipSuccess) e = hipMemcpyAsync(dk, k, kv, hipMemcpyHostToDevice, g_stream);
     if (e == hipSuccess) e = hipMemcpyAsync(dv, v, kv, hipMemcpyHostToDevice, g_stream);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_attend, dim3(1), dim3(NT), sm, g_stream, dout, dq, dk, dv, pos, (const int *)nullptr, head_dim, stride, 1, (size_t)0);
+        launch_attend(dout, dq, dk, dv, pos + 1, head_dim, stride, g_stream);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(out, dout, (size_t)head_dim * 4, hipMemcpyDeviceToHost, g_stream);

@@ -1,0 +1,90 @@
+"""l3m_k_attend (one query head over a K/V cache) where its work is split: lane groups of 1 to 32 lanes a row,
+batches of rows, one workgroup or up to 64 whose parts meet in a workspace of the stream. Against the oracle's
+l3m_attend within 1e-5 absolute (the reference's own bar, tests/test_kernels.c:145)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import l3m_amd as A
+
+pytestmark = pytest.mark.gpu
+
+
+def inputs(seed, n, hd, stride):
+    rng = np.random.default_rng(seed)
+    q = (rng.standard_normal(hd) * 2).astype(np.float32)
+    k, v = (rng.integers(0, 1 << 16, n * stride + 8, dtype=np.uint16) & 0xBF7F for _ in range(2))   # bf16, |v| < 2
+    return q, k.astype(np.uint16), v.astype(np.uint16)
+
+
+@pytest.mark.parametrize("hd", [8, 16, 40, 64, 128, 200, 256])
+@pytest.mark.parametrize("n", [1, 2, 31, 33, 255, 257, 1025, 4001, 8001])
+def test_attend_splits(dev, oracle, hd, n):
+    stride = hd + 8 * (n % 3)
+    q, k, v = inputs(hd * 10007 + n, n, hd, stride)
+    got = dev.attend(q, k, v, n - 1, hd, stride)
+    want = oracle.attend(q, k, v, n - 1, hd, stride)
+    assert np.abs(got - want).max() <= 1e-5, np.abs(got - want).max()
+    again = dev.attend(q, k, v, n - 1, hd, stride)            # whichever workgroup ends last
+    assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+    dev.free_all()
+
+
+def test_attend_unaligned_v_rows(dev, oracle):
+    """V needs no alignment beyond an element's: a V pointer one element past a 16-byte boundary."""
+    n, hd = 700, 64
+    q, k, v = inputs(5, n, hd, hd)
+    dq, dk, dv, do = dev.put(q), dev.put(k), dev.put(v), dev.alloc(hd * 4)
+    assert dev.lib.l3m_k_attend(do, dq, dk, dv + 2, n - 1, hd, hd, None) == 0
+    got = dev.get(do, hd, np.float32)
+    assert np.abs(got - oracle.attend(q, k, v[1:], n - 1, hd, hd)).max() <= 1e-5
+    dev.free_all()
+
+
+def test_attend_large_values_and_masked_rows(dev, oracle):
+    """Scores far past expf's range, and rows past the last one that hold infinities: they are not attended."""
+    n, hd = 1030, 64
+    q, k, v = inputs(6, n + 40, hd, hd)
+    q *= 20
+    k[n * hd:], v[n * hd:] = 0x7F80, 0x7F80
+    got = dev.attend(q, k, v, n - 1, hd, hd)
+    assert np.abs(got - oracle.attend(q, k[:n * hd], v[:n * hd], n - 1, hd, hd)).max() <= 1e-5
+    dev.free_all()
+
+
+def test_attend_many_streams_and_capture(dev, oracle):
+    """18 streams with a call each in flight (16 of them get a workspace), three rounds of other inputs; then a
+    call recorded into a graph, replayed between other calls on the same stream."""
+    hip = C.CDLL("libamdhip64.so")
+    n, hd = 3000, 64
+    streams = []
+    for _ in range(18):
+        st = C.c_void_p()
+        assert hip.hipStreamCreate(C.byref(st)) == 0
+        streams.append(st)
+    for rnd in range(3):
+        sets = [inputs(100 * rnd + i, n, hd, hd) for i in range(18)]
+        bufs = [(dev.put(q), dev.put(k), dev.put(v), dev.alloc(hd * 4)) for q, k, v in sets]
+        for st, (q, k, v, o) in zip(streams, bufs):
+            assert dev.lib.l3m_k_attend(o, q, k, v, n - 1, hd, hd, st) == 0
+        assert hip.hipDeviceSynchronize() == 0
+        for (q, k, v), b in zip(sets, bufs):
+            assert np.abs(dev.get(b[3], hd, np.float32) - oracle.attend(q, k, v, n - 1, hd, hd)).max() <= 1e-5
+    st, (q, k, v, o) = streams[0], bufs[0]
+    graph, ex, want = C.c_void_p(), C.c_void_p(), oracle.attend(*sets[0], n - 1, hd, hd)
+    assert hip.hipStreamBeginCapture(st, 1) == 0
+    assert dev.lib.l3m_k_attend(o, q, k, v, n - 1, hd, hd, st) == 0
+    assert hip.hipStreamEndCapture(st, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+    o2 = dev.alloc(hd * 4)
+    for _ in range(3):
+        assert hip.hipGraphLaunch(ex, st) == 0
+        assert dev.lib.l3m_k_attend(o2, q, k, v, n - 1, hd, hd, st) == 0
+        assert hip.hipStreamSynchronize(st) == 0
+        for p in (o, o2):
+            assert np.abs(dev.get(p, hd, np.float32) - want).max() <= 1e-5
+    assert hip.hipGraphExecDestroy(ex) == 0 and hip.hipGraphDestroy(graph) == 0
+    for st in streams:
+        assert hip.hipStreamDestroy(st) == 0
+    dev.free_all()
