@@ -180,50 +180,14 @@ __device__ float4 lt_elem4(const l3m_dmat &m, int r, int i) {
 
 // ------------------------------------------------------------------------------- workgroup helpers
 
-// Sum over the workgroup in a fixed order; every thread gets the result. red: 4 floats of LDS.
-__device__ float wg_sum(float v, float *red) {
-    for (int o = 32; o; o >>= 1) v += __shfl_xor(v, o);
-    const int w = threadIdx.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[w] = v;
-    __syncthreads();
-    return ((red[0] + red[1]) + red[2]) + red[3];
-}
+template <int N> __device__ __forceinline__ float lanes_sum(float v);   // cross-lane sums, below
+template <int N> __device__ __forceinline__ float lanes_max(float v);
+template <int N> __device__ __forceinline__ int lanes_sumi(int v);
+
 // (value, index) maximum; ties and NaN go to the lower index, as the reference's strict '>' scan
 // (engine.c:294, 300).
 __device__ __forceinline__ void better(float &v, int &i, float v2, int i2) {
     if (v2 > v || (v2 == v && i2 < i) || (v != v && v2 == v2)) { v = v2; i = i2; }
-}
-__device__ void wg_argmax(float &v, int &i, float *sv, int *si) {
-    for (int o = 32; o; o >>= 1) {
-        const float v2 = __shfl_xor(v, o);
-        const int i2 = __shfl_xor(i, o);
-        better(v, i, v2, i2);
-    }
-    const int w = threadIdx.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) { sv[w] = v; si[w] = i; }
-    __syncthreads();
-    v = sv[0]; i = si[0];
-    for (int k = 1; k < 4; k++) better(v, i, sv[k], si[k]);
-}
-
-// x (k values, zero up to kp) into LDS xs, optionally RMS-normalized with weights nw (ops.c:13-18:
-// s = 1/sqrt(sum x^2 / n + eps), y = x * s * w). src(i) yields x_i.
-template <class Src>
-__device__ void stage_x(float *xs, Src src, int k, int kp, const float *nw, float eps, float *red) {
-    float ss = 0.f;
-    for (int i = threadIdx.x; i < kp; i += NT) {
-        const float v = i < k ? src(i) : 0.f;
-        xs[i] = v;
-        ss = fmaf(v, v, ss);
-    }
-    if (nw) {
-        const float tot = wg_sum(ss, red);
-        const float s = 1.0f / sqrtf(tot / (float)k + eps);
-        for (int i = threadIdx.x; i < k; i += NT) xs[i] = xs[i] * s * nw[i];
-    }
-    __syncthreads();
 }
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
@@ -275,41 +239,6 @@ __device__ __forceinline__ int put_block(uint8_t *blk, int m, uint32_t P, uint32
         ((uint32_t *)blk)[m] = P;
         return q0 + q1 + q2 + q3;
     }
-}
-
-// Activation prep (pack.c:101-123): quantized -> per 32-block amax, inv = 127/amax, q = rint(x*inv),
-// scale = amax/127, sum = sum(q); bf16 -> nearest even; f32 -> as is. 8 lanes per block; the quantized
-// values are stored in the form the dtype's matvec reads (act_size).
-template <int DT>
-__device__ void prep_act(uint8_t *act, const float *xs, int kp) {
-    if constexpr (quantized(DT)) {
-        const int nb = kp / 32, g = threadIdx.x >> 3, l = threadIdx.x & 7;
-        float *scale = (float *)(act + act_qbytes(DT) * nb);
-        int *sum = (int *)(act + act_qbytes(DT) * nb + 4 * nb);
-        for (int b = g; b < nb; b += NT / 8) {
-            const float4 v = *(const float4 *)(xs + b * 32 + 4 * l);
-            float am = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-            am = fmaxf(am, __shfl_xor(am, 1));
-            am = fmaxf(am, __shfl_xor(am, 2));
-            am = fmaxf(am, __shfl_xor(am, 4));
-            const float inv = am > 0.f ? 127.0f / am : 0.f;
-            const int q0 = (int)rintf(v.x * inv), q1 = (int)rintf(v.y * inv), q2 = (int)rintf(v.z * inv), q3 = (int)rintf(v.w * inv);
-            const uint32_t P = (uint32_t)(q0 & 255) | (uint32_t)(q1 & 255) << 8 | (uint32_t)(q2 & 255) << 16 | (uint32_t)(q3 & 255) << 24;
-            const uint32_t Pp = (uint32_t)__shfl_xor((int)P, 4);
-            int s = put_block<DT>(act + b * act_qbytes(DT), l, P, Pp, q0, q1, q2, q3);
-            s += __shfl_xor(s, 1);
-            s += __shfl_xor(s, 2);
-            s += __shfl_xor(s, 4);
-            if (l == 0) { scale[b] = am / 127.0f; sum[b] = s; }
-        }
-    } else if constexpr (DT == L3M_BF16) {
-        uint16_t *o = (uint16_t *)act;
-        for (int i = threadIdx.x; i < kp; i += NT) o[i] = f32_bf16(xs[i]);
-    } else {
-        float *o = (float *)act;
-        for (int i = threadIdx.x; i < kp; i += NT) o[i] = xs[i];
-    }
-    __syncthreads();
 }
 
 // ------------------------------------------------------------------------------------- matvec core
@@ -506,23 +435,71 @@ __global__ void __launch_bounds__(NT) k_read(const u32x4 *__restrict__ buf, size
     if (x == 0x9E3779B9u) gw(sink)[0] = x;            // practically never: keeps the loads
 }
 
+// Vectors at addresses aligned to their elements alone (callers' pointers) or not at all (a prepared activation):
+// the hardware takes global accesses of any alignment.
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+typedef u32x4 u32x4_a1 __attribute__((aligned(1)));
+typedef u32x2 u32x2_a1 __attribute__((aligned(1)));
+typedef uint32_t u32_a1 __attribute__((aligned(1)));
+// Elements i .. i + 3 of x, zeros from k on.
+__device__ __forceinline__ float4 load4(const float *__restrict__ x, int i, int k) {
+    if (i + 3 < k) {
+        const f32x4 v = *(const f32x4_a4 *)(x + i);
+        return make_float4(v.x, v.y, v.z, v.w);
+    }
+    return make_float4(i < k ? x[i] : 0.f, i + 1 < k ? x[i + 1] : 0.f, i + 2 < k ? x[i + 2] : 0.f, 0.f);
+}
+
+// The standalone activation prep (pack.c:101-123: per 32-block amax, inv = 127 / amax, q = rint(x * inv), scale =
+// amax / 127, sum = sum(q), stored in the form the dtype's matvec reads (act_size); bf16 nearest even): a thread 4 values, 8 threads a block, one
+// load each and straight to memory, over as many workgroups as the vector fills. Bound by one kernel's latency:
+// q4_0 4096 values 2.1 us; 7.0 in one workgroup through LDS, copied out byte by byte.
 template <int DT>
 __global__ void __launch_bounds__(NT) k_prep(const float *__restrict__ x, int k, uint8_t *__restrict__ out) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    Smem s = carve(smem, DT, k);
-    const int kp = kpad(k);
-    stage_x(s.xs, [&](int i) { return x[i]; }, k, kp, nullptr, 0.f, s.scr);
-    prep_act<DT>(s.act, s.xs, kp);
-    const size_t n = act_size(DT, k);
-    for (size_t i = threadIdx.x; i < n; i += NT) out[i] = s.act[i];
-    if constexpr (DT == L3M_MXFP4) {
-        for (int w = threadIdx.x; w < kp / 8; w += NT) {            // one 16-byte word of f16 pairs: 8 values
-            u32x2 h, l;
-            split_hl(((const uint4 *)s.act)[w], h, l);
-            uint8_t *o = out + n + 64 * (w >> 2) + 8 * (w & 3);
-            *(u32x2 *)o = h;
-            *(u32x2 *)(o + 32) = l;
+    const int kp = kpad(k), i = 4 * (blockIdx.x * NT + threadIdx.x);
+    const float4 v = load4(x, i, k);
+    if constexpr (quantized(DT)) {
+        const int nb = kp / 32, b = i >> 5, m = threadIdx.x & 7;
+        const float am = lanes_max<8>(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+        const float inv = am > 0.f ? 127.0f / am : 0.f;
+        const int q0 = (int)rintf(v.x * inv), q1 = (int)rintf(v.y * inv), q2 = (int)rintf(v.z * inv), q3 = (int)rintf(v.w * inv);
+        const uint32_t P = (uint32_t)(q0 & 255) | (uint32_t)(q1 & 255) << 8 | (uint32_t)(q2 & 255) << 16 | (uint32_t)(q3 & 255) << 24;
+        const uint32_t Pp = (uint32_t)__shfl_xor((int)P, 4);
+        const int s = lanes_sumi<8>(DT == L3M_Q4_0 ? (q0 & 15) + (q1 & 15) + (q2 & 15) + (q3 & 15) : q0 + q1 + q2 + q3);
+        if (i >= kp) return;                          // whole blocks of lanes
+        uint8_t *blk = out + (size_t)b * act_qbytes(DT);
+        if constexpr (DT == L3M_Q8_0) ((u32_a1 *)blk)[m] = P;
+        if constexpr (DT == L3M_Q4_0) {
+            if (m < 4) {                              // put_block's nibble planes
+                ((u32_a1 *)blk)[m] = ((P >> 4) & 0x0F0F0F0Fu) | (Pp & 0xF0F0F0F0u);
+                ((u32_a1 *)blk)[4 + m] = (P & 0x0F0F0F0Fu) | ((Pp & 0x0F0F0F0Fu) << 4);
+            }
         }
+        if constexpr (DT == L3M_MXFP4) {
+            if (m < 4) {                              // a 16-byte word of f16 pairs, and its fp8 parts
+                uint32_t d[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const _Float16 lo = (_Float16)(float)(int8_t)(P >> (8 * j)), hi = (_Float16)(float)(int8_t)(Pp >> (8 * j));
+                    d[j] = (uint32_t)__builtin_bit_cast(uint16_t, lo) | (uint32_t)__builtin_bit_cast(uint16_t, hi) << 16;
+                }
+                u32x2 h, l;
+                split_hl(make_uint4(d[0], d[1], d[2], d[3]), h, l);
+                *(u32x4_a1 *)(blk + 16 * m) = u32x4{d[0], d[1], d[2], d[3]};
+                uint8_t *o = out + act_size(DT, k) + 64 * (size_t)b + 8 * m;
+                *(u32x2_a1 *)o = h;
+                *(u32x2_a1 *)(o + 32) = l;
+            }
+        }
+        if (m == 0) {
+            *(u32_a1 *)(out + (size_t)act_qbytes(DT) * nb + 4 * (size_t)b) = __float_as_uint(am / 127.0f);
+            *(u32_a1 *)(out + (size_t)(act_qbytes(DT) + 4) * nb + 4 * (size_t)b) = (uint32_t)s;
+        }
+    } else if (i < kp) {
+        if constexpr (DT == L3M_BF16)
+            *(u32x2_a1 *)(out + 2 * (size_t)i) = u32x2{(uint32_t)f32_bf16(v.x) | (uint32_t)f32_bf16(v.y) << 16, (uint32_t)f32_bf16(v.z) | (uint32_t)f32_bf16(v.w) << 16};
+        else
+            *(u32x4_a1 *)(out + 4 * (size_t)i) = u32x4{__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)};
     }
 }
 
@@ -727,11 +704,37 @@ __global__ void __launch_bounds__(NT) k_attend(float *__restrict__ out, const fl
     if (tid == 0) *(unsigned *)ws = 0;                            // for the stream's next call
 }
 
-__global__ void __launch_bounds__(NT) k_rmsnorm(float *y, const float *x, const float *w, int n, float eps) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    float *xs = (float *)smem, *scr = xs + kpad(n);
-    stage_x(xs, [&](int i) { return x[i]; }, n, kpad(n), w, eps, scr);
-    for (int i = threadIdx.x; i < n; i += NT) y[i] = xs[i];
+// y = x * s * w with s = 1 / sqrt(sum x^2 / n + eps) (ops.c:13-18), one workgroup of a thread per 4 values (C of them
+// each when n is past 4096), every load first. y may be x. 768 values 1.6 us; 4.1 with 256 threads staging x in
+// LDS.
+template <int C>
+__global__ void __launch_bounds__(1024) k_rmsnorm(float *y, const float *x, const float *w, int n, float eps) {
+    __shared__ float red[16];
+    const int t = threadIdx.x, nt = blockDim.x, wave = t >> 6;
+    float4 v[C], g[C];
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        v[c] = load4(x, 4 * (t + c * nt), n);
+        g[c] = load4(w, 4 * (t + c * nt), n);
+    }
+#pragma unroll
+    for (int c = 0; c < C; c++) ss += fmaf(v[c].x, v[c].x, v[c].y * v[c].y) + fmaf(v[c].z, v[c].z, v[c].w * v[c].w);
+    ss = lanes_sum<64>(ss);
+    if ((t & 63) == 0) red[wave] = ss;
+    __syncthreads();
+    float tot = 0.f;
+    for (int i = 0; i < nt >> 6; i++) tot += red[i];
+    const float s = 1.0f / sqrtf(tot / (float)n + eps);
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int i = 4 * (t + c * nt);
+        const f32x4 o = {v[c].x * s * g[c].x, v[c].y * s * g[c].y, v[c].z * s * g[c].z, v[c].w * s * g[c].w};
+        if (i + 3 < n) *(f32x4_a4 *)(y + i) = o;
+        else
+            for (int j = 0; j < 3; j++)
+                if (i + j < n) y[i + j] = o[j];
+    }
 }
 
 // Pairs (2i, 2i+1) of each head rotate by the table angle i (ops.c:29-40).
@@ -755,14 +758,57 @@ __global__ void __launch_bounds__(NT) k_silu_mul(float *h, const float *g, int n
     if (i < n) h[i] = silu_mul(h[i], g[i]);
 }
 
-__global__ void __launch_bounds__(NT) k_argmax(const float *x, int n, int32_t *out) {
-    __shared__ float sv[4];
-    __shared__ int si[4];
+// The first maximum of x (engine.c:290-301): one workgroup, a thread ARG_U x 4 values a round with every load first
+// (16 bytes from the first aligned address on). 49152 values: 6.0 us, 62.5
+// with 256 threads of dependent 4-byte loads.
+constexpr int ARG_U = 12;
+__global__ void __launch_bounds__(1024) k_argmax(const float *x, int n, int32_t *out) {
+    __shared__ float sv[16];
+    __shared__ int si[16];
+    const int t = threadIdx.x, head = min((int)((16 - ((uintptr_t)x & 15)) & 15) >> 2, n), nq = (n - head) >> 2, tail = head + 4 * nq;
     float v = -INFINITY;
     int idx = 0x7FFFFFFF;
-    for (int i = threadIdx.x; i < n; i += NT) better(v, idx, x[i], i);
-    wg_argmax(v, idx, sv, si);
-    if (threadIdx.x == 0) *out = idx == 0x7FFFFFFF ? 0 : idx;
+    // a value wins over an equal one by its lower index (and over the start, which no value is below); NaN never wins
+    auto take = [&](float a, int i) {
+        if (a > v || (a == v && i < idx)) { v = a; idx = i; }
+    };
+    if (t < head) take(x[t], t);
+    // the thread's first quad with the largest value, then that value's place in it
+    const float4 *xq = (const float4 *)(x + head);
+    float vq = -INFINITY;
+    int best = -1;
+    for (int q0 = 0; q0 < nq; q0 += ARG_U * 1024) {
+        float4 a[ARG_U];
+#pragma unroll
+        for (int u = 0; u < ARG_U; u++) a[u] = xq[min(q0 + u * 1024 + t, nq - 1)];   // past the end: the last again
+#pragma unroll
+        for (int u = 0; u < ARG_U; u++) {
+            const float m = fmaxf(fmaxf(a[u].x, a[u].y), fmaxf(a[u].z, a[u].w));
+            if (m > vq) { vq = m; best = min(q0 + u * 1024 + t, nq - 1); }
+        }
+    }
+    if (best >= 0) {
+        const float4 a = xq[best];
+        take(vq, head + 4 * best + (a.x == vq ? 0 : a.y == vq ? 1 : a.z == vq ? 2 : 3));
+    } else {                                          // nothing above -infinity: the first of those
+        for (int q = t; q < nq; q += 1024) {
+            const float4 a = xq[q];
+            const int i = head + 4 * q;
+            take(a.x, i); take(a.y, i + 1); take(a.z, i + 2); take(a.w, i + 3);
+        }
+    }
+    if (t < n - tail) take(x[tail + t], tail + t);
+    for (int o = 32; o; o >>= 1) {
+        const float v2 = __shfl_xor(v, o);
+        const int i2 = __shfl_xor(idx, o);
+        take(v2, i2);
+    }
+    if ((t & 63) == 0) { sv[t >> 6] = v; si[t >> 6] = idx; }
+    __syncthreads();
+    if (t == 0) {
+        for (int k = 1; k < 16; k++) take(sv[k], si[k]);
+        *out = idx == 0x7FFFFFFF ? 0 : idx;
+    }
 }
 
 // ------------------------------------------------------------------------------ decode step kernels
@@ -1085,7 +1131,7 @@ template <int N> __device__ __forceinline__ int lanes_mini(int v) {
     if constexpr (N >= 64) { float lo, hi; swap32(__int_as_float(v), lo, hi); v = min(__float_as_int(lo), __float_as_int(hi)); }
     return v;
 }
-// (value, index) maximum with the reference's tie rule (better(): the larger value, then the lower index;
+// (value, index) maximum with the reference's tie rule (the larger value, then the lower index;
 // a NaN never wins) into every thread: a wavefront's largest value (fmaxf passes NaN over), then the
 // lowest index that holds it; then the same over the wavefronts' results, which every wavefront reads
 // after one barrier. sv, si: NWE words each, not read again before a later barrier.
@@ -3919,7 +3965,7 @@ hipStream_t as_stream(void *s) { return s ? (hipStream_t)s : g_stream; }
     default: return fail_msg("bad dtype"); }
 
 template <int DT> void launch_prep(const float *x, int k, void *act, hipStream_t st) {
-    hipLaunchKernelGGL(k_prep<DT>, dim3(1), dim3(NT), smem_bytes(DT, k), st, x, k, (uint8_t *)act);
+    hipLaunchKernelGGL(k_prep<DT>, dim3((kpad(k) / 4 + NT - 1) / NT), dim3(NT), 0, st, x, k, (uint8_t *)act);
 }
 // Nibble-block matrices (q4_0, mxfp4) of at least 128 tiles whose rows are 64, 128 or 256 blocks take
 // k_gemv_deep: 8 wavefronts per tile, nb / 32 blocks per lane (measured at 14336 x 4096, warm / cold against
@@ -4354,7 +4400,9 @@ int l3m_k_attend(float *out, const float *q, const uint16_t *k, const uint16_t *
 
 int l3m_k_rmsnorm(float *y, const float *x, const float *w, int n, float eps, void *stream) {
     if (n < 1 || 4 * ((size_t)kpad(n) + 8) > LDS_MAX) return fail_msg("rmsnorm: n out of range");
-    hipLaunchKernelGGL(k_rmsnorm, dim3(1), dim3(NT), 4 * ((size_t)kpad(n) + 8), as_stream(stream), y, x, w, n, eps);
+    const int quads = (n + 3) / 4;                    // at most 4088: LDS_MAX bounds n
+    if (quads <= 1024) hipLaunchKernelGGL(k_rmsnorm<1>, dim3(1), dim3((quads + 63) & ~63), 0, as_stream(stream), y, x, w, n, eps);
+    else hipLaunchKernelGGL(k_rmsnorm<4>, dim3(1), dim3(1024), 0, as_stream(stream), y, x, w, n, eps);
     CKL("k_rmsnorm");
     return 0;
 }
@@ -4492,7 +4540,7 @@ int l3m_k_attend_decode(int mode, float *out, const float *q, const uint16_t *kc
 }
 
 int l3m_k_argmax(const float *x, int n, int32_t *out, void *stream) {
-    hipLaunchKernelGGL(k_argmax, dim3(1), dim3(NT), 0, as_stream(stream), x, n, out);
+    hipLaunchKernelGGL(k_argmax, dim3(1), dim3(1024), 0, as_stream(stream), x, n, out);
     CKL("k_argmax");
     return 0;
 }
