@@ -109,7 +109,7 @@ void        l3m_dev_clear_error(void);
 const char *l3m_dev_name(void);
 void       *l3m_dev_alloc(size_t bytes);        // zeroed; NULL on failure
 void        l3m_dev_free(void *p);
-int         l3m_dev_upload_async(void *dst, const void *src_pinned, size_t bytes);   // queued, not waited for
+int         l3m_dev_upload_async(void *dst, const void *src, size_t bytes);   // queued, not waited for: src unchanged until the stream has run it
 int         l3m_dev_zero_async(void *dst, size_t bytes);
 void       *l3m_dev_host_alloc(size_t bytes);   // pinned host memory
 void        l3m_dev_host_free(void *p);
@@ -127,6 +127,11 @@ int    l3m_k_rmsnorm(float *y, const float *x, const float *w, int n, float eps,
 int    l3m_k_rope(float *v, int n_heads, int hd, int pos, const float *table, void *stream);
 int    l3m_k_silu_mul(float *h, const float *g, int n, void *stream);
 int    l3m_k_argmax(const float *x, int n, int32_t *out, void *stream);
+
+// The reference's host tiles (kernels.h:1-11; ntiles of 16 rows x k inputs, copied to the device as they are, 64
+// bytes readable past them) as lane-tile planes; quantized k a multiple of 32. l3m_ltile_bytes: their size.
+size_t l3m_ltile_bytes(int dtype, int ntiles, int k);
+int    l3m_k_ltiles(int dtype, int ntiles, int k, const void *tiles, void *quant, void *scale, void *stream);
 
 // ------------------------------------------------------------------ decode step
 // Enqueue one decode step at the device position: per layer the attention block (one workgroup per head

@@ -503,6 +503,52 @@ __global__ void __launch_bounds__(NT) k_prep(const float *__restrict__ x, int k,
     }
 }
 
+// The reference's host tiles (kernels.h:1-11) as lane-tile planes, a thread per row of a block: per tile of 16 rows
+// f32 [k][16]; bf16 [k/2][16][2]; quantized per 32 inputs the 16 scales, then bytes: q8 value + 128 at
+// (i / 4 * 16 + row) * 4 + i % 4, q4 and mxfp4 inputs 8g + j (low nibble) and 8g + 4 + j (high) at
+// (g * 16 + row) * 4 + j. The same bytes l3m_lt_pack_ltiles writes (2048 x 768 q8_0: 4.4 us, about 0.7 ms there).
+template <int DT>
+__global__ void __launch_bounds__(NT) k_ltiles(const uint8_t *__restrict__ src, int ntiles, int k, uint8_t *__restrict__ q, uint8_t *__restrict__ s) {
+    const int nb = kpad(k) / 32, id = blockIdx.x * NT + threadIdx.x, c = id & 15, b = (id >> 4) % nb, t = (id >> 4) / nb;
+    if (t >= ntiles) return;
+    const size_t slot = (size_t)id;                   // (tile * nb + block) * 16 + row
+    if constexpr (quantized(DT)) {
+        constexpr int SB = DT == L3M_MXFP4 ? 16 : 32;
+        const uint8_t *blk = src + ((size_t)t * nb + b) * (SB + 16 * qbytes(DT));
+        const uint32_t *w = (const uint32_t *)(blk + SB) + c;
+        if constexpr (DT == L3M_MXFP4) s[slot] = blk[c];
+        else ((uint16_t *)s)[slot] = ((const uint16_t *)blk)[c];
+        uint4 *o = (uint4 *)(q + slot * qbytes(DT));
+        if constexpr (DT == L3M_Q8_0) {
+            uint32_t d[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) d[i] = w[16 * i] ^ 0x80808080u;
+            o[0] = make_uint4(d[0], d[1], d[2], d[3]);
+            o[1] = make_uint4(d[4], d[5], d[6], d[7]);
+        } else {
+            const uint32_t d0 = w[0], d1 = w[16], d2 = w[32], d3 = w[48], L = 0x0F0F0F0Fu, H = 0xF0F0F0F0u;
+            o[0] = make_uint4((d0 & L) | (d2 & L) << 4, (d0 >> 4 & L) | (d2 & H), (d1 & L) | (d3 & L) << 4, (d1 >> 4 & L) | (d3 & H));
+        }
+    } else if constexpr (DT == L3M_BF16) {
+        const uint16_t *e = (const uint16_t *)(src + (size_t)t * k * 32);
+        uint32_t *o = (uint32_t *)(q + slot * 64);
+#pragma unroll
+        for (int p = 0; p < 16; p++) {
+            const int i = 32 * b + 2 * p;
+            const size_t at = ((size_t)(i >> 1) * 16 + c) * 2;
+            o[p] = (i < k ? (uint32_t)e[at] : 0u) | (i + 1 < k ? (uint32_t)e[at + 1] << 16 : 0u);
+        }
+    } else {
+        const uint32_t *e = (const uint32_t *)(src + (size_t)t * k * 64);
+        uint32_t *o = (uint32_t *)(q + slot * 128);
+#pragma unroll
+        for (int p = 0; p < 32; p++) {
+            const int i = 32 * b + p;
+            o[p] = i < k ? e[(size_t)i * 16 + c] : 0u;
+        }
+    }
+}
+
 // STAGED: the activation is 16-byte aligned and at most GEMV_ACT_REGS * NT 16-byte words (gemv_staged).
 template <int DT, bool STAGED>
 __global__ void __launch_bounds__(NT) k_gemv(l3m_dmat m, const uint8_t *__restrict__ act_g, int k, float *__restrict__ y, int S) {
@@ -3967,6 +4013,9 @@ hipStream_t as_stream(void *s) { return s ? (hipStream_t)s : g_stream; }
 template <int DT> void launch_prep(const float *x, int k, void *act, hipStream_t st) {
     hipLaunchKernelGGL(k_prep<DT>, dim3((kpad(k) / 4 + NT - 1) / NT), dim3(NT), 0, st, x, k, (uint8_t *)act);
 }
+template <int DT> void launch_ltiles(const uint8_t *src, int ntiles, int k, uint8_t *q, uint8_t *s, unsigned n, hipStream_t st) {
+    hipLaunchKernelGGL(k_ltiles<DT>, dim3((n + NT - 1) / NT), dim3(NT), 0, st, src, ntiles, k, q, s);
+}
 // Nibble-block matrices (q4_0, mxfp4) of at least 128 tiles whose rows are 64, 128 or 256 blocks take
 // k_gemv_deep: 8 wavefronts per tile, nb / 32 blocks per lane (measured at 14336 x 4096, warm / cold against
 // the 4-wavefront k_gemv: q4_0 +10% / +7%, mxfp4 +6% / +4%; 16 wavefronts per tile was slower).
@@ -4335,6 +4384,21 @@ int l3m_k_prep(int dtype, const float *x, int k, void *act, void *stream) {
     hipStream_t st = as_stream(stream);
     DISPATCH(dtype, launch_prep, x, k, act, st);
     CKL("k_prep");
+    return 0;
+}
+
+size_t l3m_ltile_bytes(int dtype, int ntiles, int k) {
+    const size_t per = dtype == L3M_F32 ? (size_t)k * 64 : dtype == L3M_BF16 ? (size_t)k * 32
+                                                                             : (size_t)(k / 32) * (16 * (qbytes(dtype) + sbytes(dtype)));
+    return per * (size_t)ntiles;
+}
+int l3m_k_ltiles(int dtype, int ntiles, int k, const void *tiles, void *quant, void *scale, void *stream) {
+    if (k < 1 || ntiles < 1 || dtype < 0 || dtype >= L3M_NDTYPES || (quantized(dtype) && k % 32)) return fail_msg("ltiles: bad shape");
+    hipStream_t st = as_stream(stream);
+    const size_t n = (size_t)ntiles * (kpad(k) / 32) * 16;
+    if (n > 0x7FFFFFFF - NT) return fail_msg("ltiles: matrix too large");
+    DISPATCH(dtype, launch_ltiles, (const uint8_t *)tiles, ntiles, k, (uint8_t *)quant, (uint8_t *)scale, (unsigned)n, st);
+    CKL("k_ltiles");
     return 0;
 }
 
