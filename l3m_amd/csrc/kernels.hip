@@ -112,6 +112,10 @@ __device__ __forceinline__ uint32_t ldg1_if(const void *p, size_t i, bool ok) {
 template <bool COH> __device__ __forceinline__ uint4 ld16(const void *p, size_t i) { return COH ? ldcoh16(p, i) : ldg16(p, i); }
 // Element i of a uniform base p, or zeros with no memory access when ok is false (the offset past the
 // buffer's range): a load that needs no branch around it.
+template <bool COH> __device__ __forceinline__ uint4 ld16_if(const void *p, uint32_t byte, bool ok) {
+    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(buf(p), ok ? byte : OOB, 0, COH ? SC1 : 0));
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
 template <bool COH> __device__ __forceinline__ float4 ld16f_if(const void *p, size_t i, bool ok) {
     const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(buf(p), ok ? (uint32_t)(16 * i) : OOB, 0, COH ? SC1 : 0));
     return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
@@ -1681,12 +1685,16 @@ __device__ __forceinline__ float dot8_bf16(const float *q, uint4 k, float acc) {
 // exp(s - m) and the running exp-weighted V sum o, rescaled when m grows. With W > 1 the wavefronts'
 // (m, l, o) meet in LDS after one barrier and combine as exp(m_w - M) weights. K, V rows before pos come
 // from the LDS window (WIN) or the cache, row pos from cur (this step's rows, bf16 as the cache holds
-// them). vred: NWE * (hd + 2) floats of LDS. Ends with a barrier.
+// them). BATCH (from the cache): a chunk's K and V rows are all requested first, by buffer loads that answer a row
+// past the end with zeros and no access; loads under a branch a round are waited for one after the other. Taken by
+// the bodies with int8 step matrices, which have the 32 registers (8 heads of 64, 8 layers, positions 600-664: 4.5
+// us a pass less); a bf16 body's step spills with it (stories15M, which never reads the cache: 2% slower).
+// vred: NWE * (hd + 2) floats of LDS. Ends with a barrier.
 #ifndef L3M_ATT_LOG_IT
 #define L3M_ATT_LOG_IT 2
 #endif
 constexpr int ATT_LOG_IT = L3M_ATT_LOG_IT, ATT_IT = 1 << ATT_LOG_IT;
-template <bool WIN, bool COH>
+template <bool WIN, bool COH, bool BATCH>
 __device__ void attend_group(const l3m_dmodel &M, const l3m_dgroup &G, int layer, int pos, const float *qh, const uint16_t *cur,
                              const uint16_t *kvb, float *vred, float *att) {
     const int hd = M.hd, nv = hd >> 3, lg = nv <= 4 ? 2 : nv <= 8 ? 3 : nv <= 16 ? 4 : 5, LP = 1 << lg, PPW = 64 >> lg;
@@ -1707,8 +1715,10 @@ __device__ void attend_group(const l3m_dmodel &M, const l3m_dgroup &G, int layer
         if (active) {
             // (q0 + h) / hpk by an exact float reciprocal (both far below 2^20)
             const int kvl = (int)(((float)(G.q0 + h) + 0.5f) * ihpk) - G.kv0;
-            const uint16_t *kw = WIN ? kvb + kvl * win : M.kc + ((size_t)layer * M.n_kv + G.kv0 + kvl) * win;
-            const uint16_t *vw = WIN ? kvb + (G.nkv + kvl) * win : M.vc + ((size_t)layer * M.n_kv + G.kv0 + kvl) * win;
+            const int at = BATCH ? 0 : G.kv0 + kvl;   // BATCH: buffers over the layer's rows, the head's from row0 on
+            const uint16_t *kw = WIN ? kvb + kvl * win : M.kc + ((size_t)layer * M.n_kv + at) * win;
+            const uint16_t *vw = WIN ? kvb + (G.nkv + kvl) * win : M.vc + ((size_t)layer * M.n_kv + at) * win;
+            const uint32_t row0 = (uint32_t)((G.kv0 + kvl) * M.ctx);
             const uint4 *kcur = (const uint4 *)(cur + kvl * hd), *vcur = (const uint4 *)(cur + (G.nkv + kvl) * hd);
             float q[8];
             {
@@ -1721,11 +1731,31 @@ __device__ void attend_group(const l3m_dmodel &M, const l3m_dgroup &G, int layer
             for (int r0 = 0; (r0 * W + wi) * PPW < n; r0 += ATT_IT) {
                 float s[ATT_IT];
                 float cm = -INFINITY;
+                uint4 kb[ATT_IT], vb[ATT_IT];
+                if constexpr (BATCH) {
+#pragma unroll
+                    for (int k = 0; k < ATT_IT; k++) {
+                        const int t = ((r0 + k) * W + wi) * PPW + gl;
+                        kb[k] = ld16_if<COH>(kw, 16 * ((row0 + (uint32_t)t) * (uint32_t)nv + (uint32_t)j), t < pos && j < nv);
+                    }
+#pragma unroll
+                    for (int k = 0; k < ATT_IT; k++) {
+                        const int t = ((r0 + k) * W + wi) * PPW + gl;
+                        vb[k] = ld16_if<COH>(vw, 16 * ((row0 + (uint32_t)t) * (uint32_t)nv + (uint32_t)j), t < pos && j < nv);
+                    }
+                    asm volatile("" ::: "memory");
+                    const uint4 kc = kcur[j < nv ? j : 0], vc = vcur[j < nv ? j : 0];
+#pragma unroll
+                    for (int k = 0; k < ATT_IT; k++)
+                        if (((r0 + k) * W + wi) * PPW + gl == pos) { kb[k] = kc; vb[k] = vc; }
+                }
 #pragma unroll
                 for (int k = 0; k < ATT_IT; k++) {
                     const int t = ((r0 + k) * W + wi) * PPW + gl;
                     float part = 0.f;
-                    if (t < n && j < nv) {
+                    if constexpr (BATCH) {
+                        part = dot8_bf16(q, kb[k], 0.f);
+                    } else if (t < n && j < nv) {
                         uint4 kk;
                         if (t == pos) kk = kcur[j];
                         else if (WIN) kk = ((const uint4 *)(kw + (size_t)t * rs))[j];
@@ -1743,12 +1773,13 @@ __device__ void attend_group(const l3m_dmodel &M, const l3m_dgroup &G, int layer
 #pragma unroll
                 for (int k = 0; k < ATT_IT; k++) {
                     const int t = ((r0 + k) * W + wi) * PPW + gl;
-                    if (t < n) {
+                    if (BATCH || t < n) {             // batched: past the end p is 0 and the row zeros
                         const float p = expf(s[k] - mn);
                         l += p;
-                        if (j < nv) {
+                        if (BATCH || j < nv) {
                             uint4 vv;
-                            if (t == pos) vv = vcur[j];
+                            if constexpr (BATCH) vv = vb[k];
+                            else if (t == pos) vv = vcur[j];
                             else if (WIN) vv = ((const uint4 *)(vw + (size_t)t * rs))[j];
                             else vv = ld16<COH>(vw, (size_t)t * (hd >> 3) + j);
                             o[0] = fmaf(p, bf16_f32(vv.x & 0xFFFF), o[0]); o[1] = fmaf(p, bf16_f32(vv.x >> 16), o[1]);
@@ -2150,8 +2181,8 @@ __device__ __forceinline__ void attn_block(const l3m_dmodel &M, const l3m_dlayer
     __syncthreads();
     phase(gi, 5, pos, layer);
     if (mfma_att) attend_mfma(M, G, pos, qp, kvb, work, vred, att);
-    else if (kwin) attend_group<true, PRE>(M, G, layer, pos, qh, cur, kvb, vred, att);
-    else attend_group<false, PRE>(M, G, layer, pos, qh, cur, kvb, vred, att);
+    else if (kwin) attend_group<true, PRE, false>(M, G, layer, pos, qh, cur, kvb, vred, att);
+    else attend_group<false, PRE, AT == L3M_Q8_0>(M, G, layer, pos, qh, cur, kvb, vred, att);
     phase(gi, 6, pos, layer);
     // this step's k and v rows (bf16, engine.c:247-248) into the cache, for the kv heads this group writes,
     // by the wavefronts past those that prepare the attention output next (they go straight to the prep);
@@ -2649,8 +2680,8 @@ __global__ void __launch_bounds__(NTE) k_attend_decode(float *out, const float *
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (MODE == 2) attend_mfma(M, G, pos, qp, kvb, sc, vred, att);
-    else if (MODE == 1) attend_group<true, false>(M, G, 0, pos, qh, cur, kvb, vred, att);
-    else attend_group<false, false>(M, G, 0, pos, qh, cur, kvb, vred, att);
+    else if (MODE == 1) attend_group<true, false, false>(M, G, 0, pos, qh, cur, kvb, vred, att);
+    else attend_group<false, false, true>(M, G, 0, pos, qh, cur, kvb, vred, att);
     for (int i = tidx(); i < nqd; i += NTE) out[i] = att[i];
 }
 
