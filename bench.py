@@ -195,13 +195,10 @@ def cpu_first_logits(path, prompt, ctx, runs=3):
 
 def gpu_first_logits(A, path, prompt, ctx, reps=5):
     """Milliseconds to the first logits of the prompt on the GPU, median of reps after one call: batched
-    prefill replaying its captured graph (and the first call, which captures it), the same launches one by
-    one (L3M_PREFILL_GRAPH=0), and token by token (L3M_PREFILL=0)."""
+    prefill (and the first call), and token by token (L3M_PREFILL=0)."""
     out = {}
-    for key, env in (("ms_prefill", {}), ("ms_prefill_loose_launches", {"L3M_PREFILL_GRAPH": "0"}),
-                     ("ms_token_by_token", {"L3M_PREFILL": "0"})):
-        for k in ("L3M_PREFILL", "L3M_PREFILL_GRAPH"):
-            os.environ.pop(k, None)
+    for key, env in (("ms_prefill", {}), ("ms_token_by_token", {"L3M_PREFILL": "0"})):
+        os.environ.pop("L3M_PREFILL", None)
         os.environ.update(env)
         with A.Model(path, ctx=ctx) as m:
             t0 = time.perf_counter()
@@ -218,8 +215,7 @@ def gpu_first_logits(A, path, prompt, ctx, reps=5):
             if not env:
                 out["ms_prefill_first_call"] = round(first, 3)
                 out["prefilled_positions"] = m.prefilled
-    for k in ("L3M_PREFILL", "L3M_PREFILL_GRAPH"):
-        os.environ.pop(k, None)
+    os.environ.pop("L3M_PREFILL", None)
     return out
 
 

@@ -67,7 +67,6 @@ struct l3m_model {
     float        temp;         // the running generate call's temperature (0: greedy)
     l3m_pflayer *pf;           // batched prompt prefill: per-layer full matrices, NULL when unavailable
     l3m_pfbuf    pfb;
-    l3m_pfgraphs *pfg;         // the prefill's captured graphs (NULL: loose launches, L3M_PREFILL_GRAPH=0)
     int          prefill_min;  // prompts of at least this many tokens are prefilled (L3M_PREFILL_MIN)
     int          prefilled;    // positions the last generate call prefilled
     int          logits_fresh;
@@ -560,8 +559,6 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
         m->pfb.q = dalloc(m, ctx * nqd * 4);
         m->pfb.att = dalloc(m, ctx * nqd * 4);
         if (!m->pfb.x || !m->pfb.act.q || !m->pfb.act.s || !m->pfb.hact.q || !m->pfb.hact.s || !m->pfb.q || !m->pfb.att) return fail(m, "out of device memory");
-        const char *pg = getenv("L3M_PREFILL_GRAPH");  // 0: loose launches (for comparison)
-        if ((!pg || strcmp(pg, "0")) && !(m->pfg = l3m_pfgraphs_new())) return fail(m, "out of host memory");
     }
     d->logits = dalloc(m, (size_t)NSLOTS * d->vocab * 4);
     // persistent kernel: one workgroup per CU (the LDS request keeps a second one off each CU); the body
@@ -643,7 +640,6 @@ void l3m_free(l3m_model *m) {
     if (!m) return;
     l3m_dev_sync();
     l3m_graphs_free(m->graphs);
-    l3m_pfgraphs_free(m->pfg);
     l3m_dev_host_free(m->call_host);
     l3m_dev_host_free(m->out_host);
     l3m_dev_event_free(m->ev[0]);
@@ -757,8 +753,10 @@ static int run_steps(l3m_model *m, const int32_t *prompt, int n_prompt, int max_
         if (l3m_dev_upload_async(m->call_dev, m->call_host, m->call_tok + (size_t)n_prompt * 4)) return -1;
         from = -1;
         if (m->cold && evict(m)) return -1;
-        if (m->pfg ? l3m_prefill_graph(m->pfg, d, m->pf, &m->pfb, n_prompt - 1) : l3m_prefill(d, m->pf, &m->pfb, n_prompt - 1, NULL))
-            return -1;
+        // launched one by one: a kernel takes 3-5 us, a launch 1.6, so the GPU never waits. As a captured graph per
+        // prompt length the same kernels took as long (64 tokens, 30 layers: 1509 us against 1497; 480: 2306 against
+        // 2264), and each length's first prompt 0.5 ms more for the capture
+        if (l3m_prefill(d, m->pf, &m->pfb, n_prompt - 1, NULL)) return -1;
         m->prefilled = n_prompt - 1;
     }
     const int live = on_token != NULL || bos >= 0 || eos >= 0, depth = m->cold ? 1 : 2;

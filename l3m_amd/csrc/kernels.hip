@@ -4811,50 +4811,6 @@ int l3m_graphs_launch(l3m_graphs *g, int with_head, void *stream) {
     return 0;
 }
 
-constexpr int PF_GRAPHS = 8;
-struct l3m_pfgraphs {
-    int P[PF_GRAPHS];                 // 0: an empty entry
-    hipGraphExec_t e[PF_GRAPHS];
-    unsigned long long used[PF_GRAPHS], tick;
-};
-
-l3m_pfgraphs *l3m_pfgraphs_new(void) { return (l3m_pfgraphs *)calloc(1, sizeof(l3m_pfgraphs)); }
-
-void l3m_pfgraphs_free(l3m_pfgraphs *g) {
-    if (!g) return;
-    for (int i = 0; i < PF_GRAPHS; i++)
-        if (g->P[i]) (void)hipGraphExecDestroy(g->e[i]);
-    free(g);
-}
-
-int l3m_prefill_graph(l3m_pfgraphs *g, const l3m_dmodel *M, const l3m_pflayer *L, const l3m_pfbuf *B, int P) {
-    if (P < 1) return 0;
-    int k = -1, lru = 0;
-    for (int i = 0; i < PF_GRAPHS; i++) {
-        if (g->P[i] == P) k = i;
-        if (g->used[i] < g->used[lru]) lru = i;
-    }
-    if (k < 0) {                                       // capture this length into the least recently used entry
-        k = lru;
-        if (g->P[k]) { (void)hipGraphExecDestroy(g->e[k]); g->P[k] = 0; }
-        hipGraph_t graph = nullptr;
-        if (hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return fail_msg("prefill graph capture");
-        const int rc = l3m_prefill(M, L, B, P, g_stream);
-        const hipError_t ec = hipStreamEndCapture(g_stream, &graph);
-        if (ec != hipSuccess || rc) {
-            if (ec == hipSuccess && graph) (void)hipGraphDestroy(graph);   // a capture that ended holds a graph
-            return fail_msg("prefill graph capture");
-        }
-        const hipError_t e = hipGraphInstantiate(&g->e[k], graph, NULL, NULL, 0);
-        (void)hipGraphDestroy(graph);
-        if (e != hipSuccess) return fail_msg("prefill graph instantiate");
-        g->P[k] = P;
-    }
-    g->used[k] = ++g->tick;
-    CK(hipGraphLaunch(g->e[k], g_stream));
-    return 0;
-}
-
 // Mean microseconds per launch of iters launches queued back to back, after one untimed launch: one pair
 // of events around them all (events around each launch would add their own markers' time to every
 // figure). For a kernel shorter than the launch interval (l3m_time_launch_interval) this is the launch rate.
