@@ -3707,10 +3707,57 @@ __global__ void __launch_bounds__(64) k_pf_attend(const float *qb, int P, int n_
 //    free, V's operand takes the same): p, as three bf16 parts, goes from the softmax to B in registers.
 //    A = V^T, dims by positions: the wavefront transposes the chunk's V rows (4 positions x 8 dims a lane)
 //    into its own LDS span, rows of 40 elements, the lane's 8 positions contiguous.
+// A masked position's p is 0 and a part of q may be, but 0 times an infinity or a NaN in a V or K row is NaN: where
+// any of the tile's outputs is not finite, its tokens are done again one at a time (pf_attn_token), over their
+// own positions alone.
 // No barrier before the end. Bound by the chunk's chain (loads, two products, expf, LDS round trip), not by
 // bytes or products: 9 heads of 64, 479 tokens: 11.1 us a layer, against 55.7 for k_pf_attend (one wavefront
 // per token and head, a lane per position: every token reads every K and V row again); 63 tokens: 5.0 (7.0).
 constexpr int PFA_W = 4, PFA_T = 16, PFA_C = 32, PFA_VROW = 40;
+// Attention of one token over positions 0..tok by one wavefront, every product in f32 and no row past tok read:
+// lane l scores position l of each 64, then adds dims l and l + 64 up. buf: HD + 64 floats of the wavefront's
+// own LDS; the output is left in its first HD.
+template <int HD>
+__device__ void pf_attn_token(const float *q, const uint16_t *K, const uint16_t *V, int tok, float scale, float *buf) {
+    constexpr int ND = (HD + 63) / 64;
+    const int lane = tidx() & 63;
+    float *ps = buf + HD;
+    auto lds_done = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __builtin_amdgcn_wave_barrier(); };
+    lds_done();
+    for (int d = lane; d < HD; d += 64) buf[d] = q[d];
+    lds_done();
+    float m = -INFINITY, l = 0.f, o[ND];
+#pragma unroll
+    for (int i = 0; i < ND; i++) o[i] = 0.f;
+    for (int p0 = 0; p0 <= tok; p0 += 64) {
+        const int n = min(tok - p0 + 1, 64);
+        float s = -INFINITY;
+        if (lane < n) {
+            float dot = 0.f;
+            for (int d = 0; d < HD; d++) dot = fmaf(buf[d], bf16_f32(K[(size_t)(p0 + lane) * HD + d]), dot);
+            s = dot * scale;
+        }
+        const float nm = fmaxf(m, lanes_max<64>(s)), base = nm == -INFINITY ? 0.f : nm, r = expf(m - base);
+        const float p = lane < n ? expf(s - base) : 0.f;
+        l = l * r + lanes_sum<64>(p);
+        ps[lane] = p;
+        lds_done();
+#pragma unroll
+        for (int i = 0; i < ND; i++) {
+            const int d = lane + 64 * i;
+            if (d < HD) {
+                o[i] *= r;
+                for (int j = 0; j < n; j++) o[i] = fmaf(ps[j], bf16_f32(V[(size_t)(p0 + j) * HD + d]), o[i]);
+            }
+        }
+        lds_done();
+        m = nm;
+    }
+#pragma unroll
+    for (int i = 0; i < ND; i++)
+        if (lane + 64 * i < HD) buf[lane + 64 * i] = o[i] / l;
+    lds_done();
+}
 template <int DT, int HD>
 __global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qb, int P, int n_heads, int n_kv, int ctx, int layer, float scale,
                                                         const uint16_t *kc, const uint16_t *vc, float *att, l3m_pfact act) {
@@ -3718,8 +3765,11 @@ __global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qb, int P, 
     constexpr size_t VT = (size_t)HD * PFA_VROW * 2;                     // one wavefront's V^T chunk; its merge span is no larger
     static_assert((size_t)PFA_T * OROW * 4 <= VT, "the merge spans fit the V^T spans");
     __shared__ __align__(16) uint8_t lds[PFA_W * VT];
+    static_assert((HD + 64) * 4 <= VT, "pf_attn_token's floats too");
     __shared__ float ml[2][PFA_W][PFA_T];
+    __shared__ int odd;                               // an output that is not finite
     const int lane = tidx() & 63, wave = wave_id(), c16 = lane & 15, quarter = lane >> 4;
+    if (tidx() == 0) odd = 0;
     // the tiles with the most positions first
     const int t0 = PFA_T * ((int)gridDim.x - 1 - (int)blockIdx.x), h = blockIdx.y, kv = h / (n_heads / n_kv);
     const int width = n_heads * HD, tmax = (t0 + PFA_T < P ? t0 + PFA_T : P) - 1, tok = min(t0 + c16, tmax);
@@ -3834,6 +3884,14 @@ __global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qb, int P, 
     for (int n = 0; n < NT16; n++) *(float4 *)(om + 16 * n + 4 * quarter) = make_float4(o[n][0], o[n][1], o[n][2], o[n][3]);
     if (quarter == 0) { ml[0][wave][c16] = m; ml[1][wave][c16] = l; }
     __syncthreads();
+    // the output's dims d .. d + 3 of token t
+    auto put = [&](int t, int d, float4 y, bool store) {
+        if constexpr (HD % 32 == 0 || DT == L3M_BF16) {   // whole blocks of the head: prepared here, 8 lanes a block
+            pf_put4<DT>(act, t, (n_heads * HD) >> 5, h * HD + d, y, store);
+        } else if (store) {
+            *(float4 *)(att + (size_t)t * n_heads * HD + h * HD + d) = y;
+        }
+    };
     // each thread 4 dims of a token: the wavefronts' parts in order, scaled to the common maximum (wavefront 0
     // always has position 0)
     for (int u = tidx(); u < PFA_T * HD / 4; u += 64 * PFA_W) {
@@ -3851,11 +3909,16 @@ __global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qb, int P, 
             y.x += x.x * f; y.y += x.y * f; y.z += x.z * f; y.w += x.w * f;
         }
         y = make_float4(y.x / den, y.y / den, y.z / den, y.w / den);
-        if constexpr (HD % 32 == 0 || DT == L3M_BF16) {   // whole blocks of the head: prepared here, 8 lanes a block
-            pf_put4<DT>(act, t, (n_heads * HD) >> 5, h * HD + 4 * d4, y, t < P);
-        } else if (t < P) {
-            *(float4 *)(att + (size_t)t * n_heads * HD + h * HD + 4 * d4) = y;
-        }
+        if (!(y.x * 0.f + y.y * 0.f + y.z * 0.f + y.w * 0.f == 0.f)) odd = 1;
+        put(t, 4 * d4, y, t < P);
+    }
+    __syncthreads();
+    if (!odd) return;
+    for (int tt = wave; tt < PFA_T && t0 + tt < P; tt += PFA_W) {
+        float *buf = (float *)vt;
+        pf_attn_token<HD>(qb + (size_t)(t0 + tt) * width + h * HD, K, V, t0 + tt, scale, buf);
+        const bool mine = 4 * lane < HD;
+        put(t0 + tt, 4 * lane, mine ? *(const float4 *)(buf + 4 * lane) : make_float4(0.f, 0.f, 0.f, 0.f), mine);
     }
 }
 

@@ -16,6 +16,7 @@ import numpy as np
 import pytest
 
 import l3m_amd as A
+from weights import read_tensors, to_bf16
 
 pytestmark = pytest.mark.gpu
 GQA = A.Config("pf_gqa", dim=192, n_layers=3, n_heads=6, n_kv_heads=2, ffn_dim=512, vocab=512, ctx=128, dtype="q8_0")
@@ -267,3 +268,98 @@ def test_prefill_bf16(models, oracle, monkeypatch, cfg, n_prompt):
     for g, w in zip(kv, want):
         for a, b in zip(g, w):
             assert np.abs(bf16(a) - bf16(b)).max() <= 0.01 * np.abs(bf16(b)).max()
+
+
+def patch(path, out, edit):
+    """A copy of the .l3m file at path with its tensors changed by edit(name -> writable uint8 view, 2-D for matrices)."""
+    raw = np.fromfile(path, np.uint8)
+    tensors, _ = read_tensors(path)
+    toc = int(raw[72:80].view(np.uint64)[0])
+    views = {}
+    for i, (name, (_, _, data)) in enumerate(tensors.items()):
+        off, size = (int(v) for v in raw[toc + 120 * i + 104:toc + 120 * i + 120].view(np.uint64))
+        views[name] = raw[off:off + size].reshape(data.shape)
+    edit(views)
+    raw.tofile(out)
+    return out
+
+
+class Codes:
+    """Element writes into a matrix of file rows: q8_0 codes (and block scales), or bf16 values."""
+
+    def __init__(self, dtype, rows):
+        self.q8, self.n = dtype == "q8_0", len(rows)
+        self.r = rows.reshape(self.n, -1, 34) if self.q8 else rows.view(np.uint16)
+
+    def put(self, row, col, code, scale=None, alone=False):
+        """Column col = code (q8_0) or code * scale (bf16; scale 1 / 127); alone: the rest of its 32-block zero."""
+        if self.q8:
+            b = self.r[row, col // 32]
+            if alone:
+                b[..., 2:] = 0
+            b[..., 2 + col % 32] = np.int8(code).view(np.uint8)
+            if scale is not None:
+                b[..., :2] = np.array([scale], np.float16).view(np.uint8)
+        else:
+            if alone:
+                self.r[row, col // 32 * 32:col // 32 * 32 + 32] = 0
+            self.r[row, col] = to_bf16([code * (1 / 127 if scale is None else scale)])[0]
+
+
+@pytest.mark.parametrize("kind", ["nan_v", "inf_k"])
+@pytest.mark.parametrize("hd", [32, 48, 64])
+@pytest.mark.parametrize("dtype", ["q8_0", "bf16"])
+def test_prefill_values_that_are_not_finite(models, oracle, tmp_path, dtype, hd, kind):
+    """A prompt token X (position 5 of 20) whose K or V row in layer 0 is not finite, in one kv head; every other row
+    is. nan_v: its V row holds NaN in every other dim (a sum of +inf and -inf), which the tokens before it never attend, so their second
+    layer's rows are the oracle's; int8 bodies drop a NaN in the next rounding, so there the later tokens' are too.
+    inf_k: its K row ends in infinities against which every q is negative: p is 0 exactly, and every row is the
+    oracle's. Bar: 2% of the largest, as test_prefill_logits."""
+    cfg = A.Config(f"pf_odd{hd}", dim=4 * hd, n_layers=2, n_heads=4, n_kv_heads=2, ffn_dim=256, vocab=128, ctx=64, dtype=dtype)
+    base = models.get(cfg, dtype, seed=21, std=0.05, norm_jitter=0.1)
+    P, at, X = 20, 5, 7
+    ids = [X if i == at else 10 + i for i in range(P + 1)]
+    a, b, const = 0, 32, 64                           # input columns: X alone is not 0 in a and b; no token is in const
+
+    def edit(t):
+        embed = Codes(dtype, t["embed"])
+        for col in (a, b):
+            embed.put(slice(None), col, 0)
+            embed.put(X, col, 100)
+        t["blk.0.attn_norm"].view(np.float32)[[a, b]] = 1e36
+        wq, wk, wv = (Codes(dtype, t[f"blk.0.{n}"]) for n in ("wq", "wk", "wv"))
+        for col in (a, b):
+            for w in (wq, wk, wv):
+                w.put(slice(None), col, 0)
+        if kind == "nan_v":
+            for col, code in ((a, 127), (b, -127)):
+                wv.put(slice(0, hd, 2), col, code, 6e4, alone=True)
+        else:
+            embed.put(slice(None), const, 100)
+            # the last RoPE pair hardly turns: +inf in row hd - 2 of kv head 0 from X makes both of its pair, and that
+            # pair's q rows are negative for every token in the head's two query heads
+            wk.put(slice(hd - 2, hd - 1), a, 127, 6e4, alone=True)
+            for h in (0, 1):
+                rows = slice((h + 1) * hd - 2, (h + 1) * hd)
+                if dtype == "q8_0":
+                    wq.r[rows, :, 2:] = 0
+                else:
+                    wq.r[rows] = 0
+                wq.put(rows, const, -127)
+
+    path = patch(base, tmp_path / "odd.l3m", edit)
+    om = oracle.load(path)
+    om.generate(ids, 0)
+    with A.Model(path) as m:
+        m.generate(ids, 0)
+        assert m.prefilled == P
+        for kvh in range(2):
+            first = [bf16(w) for w in om.kv_rows(0, kvh, 0, P, hd)]
+            bad = first[1] if kind == "nan_v" else first[0]
+            assert (kvh == 0) == (not np.isfinite(bad[at]).all()) and np.isfinite(np.delete(bad, at, 0)).all()
+            for name, got, want in zip("kv", m.kv_rows(1, kvh, 0, P), om.kv_rows(1, kvh, 0, P, hd)):
+                g, w = bf16(got), bf16(want)
+                if kind == "nan_v" and dtype == "bf16":
+                    g, w = g[:at], w[:at]
+                assert np.isfinite(w).all() and np.isfinite(g).all(), (name, kvh)
+                assert np.abs(g - w).max() <= 0.02 * np.abs(w).max(), (name, kvh, np.abs(g - w).max() / np.abs(w).max())
