@@ -1746,8 +1746,8 @@ __device__ void attend_group(const l3m_dmodel &M, const l3m_dgroup &G, int layer
                     asm volatile("" ::: "memory");
                     const uint4 kc = kcur[j < nv ? j : 0], vc = vcur[j < nv ? j : 0];
 #pragma unroll
-                    for (int k = 0; k < ATT_IT; k++)
-                        if (((r0 + k) * W + wi) * PPW + gl == pos) { kb[k] = kc; vb[k] = vc; }
+                    for (int k = 0; k < ATT_IT; k++)  // lanes past the head keep zeros: their zero q times an infinity is NaN
+                        if (((r0 + k) * W + wi) * PPW + gl == pos && j < nv) { kb[k] = kc; vb[k] = vc; }
                 }
 #pragma unroll
                 for (int k = 0; k < ATT_IT; k++) {

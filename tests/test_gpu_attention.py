@@ -55,6 +55,23 @@ def test_decode_attention_matches_oracle(dev, oracle, case, qscale):
     print(f"worst |gpu - oracle| {worst:.2e}", flush=True)
 
 
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"mode{c[0]}-hd{c[1]}-nq{c[2]}-nkv{c[3]}")
+def test_decode_attention_infinite_score(dev, oracle, case):
+    """This step's K row begins with an infinity against which every q is negative: its score is -inf, its weight 0, and
+    the outputs are the oracle's over the other positions. Mode 2's third bf16 part of q may be 0, and its product
+    with the infinity NaN: q holds values of 24 bits whose three parts are negative."""
+    mode, hd, nq, nkv, ctx = case
+    for pos in (1, 40, 255):
+        print(f"infinite score, mode {mode} hd {hd} nq {nq} nkv {nkv} pos {pos}", flush=True)
+        q, kc, vc = inputs(77 * hd + pos, nq, nkv, hd, ctx, 1.0)
+        q[:, 0] = -(1 + 2.0 ** -9 + 2.0 ** -18)
+        kc[:, pos, 0] = 0x7F80
+        got = dev.attend_decode(mode, q, kc, vc, nq, nkv, hd, ctx, pos)
+        ref = want(oracle, q, kc, vc, nq, nkv, hd, pos)
+        assert np.isfinite(ref).all() and np.abs(got - ref).max() <= 1e-5, pos
+        dev.free_all()
+
+
 def test_attention_modes_agree_with_decode_choice(dev):
     """The mode a decode step picks (l3m_attention_mode) for the benchmark shapes: matrix cores for hd 64
     and 48 with the window in LDS, the VALU window form for a head dimension off the multiples of 16, the
