@@ -9,6 +9,7 @@
 // step, and go as they are stored to the matrix cores (fp4 operand) in the large standalone matvecs.
 // Reductions are fixed-order (wavefront shuffles, then LDS), so results are run-to-run identical.
 #include <hip/hip_runtime.h>
+#include <hip/hip_ext.h>
 #include <math.h>
 #include <pthread.h>
 #include <stdint.h>
@@ -4066,9 +4067,17 @@ hipStream_t g_stream;
 // The device address of `scratch` (below) on each device the library set up, from hipGetSymbolAddress: the
 // array's name in host code is a host-side stand-in, not a device address.
 void *g_scratch_dev[16];
-void *g_attend_ws;                   // the same of attend_ws, from the first call that wants one
-hipStream_t g_attend_stream[16];     // the stream of each workspace, under g_attend_lock
-int g_attend_streams;
+// k_attend's workspaces (attend_ws below), under g_attend_lock. Workspace 0 is the library stream's, 1 the null
+// stream's (the library's stream before l3m_dev_init); the others go to callers' streams, each with the stream that
+// used it last and that launch's own completion event. busy: a call has it and has not launched yet.
+constexpr int ATT_STREAMS = 18, ATT_OWN = 2;
+struct AttWs {
+    hipStream_t stream;
+    hipEvent_t done;
+    bool busy;
+};
+AttWs g_attend[ATT_STREAMS];
+uint8_t *g_attend_ws;
 pthread_mutex_t g_attend_lock = PTHREAD_MUTEX_INITIALIZER;
 int g_ready = -1;
 char g_name[128];
@@ -4321,12 +4330,77 @@ template <int DT> int launch_step_mv(int form, const l3m_dmat &m, const float *x
 // the process ends; every call on a GPU shares it and it keeps the last call's contents.
 constexpr size_t ATTEND_STATIC_BYTES = 4u << 20;
 static __device__ __align__(256) uint8_t scratch[ATTEND_STATIC_BYTES];
-// k_attend's workspaces, one per stream that uses it (calls on one stream follow one another), each stream's from
-// its first call on. A stream past the last one, a stream under capture (its graph may be replayed on another) and
-// the special handles (one name for several streams) have none: their calls take one workgroup.
-constexpr int ATT_STREAMS = 16;
+// k_attend's workspaces on device 0 (g_attend).
 static __device__ __align__(256) uint8_t attend_ws[ATT_STREAMS][ATT_WS];
 static_assert(ATT_WS % 256 == 0, "every workspace 256-byte aligned");
+
+// The workspace a call on st takes, or -1: none, one workgroup does it. Two calls may share one only if the
+// second cannot begin before the first has ended:
+//  - the library's stream and the null stream have their own, and neither is destroyed with work in flight;
+//  - any other stream takes the one its handle used last, behind that call's event (a handle may name a new
+//    stream whose predecessor was destroyed with the call still running), else one whose last call has ended.
+//    Never one that is in use: a stream does not wait for another's work.
+// None for a stream under capture (its graph may be replayed on another), the special handles (one name for several
+// streams) and streams of another device (the workspaces are device 0's).
+static int attend_take(hipStream_t st) {
+    int dev = -1, got = -1;
+    if ((uintptr_t)st == 1 || (uintptr_t)st == 2 || hipGetDevice(&dev) != hipSuccess || dev != 0) return -1;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (st && (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)) return -1;
+    if (st && st == g_stream) return 0;
+    pthread_mutex_lock(&g_attend_lock);
+    if (!st) {                                        // before l3m_dev_init: nothing resolved the array yet
+        if (g_attend_ws || hipGetSymbolAddress((void **)&g_attend_ws, HIP_SYMBOL(attend_ws)) == hipSuccess) got = 1;
+    } else if (g_attend_ws && hipStreamGetDevice(st, &dev) == hipSuccess && dev == 0) {
+        // an event may be asked for its state while another thread captures
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        for (int i = ATT_OWN; i < ATT_STREAMS && got < 0; i++) {
+            const AttWs &w = g_attend[i];
+            if (!w.busy && w.done && w.stream == st && hipStreamWaitEvent(st, w.done, 0) == hipSuccess) got = i;
+        }
+        if (got < 0) {
+            for (int i = ATT_OWN; i < ATT_STREAMS && got < 0; i++) {
+                AttWs &w = g_attend[i];
+                if (!w.busy && (w.done ? hipEventQuery(w.done) : hipEventCreate(&w.done)) == hipSuccess) got = i;
+            }
+            (void)hipGetLastError();                  // an event not ready is no error of the call's
+        }
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (got >= 0) g_attend[got].busy = true;
+    }
+    pthread_mutex_unlock(&g_attend_lock);
+    return got;
+}
+
+// k_attend over n rows. Up to ATT_ALONE batches of rows go to one workgroup: a second costs the hand-over (about
+// 3.5 us), a batch about 0.9 us (hd 128, 256 rows: 6.8 us in one; 512 rows: 8.3 us spread, 10.4 in one). More are spread over up to ATT_SPLITS workgroups.
+constexpr int ATT_ALONE = 4;
+// On a caller's stream the launch carries its workspace's event (hipExtLaunchKernel; hd 128, 4001 rows queued back
+// to back: 12.6-12.7 us, 12.5-12.6 without one, 15.5 with an event recorded behind the launch; waited for alone 26.5-28.9,
+// 24.2-25.1, 24.8-26.1).
+template <int L> static void attend_l(float *out, const float *q, const uint16_t *k, const uint16_t *v, int n, int hd, int stride, hipStream_t st) {
+    const int rows = NT / L * ATT_U, batches = (n + rows - 1) / rows, own = batches > ATT_ALONE ? attend_take(st) : -1;
+    uint8_t *ws = own < 0 ? nullptr : g_attend_ws + (size_t)own * ATT_WS;
+    const int per = rows * (ws ? (batches + ATT_SPLITS - 1) / ATT_SPLITS : batches), grid = (n + per - 1) / per;
+    if (own < ATT_OWN) {
+        hipLaunchKernelGGL(k_attend<L>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws);
+        return;
+    }
+    hipExtLaunchKernelGGL(k_attend<L>, dim3(grid), dim3(NT), 0, st, nullptr, g_attend[own].done, 0, out, q, k, v, n, hd, stride, per, ws);
+    pthread_mutex_lock(&g_attend_lock);
+    g_attend[own].stream = st;
+    g_attend[own].busy = false;
+    pthread_mutex_unlock(&g_attend_lock);
+}
+static void launch_attend(float *out, const float *q, const uint16_t *k, const uint16_t *v, int n, int hd, int stride, hipStream_t st) {
+    if (hd <= 8) attend_l<1>(out, q, k, v, n, hd, stride, st);
+    else if (hd <= 16) attend_l<2>(out, q, k, v, n, hd, stride, st);
+    else if (hd <= 32) attend_l<4>(out, q, k, v, n, hd, stride, st);
+    else if (hd <= 64) attend_l<8>(out, q, k, v, n, hd, stride, st);
+    else if (hd <= 128) attend_l<16>(out, q, k, v, n, hd, stride, st);
+    else attend_l<32>(out, q, k, v, n, hd, stride, st);
+}
 
 // =============================================================================================== C ABI
 
@@ -4348,6 +4422,9 @@ void l3m_dev_shutdown(void) {
     for (int i = 0; i < 2; i++)
         for (int j = 0; j < 2; j++)
             if (g_dec_ev[i][j]) { (void)hipEventDestroy(g_dec_ev[i][j]); g_dec_ev[i][j] = nullptr; }
+    for (AttWs &w : g_attend)                         // a call still running keeps its event
+        if (w.done && !w.busy && hipEventQuery(w.done) == hipSuccess) { (void)hipEventDestroy(w.done); w = AttWs{}; }
+    (void)hipGetLastError();
     (void)hipStreamDestroy(g_stream);
     g_stream = nullptr;
     g_ready = 0;
@@ -4371,6 +4448,7 @@ int l3m_dev_init(void) {
     const char *coop = getenv("L3M_COOP");
     g_coop = !(coop && !strcmp(coop, "0"));
     CK(hipGetSymbolAddress(&g_scratch_dev[0], HIP_SYMBOL(scratch)));
+    CK(hipGetSymbolAddress((void **)&g_attend_ws, HIP_SYMBOL(attend_ws)));
     int lds = 0;
     if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, 0) == hipSuccess && lds > 0) g_lds_max = (unsigned)lds;
     CK(hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking));
@@ -4507,44 +4585,6 @@ int l3m_k_gemv(const l3m_dmat *m, const void *act, int k, float *y, void *stream
     return 0;
 }
 
-// The workspace of a stream, or NULL when it has none. Before l3m_dev_init the library's stream is the null
-// stream: one stream, never captured.
-static uint8_t *attend_workspace(hipStream_t st) {
-    if ((uintptr_t)st == 1 || (uintptr_t)st == 2) return nullptr;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (st && (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)) return nullptr;
-    pthread_mutex_lock(&g_attend_lock);
-    if (!g_attend_ws && hipGetSymbolAddress(&g_attend_ws, HIP_SYMBOL(attend_ws)) != hipSuccess) {
-        (void)hipGetLastError();
-        g_attend_ws = nullptr;
-        pthread_mutex_unlock(&g_attend_lock);
-        return nullptr;
-    }
-    int i = 0;
-    while (i < g_attend_streams && g_attend_stream[i] != st) i++;
-    if (i == g_attend_streams && i < ATT_STREAMS) g_attend_stream[g_attend_streams++] = st;
-    pthread_mutex_unlock(&g_attend_lock);
-    return i < ATT_STREAMS ? (uint8_t *)g_attend_ws + (size_t)i * ATT_WS : nullptr;
-}
-
-// k_attend over n rows. Up to ATT_ALONE batches of rows go to one workgroup: a second costs the hand-over (about
-// 3.5 us), a batch about 0.9 us (hd 128, 256 rows: 6.8 us in one; 512 rows: 8.3 us spread, 10.4 in one). More are spread over up to ATT_SPLITS workgroups.
-constexpr int ATT_ALONE = 4;
-static void launch_attend(float *out, const float *q, const uint16_t *k, const uint16_t *v, int n, int hd, int stride, hipStream_t st) {
-    int L = 1;
-    while (8 * L < hd) L *= 2;
-    const int rows = NT / L * ATT_U, batches = (n + rows - 1) / rows;
-    uint8_t *ws = batches > ATT_ALONE ? attend_workspace(st) : nullptr;
-    const int per = rows * (ws ? (batches + ATT_SPLITS - 1) / ATT_SPLITS : batches), grid = (n + per - 1) / per;
-    switch (L) {
-    case 1: hipLaunchKernelGGL(k_attend<1>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws); break;
-    case 2: hipLaunchKernelGGL(k_attend<2>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws); break;
-    case 4: hipLaunchKernelGGL(k_attend<4>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws); break;
-    case 8: hipLaunchKernelGGL(k_attend<8>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws); break;
-    case 16: hipLaunchKernelGGL(k_attend<16>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws); break;
-    default: hipLaunchKernelGGL(k_attend<32>, dim3(grid), dim3(NT), 0, st, out, q, k, v, n, hd, stride, per, ws);
-    }
-}
 // The most positions a call takes: 4 (hd + ceil4(pos + 1) + NT + 8) bytes within LDS_MAX.
 static bool attend_fits(int pos, int hd) { return 4 * ((size_t)hd + ((pos + 4) & ~3) + NT + 8) <= LDS_MAX; }
 

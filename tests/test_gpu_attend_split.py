@@ -54,7 +54,7 @@ def test_attend_large_values_and_masked_rows(dev, oracle):
 
 
 def test_attend_many_streams_and_capture(dev, oracle):
-    """18 streams with a call each in flight (16 of them get a workspace), three rounds of other inputs; then a
+    """18 streams with a call each in flight (two more than there are workspaces), three rounds of other inputs; then a
     call recorded into a graph, replayed between other calls on the same stream."""
     hip = C.CDLL("libamdhip64.so")
     n, hd = 3000, 64
@@ -87,4 +87,44 @@ def test_attend_many_streams_and_capture(dev, oracle):
     assert hip.hipGraphExecDestroy(ex) == 0 and hip.hipGraphDestroy(graph) == 0
     for st in streams:
         assert hip.hipStreamDestroy(st) == 0
+    dev.free_all()
+
+
+def test_attend_streams_come_and_go(dev, oracle):
+    """40 streams, 20 at a time, each used and destroyed, the last 20 with their calls just queued: a workspace goes back
+    when its last call has ended, so a later stream's result is the library stream's bit for bit (the split's order of
+    sums; one workgroup's differs), and handles that come up again are safe."""
+    hip = C.CDLL("libamdhip64.so")
+    n, hd = 3000, 64
+    q, k, v = inputs(8, n, hd, hd)
+    dq, dk, dv, do = dev.put(q), dev.put(k), dev.put(v), dev.alloc(hd * 4)
+
+    def call(st):
+        assert dev.lib.l3m_k_attend(do, dq, dk, dv, n - 1, hd, hd, st) == 0
+
+    call(None)
+    want = dev.get(do, hd, np.float32)
+    assert np.abs(want - oracle.attend(q, k, v, n - 1, hd, hd)).max() <= 1e-5
+    for rnd in range(3):
+        streams = []
+        for _ in range(20):
+            st = C.c_void_p()
+            assert hip.hipStreamCreateWithFlags(C.byref(st), 1) == 0
+            streams.append(st)
+        for st in streams:
+            call(st)
+            if rnd < 2:
+                assert hip.hipStreamSynchronize(st) == 0
+                got = dev.get(do, hd, np.float32)
+                assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (rnd, np.abs(got - want).max())
+        for st in streams:
+            assert hip.hipStreamDestroy(st) == 0
+    st = C.c_void_p()
+    assert hip.hipStreamCreateWithFlags(C.byref(st), 1) == 0
+    for _ in range(50):
+        call(st)
+    assert hip.hipDeviceSynchronize() == 0
+    got = dev.get(do, hd, np.float32)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    assert hip.hipStreamDestroy(st) == 0
     dev.free_all()
