@@ -267,6 +267,30 @@ static int upload_prefill(l3m_model *m, const l3m_mapped *f, int l, int dt, cons
     return rc || P->qkv.dtype != (dt == L3M_BF16 ? L3M_BF16 : L3M_Q8_0) ? -1 : 0;
 }
 
+// m->pf and m->pfb, or, when the device (or the host) has no room for them, everything as before and m->pf NULL.
+static void add_prefill(l3m_model *m) {
+    const l3m_dmodel *d = &m->dm;
+    const int mark = m->n_allocs;
+    m->pf = calloc((size_t)d->n_layers, sizeof *m->pf);
+    int ok = m->pf != NULL;
+    for (int l = 0; l < d->n_layers && ok; l++) ok = !upload_prefill(m, &m->f, l, (int)l3m_map_blk(&m->f, l, "wq")->dtype, &m->layers[l]);
+    if (ok) {
+        // activations of whole 64-token groups (a GEMM's workgroup reads up to 32 tokens, past the prompt's end too)
+        const size_t nqd = (size_t)d->n_heads * d->hd, mk = (size_t)d->dim > nqd ? (size_t)d->dim : nqd, ctx = (size_t)d->ctx, c64 = (ctx + 63) / 64 * 64;
+        l3m_pfbuf *b = &m->pfb;
+        const size_t vb = m->dtype == L3M_BF16 ? 2 : 1;
+        ok = (b->x = dalloc(m, ctx * d->dim * 4)) && (b->act.q = dalloc(m, c64 * mk * vb)) && (b->act.s = dalloc(m, c64 * mk / 32 * 4)) &&
+             (b->hact.q = dalloc(m, c64 * d->ffn * vb)) && (b->hact.s = dalloc(m, c64 * d->ffn / 32 * 4)) && (b->q = dalloc(m, ctx * nqd * 4)) &&
+             (b->att = dalloc(m, ctx * nqd * 4));
+    }
+    if (ok) return;
+    while (m->n_allocs > mark) l3m_dev_free(m->allocs[--m->n_allocs]);
+    free(m->pf);
+    m->pf = NULL;
+    l3m_dev_clear_error();
+    fprintf(stderr, "l3m: no memory for the prompt matrices: prompts run token by token\n");
+}
+
 // The file row starting at input column c (whole 32-blocks for quantized rows).
 static const void *col_slice(const void *row, int dtype, int c) {
     return (const uint8_t *)row + (dtype >= L3M_Q8_0 ? l3m_file_row_bytes(dtype, c) : (size_t)c * (dtype == L3M_BF16 ? 2 : 4));
@@ -369,14 +393,6 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
     if (d->n_groups > MAX_PARTS || d->n_chunks > MAX_PARTS) return fail(m, "too many head groups or FFN chunks for the GPU kernels");
     l3m_model_layout(d);
     m->layers = calloc((size_t)d->n_layers, sizeof *m->layers);
-    // batched prefill (bf16, q8_0 and q4_0 bodies, and mxfp4 bodies whose blocks widen exactly to q8_0; whole
-    // 32-blocks): unless L3M_PREFILL=0
-    const char *pe_ = getenv("L3M_PREFILL"), *pm_ = getenv("L3M_PREFILL_MIN");
-    const int qb_ = d->dim % 32 == 0 && (d->n_heads * d->hd) % 32 == 0 && d->ffn % 32 == 0;
-    if ((!pe_ || strcmp(pe_, "0")) && !m->reference && !gpt2 && qb_ && l3m_prefill_fits(d->dim, d->ffn, d->n_heads * d->hd, d->hd) &&
-        (m->dtype == L3M_BF16 || m->dtype == L3M_Q8_0 || m->dtype == L3M_Q4_0 || m->mx_wide || (m->dtype == L3M_MXFP4 && mxfp4_body_widens(f, d->n_layers))))
-        m->pf = calloc((size_t)d->n_layers, sizeof *m->pf);
-    m->prefill_min = pm_ ? atoi(pm_) : 8;
     l3m_dgroup *groups = calloc((size_t)d->n_groups, sizeof *groups);
     l3m_dchunk *chunks = calloc((size_t)d->n_chunks, sizeof *chunks);
     int max_rows = d->dim > 2 * chunk + 32 ? d->dim : 2 * chunk + 32;
@@ -472,10 +488,6 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
             free(groups); free(chunks); free(rows);
             return fail(m, "weight upload failed");
         }
-        if (m->pf && upload_prefill(m, f, l, dt, L)) {
-            free(groups); free(chunks); free(rows);
-            return fail(m, "prefill weight upload failed");
-        }
     }
     // The K/V window: every position of the context when it fits in LDS beside the rest of the attention
     // block, else the most positions (a multiple of 32) that fit; a step at a position past it reads K and V
@@ -547,19 +559,6 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
     d->xb = dalloc(m, (size_t)d->dim * 4);
     d->po = dalloc(m, (size_t)d->n_groups * d->dim * 4);
     d->pd = dalloc(m, (size_t)d->n_chunks * d->dim * 4);
-    if (m->pf) {
-        // activations of whole 64-token groups (a GEMM's workgroup reads up to 64 tokens)
-        const size_t nqd = (size_t)d->n_heads * d->hd, mk = (size_t)d->dim > nqd ? (size_t)d->dim : nqd, ctx = (size_t)d->ctx, c64 = (ctx + 63) / 64 * 64;
-        m->pfb.x = dalloc(m, ctx * d->dim * 4);
-        const size_t vb = m->dtype == L3M_BF16 ? 2 : 1;
-        m->pfb.act.q = dalloc(m, c64 * mk * vb);
-        m->pfb.act.s = dalloc(m, c64 * mk / 32 * 4);
-        m->pfb.hact.q = dalloc(m, c64 * d->ffn * vb);
-        m->pfb.hact.s = dalloc(m, c64 * d->ffn / 32 * 4);
-        m->pfb.q = dalloc(m, ctx * nqd * 4);
-        m->pfb.att = dalloc(m, ctx * nqd * 4);
-        if (!m->pfb.x || !m->pfb.act.q || !m->pfb.act.s || !m->pfb.hact.q || !m->pfb.hact.s || !m->pfb.q || !m->pfb.att) return fail(m, "out of device memory");
-    }
     d->logits = dalloc(m, (size_t)NSLOTS * d->vocab * 4);
     // persistent kernel: one workgroup per CU (the LDS request keeps a second one off each CU); the body
     // (head groups, then FFN chunks) on the workgroups of one XCD, every other workgroup on head tiles.
@@ -621,6 +620,15 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
         m->graphs = l3m_graphs_build(d, m->layers);
         if (!m->graphs) return fail(m, "could not capture the decode step");
     }
+    // batched prefill (bf16, q8_0 and q4_0 bodies, and mxfp4 bodies whose blocks widen exactly to q8_0; whole
+    // 32-blocks): unless L3M_PREFILL=0. Last, and only if its memory is there: a model without it feeds prompts
+    // token by token
+    const char *pf_ = getenv("L3M_PREFILL"), *pm_ = getenv("L3M_PREFILL_MIN");
+    const int qb_ = d->dim % 32 == 0 && (d->n_heads * d->hd) % 32 == 0 && d->ffn % 32 == 0;
+    if ((!pf_ || strcmp(pf_, "0")) && !m->reference && !gpt2 && qb_ && l3m_prefill_fits(d->dim, d->ffn, d->n_heads * d->hd, d->hd) &&
+        (m->dtype == L3M_BF16 || m->dtype == L3M_Q8_0 || m->dtype == L3M_Q4_0 || m->mx_wide || (m->dtype == L3M_MXFP4 && mxfp4_body_widens(f, d->n_layers))))
+        add_prefill(m);
+    m->prefill_min = pm_ ? atoi(pm_) : 8;
     const char *base = strrchr(path, '/');
     base = base ? base + 1 : path;
     if (m->reference)
