@@ -1728,6 +1728,8 @@ __device__ void attend_group(const l3m_dmodel &M, const l3m_dgroup &G, int layer
                 q[0] = a.x; q[1] = a.y; q[2] = a.z; q[3] = a.w; q[4] = b.x; q[5] = b.y; q[6] = b.z; q[7] = b.w;
             }
             float m = -INFINITY, l = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            // BATCH: the position whose row is cur's; lanes past the head keep zeros (their zero q times an infinity is NaN)
+            const int own = j < nv ? pos : -1;
             // rounds r = 0, 1, ... cover positions (r * W + wi) * PPW + gl; ATT_IT rounds per chunk
             for (int r0 = 0; (r0 * W + wi) * PPW < n; r0 += ATT_IT) {
                 float s[ATT_IT];
@@ -1747,8 +1749,8 @@ __device__ void attend_group(const l3m_dmodel &M, const l3m_dgroup &G, int layer
                     asm volatile("" ::: "memory");
                     const uint4 kc = kcur[j < nv ? j : 0], vc = vcur[j < nv ? j : 0];
 #pragma unroll
-                    for (int k = 0; k < ATT_IT; k++)  // lanes past the head keep zeros: their zero q times an infinity is NaN
-                        if (((r0 + k) * W + wi) * PPW + gl == pos && j < nv) { kb[k] = kc; vb[k] = vc; }
+                    for (int k = 0; k < ATT_IT; k++)
+                        if (((r0 + k) * W + wi) * PPW + gl == own) { kb[k] = kc; vb[k] = vc; }
                 }
 #pragma unroll
                 for (int k = 0; k < ATT_IT; k++) {
