@@ -2650,10 +2650,10 @@ __host__ __device__ inline LdsAtt lds_att(int mode, int nq, int nkv, int hd, int
 }
 
 // One head group's attention exactly as the decode step runs it (attn_block): MODE 2 attend_mfma, 1
-// attend_group over the LDS window, 0 attend_group reading the cache. q: [nq][hd] f32 (after RoPE);
+// attend_group over the LDS window, 0 attend_group reading the cache (batched or not). q: [nq][hd] f32 (after RoPE);
 // kc, vc: [nkv][ctx][hd] bf16 holding rows 0..pos (row pos is this step's, which the block takes from its
 // own registers into cur and the window); out: [nq][hd]. Query head h reads kv head h / (nq / nkv).
-template <int MODE>
+template <int MODE, bool BATCH>
 __global__ void __launch_bounds__(NTE) k_attend_decode(float *out, const float *q, const uint16_t *kc, const uint16_t *vc, int nq,
                                                        int nkv, int hd, int ctx, int pos, int att_wl) {
     extern __shared__ __align__(16) uint8_t smem[];
@@ -2684,7 +2684,7 @@ __global__ void __launch_bounds__(NTE) k_attend_decode(float *out, const float *
     __syncthreads();
     if (MODE == 2) attend_mfma(M, G, pos, qp, kvb, sc, vred, att);
     else if (MODE == 1) attend_group<true, false, false>(M, G, 0, pos, qh, cur, kvb, vred, att);
-    else attend_group<false, false, true>(M, G, 0, pos, qh, cur, kvb, vred, att);
+    else attend_group<false, false, BATCH>(M, G, 0, pos, qh, cur, kvb, vred, att);
     for (int i = tidx(); i < nqd; i += NTE) out[i] = att[i];
 }
 
@@ -4732,7 +4732,10 @@ int l3m_k_attend_decode(int mode, float *out, const float *q, const uint16_t *kc
     if (lds > g_lds_max) return fail_msg("attend_decode: the K/V window does not fit in LDS");
     int wmax = nq < NWE ? NWE / nq : 1, wl = 0;       // as l3m_group_layout
     while ((2 << wl) <= wmax) wl++;
-    auto k = mode == 2 ? k_attend_decode<2> : mode == 1 ? k_attend_decode<1> : k_attend_decode<0>;
+    // the batched form's byte offsets span every kv head's rows and must lie below OOB; a model's always do (dim up
+    // to 4096, ctx up to 8192: 64 MiB)
+    const bool batch = 2 * (size_t)nkv * ctx * hd < OOB;
+    auto k = mode == 2 ? k_attend_decode<2, false> : mode == 1 ? k_attend_decode<1, false> : batch ? k_attend_decode<0, true> : k_attend_decode<0, false>;
     lds_opt_in(k, (unsigned)lds);
     hipLaunchKernelGGL(k, dim3(1), dim3(NTE), lds, as_stream(stream), out, q, kc, vc, nq, nkv, hd, ctx, pos, wl);
     CKL("k_attend_decode");

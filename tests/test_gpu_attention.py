@@ -72,6 +72,25 @@ def test_decode_attention_infinite_score(dev, oracle, case):
         dev.free_all()
 
 
+@pytest.mark.parametrize("hd", [48, 64, 256])
+def test_decode_attention_cache_of_gigabytes(dev, oracle, hd):
+    """Mode 0 over K and V of 3 GiB each, past what the batched form's byte offsets reach (the form of bf16 and f32
+    bodies reads them): the last kv head's rows begin at 2 GiB."""
+    nkv, ctx = 3, (1 << 29) // hd
+    bufs = [dev.alloc(2 * nkv * ctx * hd) for _ in range(2)]
+    for pos in (0, 40, 600):
+        print(f"cache of gigabytes, hd {hd} pos {pos}", flush=True)
+        q, kc, vc = inputs(3 * hd + pos, nkv, nkv, hd, pos + 1, 1.0)
+        for b, rows in zip(bufs, (kc, vc)):
+            for h in range(nkv):
+                assert dev.lib.l3m_dev_upload(b + 2 * h * ctx * hd, rows[h].ctypes.data, rows[h].nbytes) == 0
+        out = dev.alloc(4 * nkv * hd)
+        assert dev.lib.l3m_k_attend_decode(0, out, dev.put(q), bufs[0], bufs[1], nkv, nkv, hd, ctx, pos, None) == 0
+        got = dev.get(out, nkv * hd, np.float32).reshape(nkv, hd)
+        assert np.abs(got - want(oracle, q, kc, vc, nkv, nkv, hd, pos)).max() <= 1e-5, pos
+    dev.free_all()
+
+
 def test_attention_modes_agree_with_decode_choice(dev):
     """The mode a decode step picks (l3m_attention_mode) for the benchmark shapes: matrix cores for hd 64
     and 48 with the window in LDS, the VALU window form for a head dimension off the multiples of 16, the

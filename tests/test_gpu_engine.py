@@ -371,8 +371,9 @@ def test_context_off_the_multiples_of_32(models, oracle, monkeypatch, dtype, ctx
     np.testing.assert_array_equal(out["0"][1], out["1"][1])
 
 
-@pytest.mark.parametrize("cfg,ctx,n_new", [(A.CONFIGS["stories42M"], 1024, 600), (dataclasses.replace(SMALL, name="tiny2k", ctx=2048), 2048, 1500)],
-                         ids=["stories42M-ctx1024", "tiny-ctx2048"])
+@pytest.mark.parametrize("cfg,ctx,n_new", [(A.CONFIGS["stories42M"], 1024, 600), (dataclasses.replace(SMALL, name="tiny2k", ctx=2048), 2048, 1500),
+                                           (dataclasses.replace(SMALL, name="tiny2kb", ctx=2048, dtype="bf16"), 2048, 1500)],
+                         ids=["stories42M-ctx1024", "tiny-ctx2048", "tiny-bf16-ctx2048"])
 def test_long_context_follows_oracle(models, oracle, cfg, ctx, n_new):
     """Decoding far past the positions whose K/V window fits in LDS (the steps before the window's end attend
     over it, those past it read the cache, in one generate call): every step
@@ -393,7 +394,11 @@ def test_long_context_follows_oracle(models, oracle, cfg, ctx, n_new):
     for pos in range(len(ids) - 1 + n_new - 60, len(ids) - 1 + n_new, 7):   # logits kept for the last 128 positions
         lg, lo = m.logits_at(pos), logits[pos - (len(ids) - 1)]
         assert int(np.argmax(lg)) == int(np.argmax(lo)) or steps[pos - (len(ids) - 1)][2] < NEAR_TIE
-        assert kl(lo, lg) < 0.01 and np.abs(lg - lo).max() <= SPREAD[cfg.dtype] * np.abs(lo).max(), pos
+        # bf16: one activation of this lively 128-wide model rounded the other way (2^-8 of it) in each of the 14 matrices
+        # and the head's input moves a logit by up to about sqrt(15 / 128) 2^-8 of the largest = 1.3e-3 per flip and
+        # row: SHAPE_BAR, not the golden models' SPREAD
+        bar = SHAPE_BAR["bf16"] if cfg.dtype == "bf16" else SPREAD[cfg.dtype]
+        assert kl(lo, lg) < 0.01 and np.abs(lg - lo).max() <= bar * np.abs(lo).max(), pos
     m.close()
 
 
