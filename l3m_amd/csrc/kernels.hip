@@ -188,6 +188,7 @@ __device__ float4 lt_elem4(const l3m_dmat &m, int r, int i) {
 template <int N> __device__ __forceinline__ float lanes_sum(float v);   // cross-lane sums, below
 template <int N> __device__ __forceinline__ float lanes_max(float v);
 template <int N> __device__ __forceinline__ int lanes_sumi(int v);
+template <int N> __device__ __forceinline__ int lanes_mini(int v);
 
 // (value, index) maximum; ties and NaN go to the lower index, as the reference's strict '>' scan
 // (engine.c:294, 300).
@@ -809,11 +810,13 @@ __global__ void __launch_bounds__(NT) k_silu_mul(float *h, const float *g, int n
     if (i < n) h[i] = silu_mul(h[i], g[i]);
 }
 
-// The first maximum of x (engine.c:290-301): one workgroup, a thread ARG_U x 4 values a round with every load first
-// (16 bytes from the first aligned address on). 49152 values: 6.0 us, 62.5
-// with 256 threads of dependent 4-byte loads.
-constexpr int ARG_U = 12;
-__global__ void __launch_bounds__(1024) k_argmax(const float *x, int n, int32_t *out) {
+// The first maximum of x (engine.c:290-301): one workgroup of nt threads, each U x 4 values a round with every load
+// first (16 bytes from the first aligned address on). Bound by latency: U = 1 holds one quad a thread, up to 4096
+// values; past that 1024 threads and U = 12, and the quad with the largest value is read again for its place. Queued
+// back to back, 1000 values 3.5 us (4.7 with 1024 threads of U = 12, 3.5 with 256 threads of 4-byte loads), 4096
+// 3.5 (4.9, 5.0), 49152 3.8 (5.1, 35.2).
+template <int U>
+__global__ void __launch_bounds__(1024) k_argmax(const float *x, int n, int nt, int32_t *out) {
     __shared__ float sv[16];
     __shared__ int si[16];
     const int t = threadIdx.x, head = min((int)((16 - ((uintptr_t)x & 15)) & 15) >> 2, n), nq = (n - head) >> 2, tail = head + 4 * nq;
@@ -823,43 +826,48 @@ __global__ void __launch_bounds__(1024) k_argmax(const float *x, int n, int32_t 
     auto take = [&](float a, int i) {
         if (a > v || (a == v && i < idx)) { v = a; idx = i; }
     };
+    auto take4 = [&](float4 a, int i) {
+        take(a.x, i); take(a.y, i + 1); take(a.z, i + 2); take(a.w, i + 3);
+    };
     if (t < head) take(x[t], t);
-    // the thread's first quad with the largest value, then that value's place in it
     const float4 *xq = (const float4 *)(x + head);
-    float vq = -INFINITY;
-    int best = -1;
-    for (int q0 = 0; q0 < nq; q0 += ARG_U * 1024) {
-        float4 a[ARG_U];
+    if constexpr (U == 1) {
+        if (t < nq) take4(xq[t], head + 4 * t);
+    } else {
+        // the thread's first quad with the largest value, then that value's place in it
+        float vq = -INFINITY;
+        int best = -1;
+        for (int q0 = 0; q0 < nq; q0 += U * 1024) {
+            float4 a[U];
 #pragma unroll
-        for (int u = 0; u < ARG_U; u++) a[u] = xq[min(q0 + u * 1024 + t, nq - 1)];   // past the end: the last again
+            for (int u = 0; u < U; u++) a[u] = xq[min(q0 + u * 1024 + t, nq - 1)];   // past the end: the last again
 #pragma unroll
-        for (int u = 0; u < ARG_U; u++) {
-            const float m = fmaxf(fmaxf(a[u].x, a[u].y), fmaxf(a[u].z, a[u].w));
-            if (m > vq) { vq = m; best = min(q0 + u * 1024 + t, nq - 1); }
+            for (int u = 0; u < U; u++) {
+                const float m = fmaxf(fmaxf(a[u].x, a[u].y), fmaxf(a[u].z, a[u].w));
+                if (m > vq) { vq = m; best = min(q0 + u * 1024 + t, nq - 1); }
+            }
         }
-    }
-    if (best >= 0) {
-        const float4 a = xq[best];
-        take(vq, head + 4 * best + (a.x == vq ? 0 : a.y == vq ? 1 : a.z == vq ? 2 : 3));
-    } else {                                          // nothing above -infinity: the first of those
-        for (int q = t; q < nq; q += 1024) {
-            const float4 a = xq[q];
-            const int i = head + 4 * q;
-            take(a.x, i); take(a.y, i + 1); take(a.z, i + 2); take(a.w, i + 3);
+        if (best >= 0) {
+            const float4 a = xq[best];
+            take(vq, head + 4 * best + (a.x == vq ? 0 : a.y == vq ? 1 : a.z == vq ? 2 : 3));
+        } else {                                      // nothing above -infinity: the first of those
+            for (int q = t; q < nq; q += 1024) take4(xq[q], head + 4 * q);
         }
     }
     if (t < n - tail) take(x[tail + t], tail + t);
-    for (int o = 32; o; o >>= 1) {
-        const float v2 = __shfl_xor(v, o);
-        const int i2 = __shfl_xor(idx, o);
-        take(v2, i2);
+    // a wavefront's largest, then the lowest index that holds it; then the wavefronts' by the first of them
+    float m = lanes_max<64>(v);
+    int i = lanes_mini<64>(v == m ? idx : 0x7FFFFFFF);
+    const int waves = nt >> 6;
+    if (waves > 1) {
+        if ((t & 63) == 0) { sv[t >> 6] = m; si[t >> 6] = i; }
+        __syncthreads();
+        if (t >= 64) return;
+        v = t < waves ? sv[t] : -INFINITY;
+        m = lanes_max<64>(v);
+        i = lanes_mini<64>(t < waves && v == m ? si[t] : 0x7FFFFFFF);
     }
-    if ((t & 63) == 0) { sv[t >> 6] = v; si[t >> 6] = idx; }
-    __syncthreads();
-    if (t == 0) {
-        for (int k = 1; k < 16; k++) take(sv[k], si[k]);
-        *out = idx == 0x7FFFFFFF ? 0 : idx;
-    }
+    if (t == 0) *out = i == 0x7FFFFFFF ? 0 : i;
 }
 
 // ------------------------------------------------------------------------------ decode step kernels
@@ -4743,7 +4751,9 @@ int l3m_k_attend_decode(int mode, float *out, const float *q, const uint16_t *kc
 }
 
 int l3m_k_argmax(const float *x, int n, int32_t *out, void *stream) {
-    hipLaunchKernelGGL(k_argmax, dim3(1), dim3(1024), 0, as_stream(stream), x, n, out);
+    const int nt = min(max((n / 4 + 63) & ~63, 64), 1024);   // n / 4 quads at most, whatever x's alignment
+    if (n <= 4096) hipLaunchKernelGGL(k_argmax<1>, dim3(1), dim3(nt), 0, as_stream(stream), x, n, nt, out);
+    else hipLaunchKernelGGL(k_argmax<12>, dim3(1), dim3(1024), 0, as_stream(stream), x, n, 1024, out);
     CKL("k_argmax");
     return 0;
 }

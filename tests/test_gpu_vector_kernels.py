@@ -19,7 +19,7 @@ def argmax_at(dev, x, off):
 
 
 @pytest.mark.parametrize("off", [0, 1, 2, 3])
-@pytest.mark.parametrize("n", [1, 2, 3, 5, 63, 4099, 24576, 24579, 50257, 131075])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 63, 255, 256, 259, 1000, 1027, 4093, 4096, 4097, 4099, 24576, 24579, 50257, 131075])
 def test_argmax_edges(dev, n, off):
     rng = np.random.default_rng(n + off)
     x = rng.standard_normal(n).astype(np.float32)
