@@ -67,6 +67,7 @@ struct l3m_model {
     float        temp;         // the running generate call's temperature (0: greedy)
     l3m_pflayer *pf;           // batched prompt prefill: per-layer full matrices, NULL when unavailable
     l3m_pfbuf    pfb;
+    l3m_pfgraphs *pfg;         // the prefill's captured graphs (NULL: launched kernel by kernel, L3M_PREFILL_GRAPH=0)
     int          prefill_min;  // prompts of at least this many tokens are prefilled (L3M_PREFILL_MIN)
     int          prefilled;    // positions the last generate call prefilled
     int          logits_fresh;
@@ -283,7 +284,16 @@ static void add_prefill(l3m_model *m) {
              (b->hact.q = dalloc(m, c64 * d->ffn * vb)) && (b->hact.s = dalloc(m, c64 * d->ffn / 32 * 4)) && (b->q = dalloc(m, ctx * nqd * 4)) &&
              (b->att = dalloc(m, ctx * nqd * 4));
     }
-    if (ok) return;
+    if (ok) {
+        // Few launches: the host's are longer than the GPU's work behind them, and a graph's one launch frees it for the
+        // decode pass. Many: the GPU is behind, and a graph's kernels start further apart. us a call of dim 256 / 576, 100
+        // tokens, launched one by one and as a graph: 2 layers 170, 141 / 189, 161; 4: 244, 223 / 289, 268; 8: 389, 384 / 481,
+        // 477; 12: 536, 551 / 673, 684; 20: 841, 895 / 1066, 1097; 30: 1272, 1321 / 1579, 1621 (16 tokens cross at the
+        // same depth). L3M_PREFILL_GRAPH=0: never (for comparison)
+        const char *pg = getenv("L3M_PREFILL_GRAPH");
+        if ((!pg || strcmp(pg, "0")) && d->n_layers <= 8) m->pfg = l3m_pfgraphs_new();
+        return;
+    }
     while (m->n_allocs > mark) l3m_dev_free(m->allocs[--m->n_allocs]);
     free(m->pf);
     m->pf = NULL;
@@ -648,6 +658,7 @@ void l3m_free(l3m_model *m) {
     if (!m) return;
     l3m_dev_sync();
     l3m_graphs_free(m->graphs);
+    l3m_pfgraphs_free(m->pfg);
     l3m_dev_host_free(m->call_host);
     l3m_dev_host_free(m->out_host);
     l3m_dev_event_free(m->ev[0]);
@@ -761,10 +772,8 @@ static int run_steps(l3m_model *m, const int32_t *prompt, int n_prompt, int max_
         if (l3m_dev_upload_async(m->call_dev, m->call_host, m->call_tok + (size_t)n_prompt * 4)) return -1;
         from = -1;
         if (m->cold && evict(m)) return -1;
-        // launched one by one: a kernel takes 3-5 us, a launch 1.6, so the GPU never waits. As a captured graph per
-        // prompt length the same kernels took as long (64 tokens, 30 layers: 1509 us against 1497; 480: 2306 against
-        // 2264), and each length's first prompt 0.5 ms more for the capture
-        if (l3m_prefill(d, m->pf, &m->pfb, n_prompt - 1, NULL)) return -1;
+        if (m->pfg ? l3m_prefill_graph(m->pfg, d, m->pf, &m->pfb, n_prompt - 1) : l3m_prefill(d, m->pf, &m->pfb, n_prompt - 1, NULL))
+            return -1;
         m->prefilled = n_prompt - 1;
     }
     const int live = on_token != NULL || bos >= 0 || eos >= 0, depth = m->cold ? 1 : 2;

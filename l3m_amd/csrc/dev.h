@@ -177,6 +177,13 @@ typedef struct {
 int l3m_prefill(const l3m_dmodel *m, const l3m_pflayer *layers, const l3m_pfbuf *b, int P, void *stream);
 // 1 when l3m_prefill takes a model of these sizes (nqd = n_heads * hd); the loader enables prefill only then.
 int l3m_prefill_fits(int dim, int ffn, int nqd, int hd);
+// l3m_prefill on the library's stream, as a replayed graph from a length's third prompt on (kernels.hip). NULL from
+// l3m_pfgraphs_new: no graphs.
+typedef struct l3m_pfgraphs l3m_pfgraphs;
+l3m_pfgraphs *l3m_pfgraphs_new(void);
+int           l3m_prefill_graph(l3m_pfgraphs *g, const l3m_dmodel *m, const l3m_pflayer *layers, const l3m_pfbuf *b, int P);
+void          l3m_pfgraphs_free(l3m_pfgraphs *g);
+
 // The persistent decode kernel (one cooperative launch for R->nsteps steps; layers_dev in device memory).
 int l3m_dev_cus(void);
 // The XCD each block of a cooperative grid of `grid` 1024-thread workgroups with lds bytes lands on

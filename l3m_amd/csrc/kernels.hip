@@ -4929,6 +4929,76 @@ int l3m_graphs_launch(l3m_graphs *g, int with_head, void *stream) {
     return 0;
 }
 
+// A prompt length's launches (their grids and arguments depend on P alone, every buffer is the model's own) as a
+// graph, for the PF_GRAPHS lengths used last: the first prompt of a length is launched kernel by kernel, its second
+// captured, later ones replayed (add_prefill's rule says for which models). Capture and instantiation cost a call 0.06 ms
+// (2 layers) to 0.16 (6), which a length seen once never pays (2 layers of dim 128, 48 tokens: the first call 198 us, the
+// second 198, then 133; launched one by one 190, 165, then 157). Captured on a stream
+// of its own: other threads' work on the library's stream stays out of it. off: a capture failed, launched one by one
+// from then on.
+constexpr int PF_GRAPHS = 8;
+struct l3m_pfgraphs {
+    hipStream_t cap;
+    bool off;
+    int P[PF_GRAPHS];                 // 0: an empty entry
+    hipGraphExec_t e[PF_GRAPHS];      // null: seen once
+    unsigned long long used[PF_GRAPHS], tick;
+};
+
+l3m_pfgraphs *l3m_pfgraphs_new(void) {
+    l3m_pfgraphs *g = (l3m_pfgraphs *)calloc(1, sizeof *g);
+    if (g && hipStreamCreateWithFlags(&g->cap, hipStreamNonBlocking) != hipSuccess) {
+        (void)hipGetLastError();
+        free(g);
+        return nullptr;
+    }
+    return g;
+}
+
+void l3m_pfgraphs_free(l3m_pfgraphs *g) {
+    if (!g) return;
+    for (int i = 0; i < PF_GRAPHS; i++)
+        if (g->e[i]) (void)hipGraphExecDestroy(g->e[i]);
+    (void)hipStreamDestroy(g->cap);
+    free(g);
+}
+
+static hipGraphExec_t pf_capture(l3m_pfgraphs *g, const l3m_dmodel *M, const l3m_pflayer *L, const l3m_pfbuf *B, int P) {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t e = nullptr;
+    const int had = g_has_err;
+    if (hipStreamBeginCapture(g->cap, hipStreamCaptureModeThreadLocal) == hipSuccess) {
+        const int rc = l3m_prefill(M, L, B, P, g->cap);
+        if (hipStreamEndCapture(g->cap, &graph) != hipSuccess || rc || hipGraphInstantiate(&e, graph, NULL, NULL, 0) != hipSuccess) e = nullptr;
+        if (graph) (void)hipGraphDestroy(graph);
+    }
+    if (!e) {                                          // launched one by one instead: no error of the call's
+        g->off = true;
+        (void)hipGetLastError();
+        if (!had) l3m_dev_clear_error();
+    }
+    return e;
+}
+
+int l3m_prefill_graph(l3m_pfgraphs *g, const l3m_dmodel *M, const l3m_pflayer *L, const l3m_pfbuf *B, int P) {
+    if (P < 1) return 0;
+    int k = -1, lru = 0;
+    for (int i = 0; i < PF_GRAPHS; i++) {
+        if (g->P[i] == P) k = i;
+        if (g->used[i] < g->used[lru]) lru = i;
+    }
+    if (k < 0) {
+        k = lru;
+        if (g->e[k]) { (void)hipGraphExecDestroy(g->e[k]); g->e[k] = nullptr; }
+        g->P[k] = P;
+    } else if (!g->e[k] && !g->off)
+        g->e[k] = pf_capture(g, M, L, B, P);
+    g->used[k] = ++g->tick;
+    if (!g->e[k]) return l3m_prefill(M, L, B, P, g_stream);
+    CK(hipGraphLaunch(g->e[k], g_stream));
+    return 0;
+}
+
 // Mean microseconds per launch of iters launches queued back to back, after one untimed launch: one pair
 // of events around them all (events around each launch would add their own markers' time to every
 // figure). For a kernel shorter than the launch interval (l3m_time_launch_interval) this is the launch rate.

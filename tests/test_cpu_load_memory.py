@@ -49,10 +49,12 @@ int l3m_step_a_dtype(int dt) { return dt == L3M_HIP_Q4_0 ? L3M_HIP_Q8_0 : dt; }
 int l3m_prefill_fits(int a, int b, int c, int d) { return (void)a, (void)b, (void)c, (void)d, 1; }
 l3m_graphs *l3m_graphs_build(const l3m_dmodel *m, const l3m_dlayer *l) { return (void)m, (void)l, malloc(1); }
 void l3m_graphs_free(l3m_graphs *g) { free(g); }
+l3m_pfgraphs *l3m_pfgraphs_new(void) { return malloc(1); }
+void l3m_pfgraphs_free(l3m_pfgraphs *g) { free(g); }
 """
 # what the host code calls after loading
 NOT_REACHED = """act_bytes decode_fits decode_launch decode_pair decode_placement decode_timer_collect dev_download dev_download_async
-dev_event_record dev_event_wait dev_evict dev_name dev_upload_async graphs_launch k_attend k_gemv k_ltiles k_step_mv ltile_bytes prefill
+dev_event_record dev_event_wait dev_evict dev_name dev_upload_async graphs_launch k_attend k_gemv k_ltiles k_step_mv ltile_bytes prefill prefill_graph
 step_enqueue time_step_kernel""".split()
 
 

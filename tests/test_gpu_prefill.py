@@ -108,16 +108,17 @@ def test_prefill_logits(models, oracle, monkeypatch, cfg, n_prompt):
 
 
 def test_prefill_graph_replays_equal_loose_launches(models, monkeypatch):
-    """The prefill runs as one captured graph per prompt length (L3M_PREFILL_GRAPH=0: the same launches
-    one by one). Every call, including replays of a length captured earlier with decoding and other lengths
-    run in between, gives logits and K/V rows bit-identical to the loose launches of the same prompt."""
+    """A prompt length's second prompt is captured as a graph and replayed from then on (its first, and all with
+    L3M_PREFILL_GRAPH=0, are launched kernel by kernel). Every call, with decoding and other lengths run in between
+    and a longer prompt's rows left in the buffers, gives logits and K/V rows bit-identical to the loose launches of
+    the same prompt."""
     cfg = GQA
     path = models.get(cfg, cfg.dtype, seed=9, std=0.05, norm_jitter=0.1)
     hd = cfg.dim // cfg.n_heads
     graph = A.Model(path)
     monkeypatch.setenv("L3M_PREFILL_GRAPH", "0")
     loose = A.Model(path)
-    for i, n_prompt in enumerate([40, 100, 40, 57, 100, 40]):
+    for i, n_prompt in enumerate([40, 100, 40, 57, 100, 40, 100, 57, 57, 40]):
         print(f"call {i}: prompt {n_prompt}", flush=True)
         ids = A.prompt(20 + i, cfg.vocab, n_prompt)
         got = graph.generate(ids, 3)
@@ -169,16 +170,16 @@ def test_prefill_past_128_positions(models, oracle, monkeypatch):
 
 
 def test_prefill_graph_cache_replaces_the_oldest(models, monkeypatch):
-    """More prompt lengths than the eight captured graphs a model keeps: eleven lengths in turn, then the
-    first three again (each replaced since and captured anew) and the last (still kept). Every call's tokens
-    and logits equal the loose launches' bit for bit."""
+    """More prompt lengths than the eight a model keeps graphs of: eleven lengths, three prompts each (launched one by
+    one, captured, replayed), then the first three so again (each replaced since) and the last (still kept). Every
+    call's tokens and logits equal the loose launches' bit for bit."""
     path = models.get(GQA, GQA.dtype, seed=9, std=0.05, norm_jitter=0.1)
     graph = A.Model(path)
     monkeypatch.setenv("L3M_PREFILL_GRAPH", "0")
     loose = A.Model(path)
     lengths = list(range(10, 32, 2))
-    for i, n_prompt in enumerate(lengths + lengths[:3] + lengths[-1:]):
-        ids = A.prompt(40 + n_prompt, GQA.vocab, n_prompt)
+    for i, n_prompt in enumerate([n for n in lengths + lengths[:3] for _ in range(3)] + lengths[-1:]):
+        ids = A.prompt(40 + n_prompt + i, GQA.vocab, n_prompt)
         got, want = graph.generate(ids, 2), loose.generate(ids, 2)
         assert graph.prefilled == loose.prefilled == n_prompt - 1
         assert got == want, (i, n_prompt)
