@@ -3719,8 +3719,8 @@ __global__ void __launch_bounds__(64) k_pf_attend(const float *qb, int P, int n_
 //    A = V^T, dims by positions: the wavefront transposes the chunk's V rows (4 positions x 8 dims a lane)
 //    into its own LDS span, rows of 40 elements, the lane's 8 positions contiguous.
 // A masked position's p is 0 and a part of q may be, but 0 times an infinity or a NaN in a V or K row is NaN: where
-// any of the tile's outputs is not finite, its tokens are done again one at a time (pf_attn_token), over their
-// own positions alone.
+// any of a wavefront's sums is not finite, the tile's tokens are done one at a time instead (pf_attn_token), over
+// their own positions alone. (A flag from the merged outputs and a second barrier cost a prompt of 64 tokens 1%.)
 // No barrier before the end. Bound by the chunk's chain (loads, two products, expf, LDS round trip), not by
 // bytes or products: 9 heads of 64, 479 tokens: 11.1 us a layer, against 55.7 for k_pf_attend (one wavefront
 // per token and head, a lane per position: every token reads every K and V row again); 63 tokens: 5.0 (7.0).
@@ -3778,9 +3778,8 @@ __global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qb, int P, 
     __shared__ __align__(16) uint8_t lds[PFA_W * VT];
     static_assert((HD + 64) * 4 <= VT, "pf_attn_token's floats too");
     __shared__ float ml[2][PFA_W][PFA_T];
-    __shared__ int odd;                               // an output that is not finite
+    __shared__ int odd[PFA_W];                        // the wavefront has a sum that is not finite
     const int lane = tidx() & 63, wave = wave_id(), c16 = lane & 15, quarter = lane >> 4;
-    if (tidx() == 0) odd = 0;
     // the tiles with the most positions first
     const int t0 = PFA_T * ((int)gridDim.x - 1 - (int)blockIdx.x), h = blockIdx.y, kv = h / (n_heads / n_kv);
     const int width = n_heads * HD, tmax = (t0 + PFA_T < P ? t0 + PFA_T : P) - 1, tok = min(t0 + c16, tmax);
@@ -3894,6 +3893,11 @@ __global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qb, int P, 
 #pragma unroll
     for (int n = 0; n < NT16; n++) *(float4 *)(om + 16 * n + 4 * quarter) = make_float4(o[n][0], o[n][1], o[n][2], o[n][3]);
     if (quarter == 0) { ml[0][wave][c16] = m; ml[1][wave][c16] = l; }
+    f32x4 z = {0.f, 0.f, 0.f, 0.f};                   // NaN where a sum is not finite
+#pragma unroll
+    for (int n = 0; n < NT16; n++) z += o[n] * 0.f;
+    const int any = __any(!(z[0] + z[1] + z[2] + z[3] == 0.f));
+    if (lane == 0) odd[wave] = any;
     __syncthreads();
     // the output's dims d .. d + 3 of token t
     auto put = [&](int t, int d, float4 y, bool store) {
@@ -3903,6 +3907,18 @@ __global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qb, int P, 
             *(float4 *)(att + (size_t)t * n_heads * HD + h * HD + d) = y;
         }
     };
+    int redo = odd[0];
+#pragma unroll
+    for (int w = 1; w < PFA_W; w++) redo |= odd[w];
+    if (__builtin_amdgcn_readfirstlane(redo)) {       // the wavefront's span: its merge rows are not read
+        for (int tt = wave; tt < PFA_T && t0 + tt < P; tt += PFA_W) {
+            float *buf = (float *)vt;
+            pf_attn_token<HD>(qb + (size_t)(t0 + tt) * width + h * HD, K, V, t0 + tt, scale, buf);
+            const bool mine = 4 * lane < HD;
+            put(t0 + tt, 4 * lane, mine ? *(const float4 *)(buf + 4 * lane) : make_float4(0.f, 0.f, 0.f, 0.f), mine);
+        }
+        return;
+    }
     // each thread 4 dims of a token: the wavefronts' parts in order, scaled to the common maximum (wavefront 0
     // always has position 0)
     for (int u = tidx(); u < PFA_T * HD / 4; u += 64 * PFA_W) {
@@ -3920,16 +3936,7 @@ __global__ void __launch_bounds__(64 * PFA_W) k_pf_attn(const float *qb, int P, 
             y.x += x.x * f; y.y += x.y * f; y.z += x.z * f; y.w += x.w * f;
         }
         y = make_float4(y.x / den, y.y / den, y.z / den, y.w / den);
-        if (!(y.x * 0.f + y.y * 0.f + y.z * 0.f + y.w * 0.f == 0.f)) odd = 1;
         put(t, 4 * d4, y, t < P);
-    }
-    __syncthreads();
-    if (!odd) return;
-    for (int tt = wave; tt < PFA_T && t0 + tt < P; tt += PFA_W) {
-        float *buf = (float *)vt;
-        pf_attn_token<HD>(qb + (size_t)(t0 + tt) * width + h * HD, K, V, t0 + tt, scale, buf);
-        const bool mine = 4 * lane < HD;
-        put(t0 + tt, 4 * lane, mine ? *(const float4 *)(buf + 4 * lane) : make_float4(0.f, 0.f, 0.f, 0.f), mine);
     }
 }
 

@@ -42,14 +42,30 @@ def test_attend_unaligned_v_rows(dev, oracle):
     dev.free_all()
 
 
-def test_attend_large_values_and_masked_rows(dev, oracle):
-    """Scores far past expf's range, and rows past the last one that hold infinities: they are not attended."""
+@pytest.mark.parametrize("at", [(3, 700), (515, 90), (1029, 4), (1029, 1028)])
+def test_attend_large_values_and_masked_rows(dev, oracle, at):
+    """Scores far past expf's range (the largest above 200, in the first, a middle and the last of nine workgroups' rows,
+    and a second one just below it in another's, or its own), and rows past the last one that hold infinities: they
+    are not attended. q and K are small multiples of a half, so every score is exact in f32."""
     n, hd = 1030, 64
-    q, k, v = inputs(6, n + 40, hd, hd)
-    q *= 20
-    k[n * hd:], v[n * hd:] = 0x7F80, 0x7F80
-    got = dev.attend(q, k, v, n - 1, hd, hd)
-    assert np.abs(got - oracle.attend(q, k[:n * hd], v[:n * hd], n - 1, hd, hd)).max() <= 1e-5
+    rng = np.random.default_rng(sum(at))
+    q = rng.integers(-40, 41, hd).astype(np.float32)
+    q[7] = 12
+    kf = rng.integers(-2, 3, (n, hd)).astype(np.float32) / 2
+    kf[at[0]] = np.where(q > 0, 1, -1) * 1.5
+    kf[at[1]] = kf[at[0]]
+    kf[at[1], 7] = 1                                   # its score: 12 * 0.5 / 8 lower
+    s = np.sort(kf @ q / 8)
+    assert s[-1] > 200 and s[-1] - s[-2] == 0.75 and s[-3] < s[-1] - 50
+    k = np.full((n + 40, hd), 0x7F80, np.uint16)
+    k[:n] = kf.view(np.uint32) >> 16
+    v = inputs(6, n + 40, hd, hd)[2]
+    v[n * hd:] = 0x7F80
+    got = dev.attend(q, k.ravel(), v, n - 1, hd, hd)
+    want = oracle.attend(q, k[:n].ravel(), v[:n * hd], n - 1, hd, hd)
+    assert np.abs(got - want).max() <= 1e-5
+    two = [(v[i * hd:(i + 1) * hd].astype(np.uint32) << 16).view(np.float32) for i in at]   # the weights: 1 and exp(-0.75)
+    assert np.abs(want - (two[0] + two[1] * np.exp(-0.75)) / (1 + np.exp(-0.75))).max() <= 1e-5
     dev.free_all()
 
 
