@@ -380,27 +380,14 @@ __device__ __forceinline__ float lane_dot(const l3m_dmat &m, int tile, int b0, i
     return acc;
 }
 
-// LDS carve-up shared by the matvec kernels.
-struct Smem {
-    uint8_t *act;
-    float *xs, *red, *yv, *scr;
-    int *iscr;
-};
-__device__ Smem carve(uint8_t *base, int dt, int k) {
-    Smem s;
-    const int kp = kpad(k);
-    s.act = base;
-    s.xs = (float *)(base + align16(act_size(dt, k)));
-    s.red = s.xs + kp;
-    s.yv = s.red + 64;
-    s.scr = s.yv + 64;
-    s.iscr = (int *)(s.scr + 8);
-    return s;
-}
 // 16-byte words of the activation each k_gemv thread holds in registers while its first weights load
 constexpr int GEMV_ACT_REGS = 4;
-inline size_t smem_bytes(int dt, int k) { return align16(act_size(dt, k)) + 4 * (size_t)kpad(k) + 4 * (64 + 64 + 16); }
+// k_gemv's LDS: the prepared activation, then the wavefronts' sums (16 rows each).
+__host__ __device__ inline size_t gemv_lds(int dt, int k) { return align16(act_size(dt, k)) + 4 * 64; }
 constexpr size_t LDS_MAX = 65536;   // dynamic LDS per workgroup without opting in to more
+// The inputs l3m_k_prep and l3m_k_gemv take: rows whose prepared form and f32 values fit LDS_MAX together (what one
+// workgroup staging both holds; callers size by it, and k_gemv's own LDS is always less).
+inline bool act_fits(int dt, int k) { return align16(act_size(dt, k)) + 4 * (size_t)kpad(k) + 576 <= LDS_MAX; }
 
 int pick_split(int nb) { return nb >= 16 ? 4 : nb >= 8 ? 2 : 1; }
 
@@ -559,7 +546,8 @@ __global__ void __launch_bounds__(NT) k_ltiles(const uint8_t *__restrict__ src, 
 template <int DT, bool STAGED>
 __global__ void __launch_bounds__(NT) k_gemv(l3m_dmat m, const uint8_t *__restrict__ act_g, int k, float *__restrict__ y, int S) {
     extern __shared__ __align__(16) uint8_t smem[];
-    Smem s = carve(smem, DT, k);
+    uint8_t *act = smem;
+    float *red = (float *)(smem + align16(act_size(DT, k)));
     const int kp = kpad(k), tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     // the workgroup's 4/S tiles from tile0, each split over S wavefronts along the inputs
     const int tpw = 4 / S, tile0 = blockIdx.x * tpw, tile = tile0 + wave / S, split = wave % S;
@@ -582,23 +570,23 @@ __global__ void __launch_bounds__(NT) k_gemv(l3m_dmat m, const uint8_t *__restri
         lane_load<DT>(m, ltile, b0 + (lane >> 4), b1, lane, x);
         // clamped slots are written by several threads, with the same value
 #pragma unroll
-        for (int r = 0; r < GEMV_ACT_REGS; r++) ((u32x4 *)s.act)[min(tid + r * NT, n16 - 1)] = a[r];
-        ((uint32_t *)s.act)[4 * n16 - 1 + min(tid + 1, ntail)] = at;
+        for (int r = 0; r < GEMV_ACT_REGS; r++) ((u32x4 *)act)[min(tid + r * NT, n16 - 1)] = a[r];
+        ((uint32_t *)act)[4 * n16 - 1 + min(tid + 1, ntail)] = at;
     } else {
-        for (size_t i = tid; i < bytes / 4; i += NT) ((uint32_t *)s.act)[i] = ((const uint32_t *)act_g)[i];
+        for (size_t i = tid; i < bytes / 4; i += NT) ((uint32_t *)act)[i] = ((const uint32_t *)act_g)[i];
         lane_load<DT>(m, ltile, b0 + (lane >> 4), b1, lane, x);
     }
     __syncthreads();
-    float acc = lane_dot<DT>(m, ltile, b0, b1, s.act, kp, lane, x);
+    float acc = lane_dot<DT>(m, ltile, b0, b1, act, kp, lane, x);
     if (!live) acc = 0.f;
     acc += __shfl_xor(acc, 16);
     acc += __shfl_xor(acc, 32);
-    if (lane < 16) s.red[wave * 16 + lane] = acc;
+    if (lane < 16) red[wave * 16 + lane] = acc;
     __syncthreads();
     if (tid < tpw * 16) {
         const int tt = tid >> 4, r = tid & 15, row = (tile0 + tt) * RT + r;
-        float v = s.red[(tt * S) * 16 + r];
-        for (int sp = 1; sp < S; sp++) v += s.red[(tt * S + sp) * 16 + r];
+        float v = red[(tt * S) * 16 + r];
+        for (int sp = 1; sp < S; sp++) v += red[(tt * S + sp) * 16 + r];
         if (row < m.rows) y[row] = v;
     }
 }
@@ -4174,8 +4162,8 @@ template <int DT> void launch_gemv(const l3m_dmat &m, const void *act, int k, fl
     const int grid = (m.tiles + 4 / S - 1) / (4 / S);
     const size_t n16 = act_size(DT, k) / 16;
     const bool staged = n16 > 0 && n16 <= (size_t)GEMV_ACT_REGS * NT && ((uintptr_t)act & 15) == 0;
-    if (staged) hipLaunchKernelGGL((k_gemv<DT, true>), dim3(grid), dim3(NT), smem_bytes(DT, k), st, m, (const uint8_t *)act, k, y, S);
-    else hipLaunchKernelGGL((k_gemv<DT, false>), dim3(grid), dim3(NT), smem_bytes(DT, k), st, m, (const uint8_t *)act, k, y, S);
+    if (staged) hipLaunchKernelGGL((k_gemv<DT, true>), dim3(grid), dim3(NT), gemv_lds(DT, k), st, m, (const uint8_t *)act, k, y, S);
+    else hipLaunchKernelGGL((k_gemv<DT, false>), dim3(grid), dim3(NT), gemv_lds(DT, k), st, m, (const uint8_t *)act, k, y, S);
 }
 // Kernels that take more than 64 KiB of dynamic LDS declare it once.
 template <class K> void lds_opt_in(K kernel, unsigned bytes) {
@@ -4569,7 +4557,7 @@ int l3m_gemv_matrix_cores(int on) {
 }
 
 int l3m_k_prep(int dtype, const float *x, int k, void *act, void *stream) {
-    if (k < 1 || dtype < 0 || dtype >= L3M_NDTYPES || smem_bytes(dtype, k) > LDS_MAX) return fail_msg("prep: k out of range for this dtype");
+    if (k < 1 || dtype < 0 || dtype >= L3M_NDTYPES || !act_fits(dtype, k)) return fail_msg("prep: k out of range for this dtype");
     hipStream_t st = as_stream(stream);
     DISPATCH(dtype, launch_prep, x, k, act, st);
     CKL("k_prep");
@@ -4594,7 +4582,7 @@ int l3m_k_ltiles(int dtype, int ntiles, int k, const void *tiles, void *quant, v
 int l3m_k_gemv(const l3m_dmat *m, const void *act, int k, float *y, void *stream) {
     if (k < 1 || m->dtype < 0 || m->dtype >= L3M_NDTYPES || kpad(k) / 32 != m->nb || m->tiles != (m->rows + 15) / 16 || m->rows < 1)
         return fail_msg("gemv: shape does not match the matrix");
-    if (smem_bytes(m->dtype, k) > LDS_MAX) return fail_msg("gemv: k too large for this dtype");
+    if (!act_fits(m->dtype, k)) return fail_msg("gemv: k too large for this dtype");
     hipStream_t st = as_stream(stream);
     const int S = pick_split(m->nb);
     DISPATCH(m->dtype, launch_gemv, *m, act, k, y, S, st);
@@ -4602,7 +4590,8 @@ int l3m_k_gemv(const l3m_dmat *m, const void *act, int k, float *y, void *stream
     return 0;
 }
 
-// The most positions a call takes: 4 (hd + ceil4(pos + 1) + NT + 8) bytes within LDS_MAX.
+// The most positions a call takes, unchanged since one workgroup held q, every score and its threads' sums in LDS
+// (16,128 - hd or so; k_attend itself has no such bound): 4 (hd + ceil4(pos + 1) + NT + 8) bytes within LDS_MAX.
 static bool attend_fits(int pos, int hd) { return 4 * ((size_t)hd + ((pos + 4) & ~3) + NT + 8) <= LDS_MAX; }
 
 int l3m_k_attend(float *out, const float *q, const uint16_t *k, const uint16_t *v, int pos, int hd, int stride, void *stream) {
