@@ -444,9 +444,10 @@ __device__ __forceinline__ float4 load4(const float *__restrict__ x, int i, int 
 }
 
 // The standalone activation prep (pack.c:101-123: per 32-block amax, inv = 127 / amax, q = rint(x * inv), scale =
-// amax / 127, sum = sum(q), stored in the form the dtype's matvec reads (act_size); bf16 nearest even): a thread 4 values, 8 threads a block, one
-// load each and straight to memory, over as many workgroups as the vector fills. Bound by one kernel's latency:
-// q4_0 4096 values 2.1 us; 7.0 in one workgroup through LDS, copied out byte by byte.
+// amax / 127, sum = sum(q), stored in the form the dtype's matvec reads (act_size); bf16 nearest even): a thread 4
+// values, 8 threads a block, one load each and straight to memory at any alignment (put_block's forms, which the decode
+// step keeps for aligned LDS: with one definition for both it compiled to 0.6% slower tokens), over as many workgroups
+// as the vector fills. Bound by one kernel's latency: q4_0 4096 values 2.1 us; 7.0 in one workgroup through LDS, copied out byte by byte.
 template <int DT>
 __global__ void __launch_bounds__(NT) k_prep(const float *__restrict__ x, int k, uint8_t *__restrict__ out) {
     const int kp = kpad(k), i = 4 * (blockIdx.x * NT + threadIdx.x);
@@ -3396,9 +3397,9 @@ __global__ void __launch_bounds__(256) k_pf_rows(const float *y, int k, const fl
 // block scales into the f32 sum; bf16: v_mfma_f32_16x16x32_bf16 onto the f32 sum. Blocks in order. Lane l holds
 // row (token) l % 16, the 8 values at 8 (l / 16) of the block, and gets rows 4 (l / 16) + i of token l % 16.
 //
-// A row's blocks fall into ranges of PF_RANGE blocks or so (pf_ranges), each summed by itself, then added in
-// order. A wavefront takes RT x TT tiles over its share of the ranges: KS = blockDim / (64 WR) wavefronts split
-// them, and their sums are added in order through LDS; WR wavefronts of each share lie side by side. Operands come straight from L2 in the layouts they lie in (a contiguous run a tile and
+// A row's blocks fall into ranges of PF_RANGE blocks or so (pf_ranges). int8: each range is summed by itself and the sums
+// added in order; bf16: every product goes onto one sum. A wavefront takes RT x TT tiles over its share of the ranges:
+// KS = blockDim / (64 WR) wavefronts split them, and their sums are added in order through LDS; WR wavefronts of each share lie side by side. Operands come straight from L2 in the layouts they lie in (a contiguous run a tile and
 // block), PB blocks ahead; nothing is staged. Per q8_0 product a lane spends 12 VALU instructions on the scales
 // (48 clocks of its SIMD against 8 for the product), which bounds the largest shapes; RT = TT = 2 loads each
 // operand once for two products. The others are bound by latency, a chain of loads over few wavefronts: they
@@ -4282,6 +4283,8 @@ template <int DT> void pf_attention(const l3m_dmodel *M, const l3m_pfbuf *B, int
 // wavefronts; fewest, 32 x 16 tiles with the ranges split over up to 8. Measured (30 layers of dim 576, ffn 1536;
 // us to the first logits, each split for every matrix): 64 tokens 2065 / 1685 / 1509, 200 tokens 2282 / 1918 /
 // 1941, 480 tokens 2549 / 2394 / 2846; gate and up alone at 480 tokens 12.0 / 15.1 / 25.9 us, at 64 - / 7.6 / 7.0.
+// bf16 has no scales to multiply and crosses at the same sizes: 64 tokens 2070 / 1838 / 1715, 200 tokens 2196 / 2008 /
+// 2001, 480 tokens 2543 / 2557 / 2945, by this rule 1727 / 1944 / 2460 (runs of one side differ by 1%).
 constexpr int PF_WIDE = 1024;
 template <int DT, int EPI> void pf_gemm(const PfGemm &G, hipStream_t st) {
     constexpr int WR = EPI == 2 ? 2 : 1, MID = EPI == 2 ? 256 : 160;
@@ -4491,11 +4494,12 @@ int l3m_dev_upload(void *dst, const void *src, size_t bytes) {
     CK(hipStreamSynchronize(g_stream));
     return 0;
 }
-// Queued on the library's stream without waiting: a copy from pinned host memory (l3m_dev_host_alloc,
-// which must stay unchanged until the stream has run it) and a fill with zero bytes.
-int l3m_dev_upload_async(void *dst, const void *src_pinned, size_t bytes) {
+// Queued on the library's stream without waiting: a copy from host memory that stays unchanged until the stream has
+// run it (pinned, l3m_dev_host_alloc, to return at once; the kernel table's pageable tiles are staged first) and a
+// fill with zero bytes.
+int l3m_dev_upload_async(void *dst, const void *src, size_t bytes) {
     if (l3m_dev_init()) return -1;
-    CK(hipMemcpyAsync(dst, src_pinned, bytes, hipMemcpyHostToDevice, g_stream));
+    CK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g_stream));
     return 0;
 }
 int l3m_dev_zero_async(void *dst, size_t bytes) {
