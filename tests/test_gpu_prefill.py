@@ -5,10 +5,10 @@ that fills the K/V cache; decoding then starts at the last prompt token. The log
 must meet the engine bar of test_gpu_engine.py against the oracle (the reference's token-by-token order)
 and against the GPU's own token-by-token path (L3M_PREFILL=0): equal argmax, KL < 0.01 nats, max-abs
 within 2% of max|logit| (the int8 activation noise floor of the quantized paths). Prompts of 8 (the
-threshold: 7 positions, less than one 16-token group of the GEMM), 9 and 17 (a group boundary), 40 and 100
-tokens cover one to seven 16-token groups of the GEMM, and 65 ends exactly at the attention's second
-64-position chunk; head dims of 32 and 64 prepare the attention output inside the attention kernel, hd 48 in one of
-its own. q4_0 and
+threshold: 7 positions, less than one 16-token tile), 9 and 17 (a tile boundary), 40 and 100 tokens cover one to seven
+16-token tiles of the GEMM and the attention (hd 64, 32 and 48 on the matrix cores, 32-position chunks), and 65
+ends exactly at a tile's and a chunk's boundary; whole 32-blocks per head prepare the attention output inside the
+attention kernel, hd 48 in one of its own. q4_0 and
 mxfp4 bodies run the same int8 GEMM on q8_0 copies of their matrices with the same values (an mxfp4 block's
 scale 2^(e-128) is an f16 and its doubled e2m1 codes are int8).
 """
@@ -137,8 +137,8 @@ LONG = A.Config("pf_long", dim=128, n_layers=2, n_heads=4, n_kv_heads=2, ffn_dim
 
 
 def test_prefill_past_128_positions(models, oracle, monkeypatch):
-    """A 200-token prompt at ctx 256: 199 prefilled positions, past the 128-slot logits ring and over four of
-    the attention's 64-position chunks. The logits after the prompt meet the engine bar against the oracle
+    """A 200-token prompt at ctx 256: 199 prefilled positions, past the 128-slot logits ring and over seven of
+    the attention's 32-position chunks. The logits after the prompt meet the engine bar against the oracle
     and the GPU's token-by-token path, and each of the 30 greedy tokens that follow is the oracle's argmax
     given the same prefix (its second at a near-tie)."""
     path = models.get(LONG, "q8_0", seed=3, std=0.08, norm_jitter=0.2)
