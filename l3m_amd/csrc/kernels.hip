@@ -1713,10 +1713,8 @@ __device__ void attend_group(const l3m_dmodel &M, const l3m_dgroup &G, int layer
         if (active) {
             // (q0 + h) / hpk by an exact float reciprocal (both far below 2^20)
             const int kvl = (int)(((float)(G.q0 + h) + 0.5f) * ihpk) - G.kv0;
-            const int at = BATCH ? 0 : G.kv0 + kvl;   // BATCH: buffers over the layer's rows, the head's from row0 on
-            const uint16_t *kw = WIN ? kvb + kvl * win : M.kc + ((size_t)layer * M.n_kv + at) * win;
-            const uint16_t *vw = WIN ? kvb + (G.nkv + kvl) * win : M.vc + ((size_t)layer * M.n_kv + at) * win;
-            const uint32_t row0 = (uint32_t)((G.kv0 + kvl) * M.ctx);
+            const uint16_t *kw = WIN ? kvb + kvl * win : M.kc + ((size_t)layer * M.n_kv + G.kv0 + kvl) * win;
+            const uint16_t *vw = WIN ? kvb + (G.nkv + kvl) * win : M.vc + ((size_t)layer * M.n_kv + G.kv0 + kvl) * win;
             const uint4 *kcur = (const uint4 *)(cur + kvl * hd), *vcur = (const uint4 *)(cur + (G.nkv + kvl) * hd);
             float q[8];
             {
@@ -1725,37 +1723,64 @@ __device__ void attend_group(const l3m_dmodel &M, const l3m_dgroup &G, int layer
                 q[0] = a.x; q[1] = a.y; q[2] = a.z; q[3] = a.w; q[4] = b.x; q[5] = b.y; q[6] = b.z; q[7] = b.w;
             }
             float m = -INFINITY, l = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            // BATCH: the position whose row is cur's; lanes past the head keep zeros (their zero q times an infinity is NaN)
-            const int own = j < nv ? pos : -1;
             // rounds r = 0, 1, ... cover positions (r * W + wi) * PPW + gl; ATT_IT rounds per chunk
             for (int r0 = 0; (r0 * W + wi) * PPW < n; r0 += ATT_IT) {
-                float s[ATT_IT];
-                float cm = -INFINITY;
-                uint4 kb[ATT_IT], vb[ATT_IT];
                 if constexpr (BATCH) {
+                    // buffers over the layer's rows (a uniform base), the head's from row0 on; own: the position whose row is
+                    // cur's. Lanes past the head keep zeros (their zero q times an infinity is NaN)
+                    const uint16_t *kl = M.kc + (size_t)layer * M.n_kv * win, *vl = M.vc + (size_t)layer * M.n_kv * win;
+                    const uint32_t row0 = (uint32_t)((G.kv0 + kvl) * M.ctx);
+                    const int own = j < nv ? pos : -1;
+                    float s[ATT_IT];
+                    float cm = -INFINITY;
+                    uint4 kb[ATT_IT], vb[ATT_IT];
 #pragma unroll
                     for (int k = 0; k < ATT_IT; k++) {
                         const int t = ((r0 + k) * W + wi) * PPW + gl;
-                        kb[k] = ld16_if<COH>(kw, 16 * ((row0 + (uint32_t)t) * (uint32_t)nv + (uint32_t)j), t < pos && j < nv);
+                        kb[k] = ld16_if<COH>(kl, 16 * ((row0 + (uint32_t)t) * (uint32_t)nv + (uint32_t)j), t < pos && j < nv);
                     }
 #pragma unroll
                     for (int k = 0; k < ATT_IT; k++) {
                         const int t = ((r0 + k) * W + wi) * PPW + gl;
-                        vb[k] = ld16_if<COH>(vw, 16 * ((row0 + (uint32_t)t) * (uint32_t)nv + (uint32_t)j), t < pos && j < nv);
+                        vb[k] = ld16_if<COH>(vl, 16 * ((row0 + (uint32_t)t) * (uint32_t)nv + (uint32_t)j), t < pos && j < nv);
                     }
                     asm volatile("" ::: "memory");
                     const uint4 kc = kcur[j < nv ? j : 0], vc = vcur[j < nv ? j : 0];
 #pragma unroll
                     for (int k = 0; k < ATT_IT; k++)
                         if (((r0 + k) * W + wi) * PPW + gl == own) { kb[k] = kc; vb[k] = vc; }
+#pragma unroll
+                    for (int k = 0; k < ATT_IT; k++) {
+                        const int t = ((r0 + k) * W + wi) * PPW + gl;
+                        const float part = dot8_bf16(q, kb[k], 0.f);
+                        s[k] = t < n ? lanes_sum_n(part, LP) * scale : -INFINITY;
+                        cm = fmaxf(cm, s[k]);
+                    }
+                    const float mn = fmaxf(m, lanes_max<64>(cm));
+                    const float alpha = expf(m - mn);
+                    l *= alpha;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) o[e] *= alpha;
+#pragma unroll
+                    for (int k = 0; k < ATT_IT; k++) {  // past the end p is 0 and the row zeros
+                        const float p = expf(s[k] - mn);
+                        l += p;
+                        const uint4 vv = vb[k];
+                        o[0] = fmaf(p, bf16_f32(vv.x & 0xFFFF), o[0]); o[1] = fmaf(p, bf16_f32(vv.x >> 16), o[1]);
+                        o[2] = fmaf(p, bf16_f32(vv.y & 0xFFFF), o[2]); o[3] = fmaf(p, bf16_f32(vv.y >> 16), o[3]);
+                        o[4] = fmaf(p, bf16_f32(vv.z & 0xFFFF), o[4]); o[5] = fmaf(p, bf16_f32(vv.z >> 16), o[5]);
+                        o[6] = fmaf(p, bf16_f32(vv.w & 0xFFFF), o[6]); o[7] = fmaf(p, bf16_f32(vv.w >> 16), o[7]);
+                    }
+                    m = mn;
+                    continue;
                 }
+                float s[ATT_IT];
+                float cm = -INFINITY;
 #pragma unroll
                 for (int k = 0; k < ATT_IT; k++) {
                     const int t = ((r0 + k) * W + wi) * PPW + gl;
                     float part = 0.f;
-                    if constexpr (BATCH) {
-                        part = dot8_bf16(q, kb[k], 0.f);
-                    } else if (t < n && j < nv) {
+                    if (t < n && j < nv) {
                         uint4 kk;
                         if (t == pos) kk = kcur[j];
                         else if (WIN) kk = ((const uint4 *)(kw + (size_t)t * rs))[j];
@@ -1773,13 +1798,12 @@ __device__ void attend_group(const l3m_dmodel &M, const l3m_dgroup &G, int layer
 #pragma unroll
                 for (int k = 0; k < ATT_IT; k++) {
                     const int t = ((r0 + k) * W + wi) * PPW + gl;
-                    if (BATCH || t < n) {             // batched: past the end p is 0 and the row zeros
+                    if (t < n) {
                         const float p = expf(s[k] - mn);
                         l += p;
-                        if (BATCH || j < nv) {
+                        if (j < nv) {
                             uint4 vv;
-                            if constexpr (BATCH) vv = vb[k];
-                            else if (t == pos) vv = vcur[j];
+                            if (t == pos) vv = vcur[j];
                             else if (WIN) vv = ((const uint4 *)(vw + (size_t)t * rs))[j];
                             else vv = ld16<COH>(vw, (size_t)t * (hd >> 3) + j);
                             o[0] = fmaf(p, bf16_f32(vv.x & 0xFFFF), o[0]); o[1] = fmaf(p, bf16_f32(vv.x >> 16), o[1]);
