@@ -2,6 +2,7 @@
 batches of rows, one workgroup or up to 64 whose parts meet in a workspace of the stream. Against the oracle's
 l3m_attend within 1e-5 absolute (the reference's own bar, tests/test_kernels.c:145)."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -143,4 +144,42 @@ def test_attend_streams_come_and_go(dev, oracle):
     got = dev.get(do, hd, np.float32)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
     assert hip.hipStreamDestroy(st) == 0
+    dev.free_all()
+
+
+def test_attend_threads_on_their_own_streams(dev, oracle):
+    """Four threads, each with two streams and inputs of its own, 60 calls on each while the others do the
+    same: every call's output is its inputs'."""
+    hip = C.CDLL("libamdhip64.so")
+    n, hd, calls = 2000, 64, 60
+    sets = [inputs(50 + i, n, hd, hd) for i in range(8)]
+    bufs = [(dev.put(q), dev.put(k), dev.put(v)) for q, k, v in sets]
+    outs = [[dev.alloc(hd * 4) for _ in range(calls)] for _ in sets]
+    streams = []
+    for _ in sets:
+        st = C.c_void_p()
+        assert hip.hipStreamCreateWithFlags(C.byref(st), 1) == 0
+        streams.append(st)
+    failed = []
+
+    def work(t):
+        try:
+            for c in range(calls):
+                for i in (2 * t, 2 * t + 1):
+                    assert dev.lib.l3m_k_attend(outs[i][c], *bufs[i], n - 1, hd, hd, streams[i]) == 0
+        except BaseException as e:
+            failed.append(e)
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed and hip.hipDeviceSynchronize() == 0
+    for (q, k, v), o in zip(sets, outs):
+        want = oracle.attend(q, k, v, n - 1, hd, hd)
+        for p in o:
+            assert np.abs(dev.get(p, hd, np.float32) - want).max() <= 1e-5
+    for st in streams:
+        assert hip.hipStreamDestroy(st) == 0
     dev.free_all()
