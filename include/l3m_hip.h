@@ -220,7 +220,8 @@ int    l3m_phase_stamps(int mode, int pos, int layer, unsigned long long *out);
 int    l3m_logits_at(const l3m_model *m, int pos, float *out);
 // Prompt positions the last generate call ran as one batched prefill (0: token by token). Prompts of at
 // least L3M_PREFILL_MIN (default 8) tokens on bf16, q8_0 and q4_0 bodies (and mxfp4 bodies whose blocks widen
-// exactly to q8_0) are prefilled unless L3M_PREFILL=0.
+// exactly to q8_0) are prefilled unless L3M_PREFILL=0 or the device had no room for the second copy of the
+// matrices that prompts run on.
 int    l3m_prefill_positions(const l3m_model *m);
 // The attention mode the decode step of m runs at positions inside its K/V window (l3m_attention_mode's
 // codes); and the window's size in positions: ctx when every position fits in LDS, else the most (a
