@@ -67,6 +67,7 @@ struct l3m_model {
     float        temp;         // the running generate call's temperature (0: greedy)
     l3m_pflayer *pf;           // batched prompt prefill: per-layer full matrices, NULL when unavailable
     l3m_pfbuf    pfb;
+    int         *no_room;      // while loading: set when memory ran out with the prompt matrices in it
     l3m_pfgraphs *pfg;         // the prefill's captured graphs (NULL: launched kernel by kernel, L3M_PREFILL_GRAPH=0)
     int          prefill_min;  // prompts of at least this many tokens are prefilled (L3M_PREFILL_MIN)
     int          prefilled;    // positions the last generate call prefilled
@@ -96,6 +97,7 @@ static void *dalloc(l3m_model *m, size_t bytes) {
         m->cap_allocs = cap;
     }
     void *p = l3m_dev_alloc(bytes);
+    if (!p && m->pf) *m->no_room = 1;
     if (p) m->allocs[m->n_allocs++] = p;
     return p;
 }
@@ -268,39 +270,6 @@ static int upload_prefill(l3m_model *m, const l3m_mapped *f, int l, int dt, cons
     return rc || P->qkv.dtype != (dt == L3M_BF16 ? L3M_BF16 : L3M_Q8_0) ? -1 : 0;
 }
 
-// m->pf and m->pfb, or, when the device (or the host) has no room for them, everything as before and m->pf NULL.
-static void add_prefill(l3m_model *m) {
-    const l3m_dmodel *d = &m->dm;
-    const int mark = m->n_allocs;
-    m->pf = calloc((size_t)d->n_layers, sizeof *m->pf);
-    int ok = m->pf != NULL;
-    for (int l = 0; l < d->n_layers && ok; l++) ok = !upload_prefill(m, &m->f, l, (int)l3m_map_blk(&m->f, l, "wq")->dtype, &m->layers[l]);
-    if (ok) {
-        // activations of whole 64-token groups (a GEMM's workgroup reads up to 32 tokens, past the prompt's end too)
-        const size_t nqd = (size_t)d->n_heads * d->hd, mk = (size_t)d->dim > nqd ? (size_t)d->dim : nqd, ctx = (size_t)d->ctx, c64 = (ctx + 63) / 64 * 64;
-        l3m_pfbuf *b = &m->pfb;
-        const size_t vb = m->dtype == L3M_BF16 ? 2 : 1;
-        ok = (b->x = dalloc(m, ctx * d->dim * 4)) && (b->act.q = dalloc(m, c64 * mk * vb)) && (b->act.s = dalloc(m, c64 * mk / 32 * 4)) &&
-             (b->hact.q = dalloc(m, c64 * d->ffn * vb)) && (b->hact.s = dalloc(m, c64 * d->ffn / 32 * 4)) && (b->q = dalloc(m, ctx * nqd * 4)) &&
-             (b->att = dalloc(m, ctx * nqd * 4));
-    }
-    if (ok) {
-        // Few launches: the host's are longer than the GPU's work behind them, and a graph's one launch frees it for the
-        // decode pass. Many: the GPU is behind, and a graph's kernels start further apart. us a call of dim 256 / 576, 100
-        // tokens, launched one by one and as a graph: 2 layers 170, 141 / 189, 161; 4: 244, 223 / 289, 268; 8: 389, 384 / 481,
-        // 477; 12: 536, 551 / 673, 684; 20: 841, 895 / 1066, 1097; 30: 1272, 1321 / 1579, 1621 (16 tokens cross at the
-        // same depth). L3M_PREFILL_GRAPH=0: never (for comparison)
-        const char *pg = getenv("L3M_PREFILL_GRAPH");
-        if ((!pg || strcmp(pg, "0")) && d->n_layers <= 8) m->pfg = l3m_pfgraphs_new();
-        return;
-    }
-    while (m->n_allocs > mark) l3m_dev_free(m->allocs[--m->n_allocs]);
-    free(m->pf);
-    m->pf = NULL;
-    l3m_dev_clear_error();
-    fprintf(stderr, "l3m: no memory for the prompt matrices: prompts run token by token\n");
-}
-
 // The file row starting at input column c (whole 32-blocks for quantized rows).
 static const void *col_slice(const void *row, int dtype, int c) {
     return (const uint8_t *)row + (dtype >= L3M_Q8_0 ? l3m_file_row_bytes(dtype, c) : (size_t)c * (dtype == L3M_BF16 ? 2 : 4));
@@ -317,7 +286,7 @@ static int upload_tensor(l3m_model *m, l3m_dmat *out, const l3m_tensor *t) {
 }
 
 static l3m_model *fail(l3m_model *m, const char *msg) {
-    if (msg) fprintf(stderr, "l3m: %s\n", msg);
+    if (msg && !*m->no_room) fprintf(stderr, "l3m: %s\n", msg);
     l3m_free(m);
     return NULL;
 }
@@ -332,11 +301,12 @@ void l3m_rope_table(float *table, int ctx, int hd, float theta) {
         }
 }
 
-l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
+static l3m_model *load(const char *path, const l3m_opts *opts, int prefill, int *no_room) {
     l3m_opts o = {0};
     if (opts) o = *opts;
     l3m_model *m = calloc(1, sizeof *m);
     if (!m) return NULL;
+    m->no_room = no_room;
     m->logits_pos = -1;
     m->spin_limit = SPIN_LIMIT;
     if (l3m_map_open(&m->f, path)) { free(m); return NULL; }      // a bad file is reported as such first
@@ -403,6 +373,14 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
     if (d->n_groups > MAX_PARTS || d->n_chunks > MAX_PARTS) return fail(m, "too many head groups or FFN chunks for the GPU kernels");
     l3m_model_layout(d);
     m->layers = calloc((size_t)d->n_layers, sizeof *m->layers);
+    // batched prefill (bf16, q8_0 and q4_0 bodies, and mxfp4 bodies whose blocks widen exactly to q8_0; whole
+    // 32-blocks): unless L3M_PREFILL=0
+    const char *pe_ = getenv("L3M_PREFILL"), *pm_ = getenv("L3M_PREFILL_MIN");
+    const int qb_ = d->dim % 32 == 0 && (d->n_heads * d->hd) % 32 == 0 && d->ffn % 32 == 0;
+    if (prefill && (!pe_ || strcmp(pe_, "0")) && !m->reference && !gpt2 && qb_ && l3m_prefill_fits(d->dim, d->ffn, d->n_heads * d->hd, d->hd) &&
+        (m->dtype == L3M_BF16 || m->dtype == L3M_Q8_0 || m->dtype == L3M_Q4_0 || m->mx_wide || (m->dtype == L3M_MXFP4 && mxfp4_body_widens(f, d->n_layers))))
+        m->pf = calloc((size_t)d->n_layers, sizeof *m->pf);
+    m->prefill_min = pm_ ? atoi(pm_) : 8;
     l3m_dgroup *groups = calloc((size_t)d->n_groups, sizeof *groups);
     l3m_dchunk *chunks = calloc((size_t)d->n_chunks, sizeof *chunks);
     int max_rows = d->dim > 2 * chunk + 32 ? d->dim : 2 * chunk + 32;
@@ -498,6 +476,11 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
             free(groups); free(chunks); free(rows);
             return fail(m, "weight upload failed");
         }
+        if (m->pf && upload_prefill(m, f, l, dt, L)) {
+            free(groups); free(chunks); free(rows);
+            *m->no_room = 1;
+            return fail(m, "prefill weight upload failed");
+        }
     }
     // The K/V window: every position of the context when it fits in LDS beside the rest of the attention
     // block, else the most positions (a multiple of 32) that fit; a step at a position past it reads K and V
@@ -569,6 +552,26 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
     d->xb = dalloc(m, (size_t)d->dim * 4);
     d->po = dalloc(m, (size_t)d->n_groups * d->dim * 4);
     d->pd = dalloc(m, (size_t)d->n_chunks * d->dim * 4);
+    if (m->pf) {
+        // activations of whole 64-token groups (a GEMM's workgroup reads up to 32 tokens, past the prompt's end too)
+        const size_t nqd = (size_t)d->n_heads * d->hd, mk = (size_t)d->dim > nqd ? (size_t)d->dim : nqd, ctx = (size_t)d->ctx, c64 = (ctx + 63) / 64 * 64;
+        m->pfb.x = dalloc(m, ctx * d->dim * 4);
+        const size_t vb = m->dtype == L3M_BF16 ? 2 : 1;
+        m->pfb.act.q = dalloc(m, c64 * mk * vb);
+        m->pfb.act.s = dalloc(m, c64 * mk / 32 * 4);
+        m->pfb.hact.q = dalloc(m, c64 * d->ffn * vb);
+        m->pfb.hact.s = dalloc(m, c64 * d->ffn / 32 * 4);
+        m->pfb.q = dalloc(m, ctx * nqd * 4);
+        m->pfb.att = dalloc(m, ctx * nqd * 4);
+        if (!m->pfb.x || !m->pfb.act.q || !m->pfb.act.s || !m->pfb.hact.q || !m->pfb.hact.s || !m->pfb.q || !m->pfb.att) return fail(m, "out of device memory");
+        // Few launches: the host's are longer than the GPU's work behind them, and a graph's one launch frees it for the
+        // decode pass. Many: the GPU is behind, and a graph's kernels start further apart. us a call of dim 256 / 576, 100
+        // tokens, launched one by one and as a graph: 2 layers 170, 141 / 189, 161; 4: 244, 223 / 289, 268; 8: 389, 384 / 481,
+        // 477; 12: 536, 551 / 673, 684; 20: 841, 895 / 1066, 1097; 30: 1272, 1321 / 1579, 1621 (16 tokens cross at the
+        // same depth). L3M_PREFILL_GRAPH=0: never (for comparison)
+        const char *pg = getenv("L3M_PREFILL_GRAPH");
+        if ((!pg || strcmp(pg, "0")) && d->n_layers <= 8) m->pfg = l3m_pfgraphs_new();
+    }
     d->logits = dalloc(m, (size_t)NSLOTS * d->vocab * 4);
     // persistent kernel: one workgroup per CU (the LDS request keeps a second one off each CU); the body
     // (head groups, then FFN chunks) on the workgroups of one XCD, every other workgroup on head tiles.
@@ -630,15 +633,6 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
         m->graphs = l3m_graphs_build(d, m->layers);
         if (!m->graphs) return fail(m, "could not capture the decode step");
     }
-    // batched prefill (bf16, q8_0 and q4_0 bodies, and mxfp4 bodies whose blocks widen exactly to q8_0; whole
-    // 32-blocks): unless L3M_PREFILL=0. Last, and only if its memory is there: a model without it feeds prompts
-    // token by token
-    const char *pf_ = getenv("L3M_PREFILL"), *pm_ = getenv("L3M_PREFILL_MIN");
-    const int qb_ = d->dim % 32 == 0 && (d->n_heads * d->hd) % 32 == 0 && d->ffn % 32 == 0;
-    if ((!pf_ || strcmp(pf_, "0")) && !m->reference && !gpt2 && qb_ && l3m_prefill_fits(d->dim, d->ffn, d->n_heads * d->hd, d->hd) &&
-        (m->dtype == L3M_BF16 || m->dtype == L3M_Q8_0 || m->dtype == L3M_Q4_0 || m->mx_wide || (m->dtype == L3M_MXFP4 && mxfp4_body_widens(f, d->n_layers))))
-        add_prefill(m);
-    m->prefill_min = pm_ ? atoi(pm_) : 8;
     const char *base = strrchr(path, '/');
     base = base ? base + 1 : path;
     if (m->reference)
@@ -651,6 +645,21 @@ l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
                 "persistent %d (grid %d, body on xcd %d, head %d x %d tiles, lds %u)\n", m->desc, d->ctx, l3m_dev_name(), d->n_groups,
                 d->n_chunks, d->head_grid, d->head_tiles_per_wg, d->lds_a, d->lds_b, d->lds_h, d->kv_lds, d->kv_win, m->persist, m->grid, m->body_xcc,
                 m->n_head, m->head_tpw, m->lds_decode);
+    return m;
+}
+
+// With the prompt matrices (a second copy of the body) where they fit beside the model, else without them: prompts then
+// run token by token. (Allocated after all the rest instead, to be dropped alone, they left deep prompts 1% slower: 30
+// layers of dim 576, 480 tokens 2,361 us a call against 2,337, a model's first 2,636 against 2,603.)
+l3m_model *l3m_load(const char *path, const l3m_opts *opts) {
+    int no_room = 0;
+    l3m_model *m = load(path, opts, 1, &no_room);
+    if (no_room && !m) {
+        l3m_dev_clear_error();
+        fprintf(stderr, "l3m: no room for a second copy of the matrices: prompts run token by token\n");
+        no_room = 0;
+        m = load(path, opts, 0, &no_room);
+    }
     return m;
 }
 

@@ -4955,7 +4955,7 @@ int l3m_graphs_launch(l3m_graphs *g, int with_head, void *stream) {
 
 // A prompt length's launches (their grids and arguments depend on P alone, every buffer is the model's own) as a
 // graph, for the PF_GRAPHS lengths used last: the first prompt of a length is launched kernel by kernel, its second
-// captured, later ones replayed (add_prefill's rule says for which models). Capture and instantiation cost a call 0.06 ms
+// captured, later ones replayed (the loader's rule says for which models). Capture and instantiation cost a call 0.06 ms
 // (2 layers) to 0.16 (6), which a length seen once never pays (2 layers of dim 128, 48 tokens: the first call 198 us, the
 // second 198, then 133; launched one by one 190, 165, then 157). Captured on a stream
 // of its own: other threads' work on the library's stream stays out of it. off: a capture failed, launched one by one
